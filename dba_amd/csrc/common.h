@@ -101,6 +101,13 @@ __device__ __forceinline__ int bit_of(const gu64* bm, int t) {
     return (int)((bm[t >> 6] >> (t & 63)) & 1ull);
 }
 
+// Workgroup barrier that orders LDS only: outstanding global loads stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Workgroup-wide OR of a per-thread predicate (wave ballot, then LDS across waves).
 template <int NT>
 __device__ __forceinline__ int block_any(int pred, int* lds_scratch) {
@@ -271,19 +278,24 @@ __device__ __forceinline__ int nb_dir1(int l) {
     return l < H ? 0 : (l < TB + H ? 1 : 2);
 }
 
-template <int NT>
-__device__ __forceinline__ double block_max(double v, double* lds_scratch) {
-    constexpr int NW = NT / 64;
-    // the shift tree of wave_sum_down with fmax (lane 0 sees the same operands:
-    // none of the lanes it reads is a row shift's zero filler, so the result holds
-    // for values of any sign; the same DPP shifts are pinned bit-exactly by the
-    // field-sum test of dba_field_sum)
+// Lane 0 gets the maximum over the wave: the shift tree of wave_sum_down with
+// fmax (none of the lanes lane 0 reads is a row shift's zero filler, so the
+// result holds for values of any sign; the same DPP shifts are pinned bit-exactly
+// by the field-sum test of dba_field_sum)
+__device__ __forceinline__ double wave_max_down(double v) {
     v = fmax(v, __shfl_down(v, 32, 64));
     v = fmax(v, __shfl_down(v, 16, 64));
     v = fmax(v, dpp_row_down<8>(v));
     v = fmax(v, dpp_row_down<4>(v));
     v = fmax(v, dpp_row_down<2>(v));
     v = fmax(v, dpp_row_down<1>(v));
+    return v;
+}
+
+template <int NT>
+__device__ __forceinline__ double block_max(double v, double* lds_scratch) {
+    constexpr int NW = NT / 64;
+    v = wave_max_down(v);
     int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (lane == 0) lds_scratch[wid] = v;
     __syncthreads();

@@ -488,7 +488,7 @@ dba_status get_group(dba_ctx* ctx, const std::vector<int>& ids, Group** out) {
               first->h.full_tiles && first->h.nt <= 1024;
     // KH divides by dx, dy and the cell area; when all three are powers of two
     // (a power-of-two grid on the unit square) the step multiplies by their exact
-    // reciprocals instead, which gives the same doubles (kdiv in k_kh.h)
+    // reciprocals instead, which gives the same doubles (kh_cdiv in k_kh.h)
     if (g->model == DBA_MODEL_KH) {
         auto pow2 = [](double d) {
             int e = 0;
@@ -581,11 +581,13 @@ void launch_step_tb(const Group* g, hipStream_t s) {
                 hipLaunchKernelGGL((k93_step_kernel<TB, NT, false>), grid, block, 0, s, wl_of(g));
             break;
         case DBA_MODEL_KH:
-            if constexpr (TB <= 16 && NT <= 256) {
+            // one thread per cell, whatever workgroup size the instance asks for
+            // (it never changes results)
+            if constexpr (TB <= 16) {
                 if (g->kh_p2)
-                    hipLaunchKernelGGL((kh_step_kernel<TB, NT, true>), grid, block, 0, s, wl_of(g));
+                    hipLaunchKernelGGL((kh_step_kernel<TB, true>), grid, dim3(TB * TB), 0, s, wl_of(g));
                 else
-                    hipLaunchKernelGGL((kh_step_kernel<TB, NT, false>), grid, block, 0, s, wl_of(g));
+                    hipLaunchKernelGGL((kh_step_kernel<TB, false>), grid, dim3(TB * TB), 0, s, wl_of(g));
             }
             break;
         default:

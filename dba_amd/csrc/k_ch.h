@@ -533,13 +533,6 @@ namespace dba {
 // neighbours and the bytes written are those of ch_dense_kernel, so the two
 // give identical results.
 
-// Workgroup barrier that orders LDS only: outstanding global loads stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 constexpr int kMarchRing = 64;  // LDS ring rows (a power of two >= 36 + 32 - 4)
 constexpr int kMarchMinTiles = 4096;  // grids from 2048^2 (32 x 32 tiles) march
 

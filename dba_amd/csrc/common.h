@@ -63,7 +63,8 @@ struct Inst {
     double ntotal;               // number of cells (conserved mean)
     // derived constants, computed on the host with the same expressions as the oracle
     double invdx2, inv6dx2, inv2dx, dt_tau, alpha_pi, cos_jt0, sin_jt0, k_epsp;
-    double mb_cx, mb_cy, mb_cz, mb_lk, mb_omz;  // Model B: -1 + 1/r_x.., log(k_eq)/r_z, 1 - z_crit
+    double mb_cx, mb_cy, mb_cz, mb_lk;  // Model B: -1 + 1/r_x.., log(k_eq)/r_z
+    double mb_irx, mb_iry, mb_irz, mb_hiomz;  // ... 1/r_x.., 1 / (2 (1 - z_crit))
     // model constants
     double tau, eps_bar, delta, alpha, gamma, theta0, latent_k, t_eq;
     double mobility, kappa, react_gamma, cbar;
@@ -83,6 +84,12 @@ using CInst = const DBA_CONST Inst;
 // would otherwise become a scalar load that the wave waits for at once).
 __device__ __forceinline__ int load_early(const gi32* p) {
     return __hip_atomic_load((int*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// The double `off` bytes past a uniform address: one 32-bit offset register
+// instead of a 64-bit address per access.
+__device__ __forceinline__ gdouble& at_bytes(gdouble* p, unsigned off) {
+    return *(gdouble*)((DBA_GLOBAL char*)p + off);
 }
 
 // Boundary index map: periodic wrap, or mirror about the boundary face.

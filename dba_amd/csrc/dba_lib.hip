@@ -106,7 +106,8 @@ struct Group {
     int march = 0;                // column-march single-launch steps: tiles per strip (0: off)
     bool spec = false;            // K93 single-launch steps with speculative staging
     bool kh_p2 = false;           // KH: dx, dy and the cell area of every instance are powers of two
-    int sb_from = 0;              // Model B: lists of at least this many blocks step on superblocks (0: never)
+    int march_from = 0;           // Model B: lists of at least this many blocks take the column march (0: never)
+    int mb_nl = 1, mb_ncx = 0, mb_ncy = 0, mb_ntz = 0;  // ... layers per strip, columns in x and y, layers
     bool nine = true;             // CH 9-point stencil (the march kernel is instanced on it)
     Inst* d_insts = nullptr;
     Seg* d_segs = nullptr;
@@ -144,6 +145,7 @@ struct CachedGraph {
 
 struct dba_ctx {
     int device = 0;
+    int n_cu = 256;                // compute units of the device
     hipStream_t stream = nullptr;  // compute stream: steps, finalize, downloads
     hipStream_t setup = nullptr;   // instance and group set-up, uploads of never-stepped instances
     int next_id = 1;
@@ -184,7 +186,10 @@ void derive_constants(const dba_params& p, Inst& h) {
         h.mb_cz = -1.0 + 1.0 / p.r_z;
         h.mb_lk = std::log(p.k_eq) / p.r_z;
     }
-    h.mb_omz = 1.0 - p.z_crit;
+    h.mb_irx = 1.0 / p.r_x;
+    h.mb_iry = 1.0 / p.r_y;
+    h.mb_irz = 1.0 / p.r_z;
+    h.mb_hiomz = 0.5 / (1.0 - p.z_crit);
 }
 
 dba_status validate(const dba_params& p) {
@@ -504,20 +509,32 @@ dba_status get_group(dba_ctx* ctx, const std::vector<int>& ids, Group** out) {
     // measured faster than 16384 or 3072 with longer pipelines per wave
     int64_t cap = g->model == DBA_MODEL_MODELB ? 65536 : (g->model == DBA_MODEL_DENDRITE_K94 ? 16384 : 4096);
     g->grid = (int)std::max<int64_t>(1, std::min<int64_t>(g->total_tiles, cap));
-    // Model B superblocks (modelb_mu_sb_kernel): one 3D instance of full 4x4x4
-    // blocks, an even number of blocks in x and y, no conserved shift; steps with
-    // at least a quarter of the blocks awake. DBA_MODELB_SUPERBLOCKS=0 turns them
-    // off and =1 uses them for every non-empty list (both give the same doubles).
+    // Model B column march (modelb_march_kernel): one 3D instance, steps with at
+    // least a quarter of the blocks awake. DBA_MODELB_SUPERBLOCKS=0 turns it off and
+    // =1 uses it for every non-empty list (without conserved DBA both give the same
+    // doubles). Layers per strip: the fewest rounds of resident workgroups, each
+    // round 4 nl + 4 planes long.
     if (g->model == DBA_MODEL_MODELB && ids.size() == 1 && g->tile == 4 && g->tile_z == 4) {
         const Inst& h = first->h;
-        if (first->p.mode != DBA_MODE_CONSERVED && h.full_tiles && h.nz > 1 && h.ntx % 2 == 0 &&
-            h.nty % 2 == 0) {
+        if (h.full_tiles && h.nz > 1 && (int64_t)h.nx * h.ny < (1 << 28)) {
             const char* env = std::getenv("DBA_MODELB_SUPERBLOCKS");
             const std::string e = env ? env : "";
-            g->sb_from = e == "0" ? 0 : (e == "1" ? 1 : (int)((h.nt + 3) / 4));
-            // the block kernels then only take lists shorter than sb_from
-            if (g->sb_from > 0)
-                g->grid = (int)std::max<int64_t>(1, std::min<int64_t>(g->grid, (g->sb_from + 7) / 8));
+            g->march_from = e == "0" ? 0 : (e == "1" ? 1 : (int)((h.nt + 3) / 4));
+            g->mb_ntz = h.ntz;
+            g->mb_ncx = (h.nx + MbMarch::TX - 1) / MbMarch::TX;
+            g->mb_ncy = (h.ny + MbMarch::TY - 1) / MbMarch::TY;
+            const int64_t cols = (int64_t)g->mb_ncx * g->mb_ncy, slots = (g->conserved ? 1 : 2) * (int64_t)ctx->n_cu;
+            int64_t best = INT64_MAX;
+            for (int nl = 1; nl <= (g->conserved ? MbMarch::MLC : MbMarch::ML) && nl <= h.ntz; nl++) {
+                const int64_t wgs = cols * ((h.ntz + nl - 1) / nl), cost = (wgs + slots - 1) / slots * (4 * nl + 4);
+                if (cost < best) {
+                    best = cost;
+                    g->mb_nl = nl;
+                }
+            }
+            // the block kernels then only take lists shorter than march_from
+            if (g->march_from > 0)
+                g->grid = (int)std::max<int64_t>(1, std::min<int64_t>(g->grid, (g->march_from + 7) / 8));
         }
     }
     size_t n = ids.size();
@@ -610,15 +627,21 @@ void launch_step(const Group* g, hipStream_t s) {
     if (g->model == DBA_MODEL_DENDRITE_K94 || g->model == DBA_MODEL_MODELB) {
         dim3 grid(g->grid), block(64);
         if (g->model == DBA_MODEL_MODELB) {
-            // each pair returns at once when the other takes the step (by list length);
-            // superblocks of 2 x 2 x 1 blocks (2 x 2 x 2 on 8-wave workgroups measured slower)
-            const int from = g->sb_from > 0 ? g->sb_from : INT_MAX;
-            const dim3 sgrid((unsigned)std::max<int64_t>(1, g->total_tiles / 4)), sblock(Sb<1>::NT);
+            // the march and the pair of block kernels: by list length, one of them
+            // returns at once
+            const int from = g->march_from > 0 ? g->march_from : INT_MAX;
             if (g->tile_z == 4) {
-                if (g->sb_from > 0) hipLaunchKernelGGL(modelb_mu_sb_kernel<1>, sgrid, sblock, 0, s, wl_of(g), from);
+                if (g->march_from > 0) {
+                    const int ntz = g->mb_ntz, ncol = g->mb_ncx * g->mb_ncy;
+                    const dim3 mgrid((unsigned)(ncol * ((ntz + g->mb_nl - 1) / g->mb_nl)));
+                    if (g->conserved)
+                        hipLaunchKernelGGL(modelb_march_kernel<true>, mgrid, dim3(MbMarch::NT), 0, s, wl_of(g), from,
+                                           g->mb_nl, g->mb_ncx, g->mb_ncy);
+                    else
+                        hipLaunchKernelGGL(modelb_march_kernel<false>, mgrid, dim3(MbMarch::NT), 0, s, wl_of(g), from,
+                                           g->mb_nl, g->mb_ncx, g->mb_ncy);
+                }
                 hipLaunchKernelGGL((modelb_mu_kernel<4, 4>), grid, block, 0, s, wl_of(g), from);
-                if (g->sb_from > 0)
-                    hipLaunchKernelGGL(modelb_update_sb_kernel<1>, sgrid, sblock, 0, s, wl_of(g), from);
                 hipLaunchKernelGGL((modelb_update_kernel<4, 4>), grid, block, 0, s, wl_of(g), from);
             } else {
                 hipLaunchKernelGGL((modelb_mu_kernel<4, 1>), grid, block, 0, s, wl_of(g), from);
@@ -933,6 +956,9 @@ dba_status dba_init(int32_t device, dba_ctx** out) {
         return fail(DBA_ERR_HIP, "hipGetSymbolAddress(scratch) failed: %s", hipGetErrorString(e));
     }
     ctx->scratch = (unsigned char*)sp;
+    int cu = 0;
+    if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cu > 0)
+        ctx->n_cu = cu;
     HIP_TRY(hipMalloc(&ctx->d_flag, sizeof(int)));
     HIP_TRY(hipMalloc(&ctx->d_diag, sizeof(double) * (3 * kDiagBlocks + kMaxFrontCols + 8)));
     HIP_TRY(hipMalloc(&ctx->d_cols, sizeof(int32_t) * kMaxFrontCols));

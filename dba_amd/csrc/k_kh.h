@@ -271,12 +271,6 @@ struct KhHalo {
     }
 };
 
-// The double `off` bytes past a uniform address: one 32-bit offset register
-// instead of a 64-bit address per access.
-__device__ __forceinline__ gdouble& at_bytes(gdouble* p, unsigned off) {
-    return *(gdouble*)((DBA_GLOBAL char*)p + off);
-}
-
 // The thread's loads of a tile, left in flight: U of its cell and its halo cells
 // (U of the owner's current buffer, or the primitives a sleeping owner's ring kept).
 template <int TB>

@@ -62,19 +62,35 @@ __device__ __forceinline__ int wrapi(int i, int n) {
     return i;
 }
 
-// 27-point isotropic Laplacian from an LDS box with row stride RX and plane
-// stride PZ, in the summation order of example_Reactive_ModelB/kernel.cu:333-344.
+// 27-point isotropic Laplacian (the weights of example_Reactive_ModelB/kernel.cu:
+// 333-344) from three planes: with c the centre of a plane, e its four edge
+// neighbours and d its four diagonal ones summed,
+//     lap = (own(z) + side(z - 1)) + side(z + 1),
+//     own = -64/15 c + 7/15 e + d/10,  side = 7/15 c + e/10 + d/30,
+// so a march in z reads 8 neighbours per cell and field instead of 26; the block
+// kernels evaluate the same expressions.
+struct Plane3 {
+    double c, own, side;
+};
+
+// the sums of one plane around s[0] (row stride RX)
+template <int RX>
+__device__ __forceinline__ Plane3 plane_sums(const double* s) {
+    Plane3 p;
+    p.c = s[0];
+    const double e = (s[1] + s[-1]) + (s[RX] + s[-RX]);
+    const double d = (s[RX + 1] + s[RX - 1]) + (s[-RX + 1] + s[-RX - 1]);
+    p.own = __builtin_fma(0.1, d, __builtin_fma(7.0 / 15.0, e, -64.0 / 15.0 * p.c));
+    p.side = __builtin_fma(1.0 / 30.0, d, __builtin_fma(0.1, e, 7.0 / 15.0 * p.c));
+    return p;
+}
+
+// the Laplacian at (x, y, z) of an LDS box with row stride RX and plane stride PZ
 template <int RX, int PZ>
 __device__ __forceinline__ double lds_lap27(const double* s, int x, int y, int z, double inv_dx2) {
-#define S3(a, b, c) s[(x + (a)) + (y + (b)) * RX + (z + (c)) * PZ]
-    return inv_dx2 *
-           (-64.0 / 15.0 * S3(0, 0, 0) +
-            7.0 / 15.0 * (S3(1, 0, 0) + S3(-1, 0, 0) + S3(0, 1, 0) + S3(0, -1, 0) + S3(0, 0, 1) + S3(0, 0, -1)) +
-            0.1 * (S3(1, 1, 0) + S3(1, -1, 0) + S3(-1, 1, 0) + S3(-1, -1, 0) + S3(1, 0, 1) + S3(0, 1, 1) +
-                   S3(0, -1, 1) + S3(-1, 0, 1) + S3(1, 0, -1) + S3(0, 1, -1) + S3(0, -1, -1) + S3(-1, 0, -1)) +
-            1.0 / 30.0 * (S3(1, 1, 1) + S3(-1, 1, 1) + S3(-1, -1, 1) + S3(1, -1, 1) + S3(1, 1, -1) +
-                          S3(-1, 1, -1) + S3(-1, -1, -1) + S3(1, -1, -1)));
-#undef S3
+    const double* q = s + x + y * RX + z * PZ;
+    const double below = plane_sums<RX>(q - PZ).side, open = plane_sums<RX>(q).own + below;
+    return (open + plane_sums<RX>(q + PZ).side) * inv_dx2;
 }
 
 template <int TB, int TZ, int H>
@@ -254,17 +270,46 @@ __device__ __forceinline__ int64_t mb_own_index(const MbBlock& b, int lane) {
     return (b.x0 + lx) + (int64_t)(b.y0 + ly) * I.nx + (int64_t)(b.z0 + lz) * ((int64_t)I.nx * I.ny);
 }
 
-// The chemical potentials of the cell at (cx, cy, cz) of an LDS box of x, y, z
-// (field f at sc + f AP) into df; returns lap z for the detector
-// (example_Reactive_ModelB/kernel.cu:557-587).
+// The chemical potentials of a cell (example_Reactive_ModelB/kernel.cu:557-587)
+// from x, y, z, phi, the logarithms and the three Laplacians, in parts: what the
+// three share (the solvent's terms), then each one's own.
+__device__ __forceinline__ double mb_shared(CInst& I, double X, double Y, double Z, double logB) {
+    return -(I.chi_xb * X + I.chi_yb * Y + I.chi_zb * Z) - logB;
+}
+
+__device__ __forceinline__ double mb_mu_x(CInst& I, double Y, double Z, double B, double com, double logX, double lap) {
+    return (I.mb_cx + I.chi_xy * Y + I.chi_xz * Z + I.chi_xb * B + com + logX * I.mb_irx) - I.epsx_sq * lap;
+}
+
+__device__ __forceinline__ double mb_mu_y(CInst& I, double X, double Z, double B, double com, double logY, double lap) {
+    return (I.mb_cy + I.chi_xy * X + I.chi_yz * Z + I.chi_yb * B + com + logY * I.mb_iry) - I.epsy_sq * lap;
+}
+
+__device__ __forceinline__ double mb_mu_z(CInst& I, double X, double Y, double B, double com, double logZ, double lap,
+                                          double phi) {
+    return (I.mb_cz + I.chi_xz * X + I.chi_yz * Y + I.chi_zb * B + com + logZ * I.mb_irz -
+            I.p_gel * phi * phi * I.mb_hiomz) - I.epsz_sq * lap - I.mb_lk;
+}
+
+// The changes of x, y, z of a cell (example_Reactive_ModelB/kernel.cu:419-432):
+// dt v_f (mob_f lap mu_f -/+ the reaction)
+__device__ __forceinline__ void mb_change(CInst& I, double dfx, double dfy, double dfz, double lx_, double ly_,
+                                          double lz_, double (&ch)[3]) {
+    const double R = I.k_0 * (exp(I.n_exp * I.v_x * dfx + I.m_exp * I.v_y * dfy) - exp(I.v_z * dfz));
+    ch[0] = I.dt * I.v_x * (I.mob_x * lx_ - I.n_exp * R);
+    ch[1] = I.dt * I.v_y * (I.mob_y * ly_ - I.m_exp * R);
+    ch[2] = I.dt * I.v_z * (I.mob_z * lz_ + R);
+}
+
+// ... of the cell at (cx, cy, cz) of an LDS box (field f at sc + f AP); returns
+// lap z for the detector. Logarithms first, then one Laplacian at a time: left
+// free, the scheduler hoists all 81 LDS reads above the logarithms (250 VGPRs).
 template <int RX, int PZ, int AP>
 __device__ __forceinline__ double mb_mu_at(CInst& I, const double* sc, int cx, int cy, int cz, double phi,
                                            double (&df)[3]) {
     const int q = cx + cy * RX + cz * PZ;
     const double X = sc[q], Y = sc[AP + q], Z = sc[2 * AP + q];
     const double B = 1.0 - X - Y - Z;
-    // logarithms first, then one Laplacian at a time: left free, the
-    // scheduler hoists all 81 LDS reads above the logarithms (250 VGPRs)
     const double logB = log_f64(B), logX = log_f64(X), logY = log_f64(Y), logZ = log_f64(Z);
     __builtin_amdgcn_sched_barrier(0);
     const double inv_dx2 = I.invdx2;
@@ -273,35 +318,32 @@ __device__ __forceinline__ double mb_mu_at(CInst& I, const double* sc, int cx, i
     const double ly_ = lds_lap27<RX, PZ>(sc + AP, cx, cy, cz, inv_dx2);
     __builtin_amdgcn_sched_barrier(0);
     const double lz_ = lds_lap27<RX, PZ>(sc + 2 * AP, cx, cy, cz, inv_dx2);
-    df[0] = I.mb_cx + I.chi_xy * Y + I.chi_xz * Z + I.chi_xb * B - I.chi_xb * X - I.chi_yb * Y - I.chi_zb * Z +
-            logX / I.r_x - logB - I.epsx_sq * lx_;
-    df[1] = I.mb_cy + I.chi_xy * X + I.chi_yz * Z + I.chi_yb * B - I.chi_xb * X - I.chi_yb * Y - I.chi_zb * Z +
-            logY / I.r_y - logB - I.epsy_sq * ly_;
-    df[2] = I.mb_cz + I.chi_xz * X + I.chi_yz * Y + I.chi_zb * B - I.chi_xb * X - I.chi_yb * Y - I.chi_zb * Z +
-            logZ / I.r_z - logB - I.p_gel * phi * phi / 2.0 / I.mb_omz - I.epsz_sq * lz_ - I.mb_lk;
+    __builtin_amdgcn_sched_barrier(0);
+    const double com = mb_shared(I, X, Y, Z, logB);
+    df[0] = mb_mu_x(I, Y, Z, B, com, logX, lx_);
+    df[1] = mb_mu_y(I, X, Z, B, com, logY, ly_);
+    df[2] = mb_mu_z(I, X, Y, B, com, logZ, lz_, phi);
     return lz_;
 }
 
-// The changes of x, y, z at (cx, cy, cz) from an LDS box of the potentials
-// (example_Reactive_ModelB/kernel.cu:419-432): dt v_f (mob_f lap mu_f -/+ the reaction)
 template <int RX, int PZ, int AP>
 __device__ __forceinline__ void mb_change_at(CInst& I, const double* smu, int cx, int cy, int cz,
                                              double (&ch)[3]) {
     const double inv_dx2 = I.invdx2;
     const int mq = cx + cy * RX + cz * PZ;
     const double dfx = smu[mq], dfy = smu[AP + mq], dfz = smu[2 * AP + mq];
-    const double R = I.k_0 * (exp(I.n_exp * I.v_x * dfx + I.m_exp * I.v_y * dfy) - exp(I.v_z * dfz));
+    const double lx_ = lds_lap27<RX, PZ>(smu, cx, cy, cz, inv_dx2);
     __builtin_amdgcn_sched_barrier(0);
-    ch[0] = I.dt * I.v_x * (I.mob_x * lds_lap27<RX, PZ>(smu, cx, cy, cz, inv_dx2) - I.n_exp * R);
+    const double ly_ = lds_lap27<RX, PZ>(smu + AP, cx, cy, cz, inv_dx2);
     __builtin_amdgcn_sched_barrier(0);
-    ch[1] = I.dt * I.v_y * (I.mob_y * lds_lap27<RX, PZ>(smu + AP, cx, cy, cz, inv_dx2) - I.m_exp * R);
+    const double lz_ = lds_lap27<RX, PZ>(smu + 2 * AP, cx, cy, cz, inv_dx2);
     __builtin_amdgcn_sched_barrier(0);
-    ch[2] = I.dt * I.v_z * (I.mob_z * lds_lap27<RX, PZ>(smu + 2 * AP, cx, cy, cz, inv_dx2) + R);
+    mb_change(I, dfx, dfy, dfz, lx_, ly_, lz_, ch);
 }
 
 // Calc_mu(_wakeup) + the detector |lap z| > eps (example_Reactive_ModelB/kernel.cu:290-420)
 template <int TB, int TZ>
-__global__ __launch_bounds__(64) void modelb_mu_kernel(const WorkList wl, int sb_from) {
+__global__ __launch_bounds__(64) void modelb_mu_kernel(const WorkList wl, int from) {
     using B1 = Box1<TB, TZ>;
     constexpr int A = B1::A, NH = B1::NH, C = TB * TB * TZ, RX = B1::RX, PZ = B1::PZ, AP = B1::AP;
     static_assert(C <= 64, "at most one cell per lane");
@@ -346,8 +388,8 @@ __global__ __launch_bounds__(64) void modelb_mu_kernel(const WorkList wl, int sb
     };
 
     const int total = wl.offsets[wl.nseg];
-    // a list of at least sb_from blocks is the superblock kernels' step
-    if (total >= sb_from) return;
+    // a list of at least `from` blocks is the march's step
+    if (total >= from) return;
     const BandSweep bs = band_sweep_setup(wl, total);
     for (int round0 = 0; (int64_t)round0 * gridDim.x < total; round0 += 64) {
         const RoundList L = bs.cx ? band_sweep_round(bs, round0) : round_list(wl, total, round0);
@@ -424,10 +466,21 @@ __global__ __launch_bounds__(64) void modelb_mu_kernel(const WorkList wl, int sb
     }
 }
 
+// Lane 0 gets the sum over a block's cells (lane x + 4 y + 16 z) in the march's
+// order: up in z, then pairs in x, the pairs' pairs, the rows the same way.
+__device__ __forceinline__ double mb_block_sum(double v) {
+    double s = ((v + __shfl_down(v, 16, 64)) + __shfl_down(v, 32, 64)) + __shfl_down(v, 48, 64);
+    s += __shfl_xor(s, 1, 64);
+    s += __shfl_xor(s, 2, 64);
+    s += __shfl_xor(s, 4, 64);
+    s += __shfl_xor(s, 8, 64);
+    return s;
+}
+
 // Update(_wakeup) + copy-back + conserved change capture
 // (example_Reactive_ModelB/kernel.cu:430-560, Conserved/kernel.cu:630-702)
 template <int TB, int TZ>
-__global__ __launch_bounds__(64) void modelb_update_kernel(const WorkList wl, int sb_from) {
+__global__ __launch_bounds__(64) void modelb_update_kernel(const WorkList wl, int from) {
     using B1 = Box1<TB, TZ>;
     constexpr int A = B1::A, NH = B1::NH, C = TB * TB * TZ, RX = B1::RX, PZ = B1::PZ, AP = B1::AP;
     static_assert(C <= 64, "at most one cell per lane");
@@ -471,8 +524,8 @@ __global__ __launch_bounds__(64) void modelb_update_kernel(const WorkList wl, in
     };
 
     const int total = wl.offsets[wl.nseg];
-    // a list of at least sb_from blocks is the superblock kernels' step
-    if (total >= sb_from) return;
+    // a list of at least `from` blocks is the march's step
+    if (total >= from) return;
     const BandSweep bs = band_sweep_setup(wl, total);
     for (int round0 = 0; (int64_t)round0 * gridDim.x < total; round0 += 64) {
         const RoundList L = bs.cx ? band_sweep_round(bs, round0) : round_list(wl, total, round0);
@@ -530,7 +583,7 @@ __global__ __launch_bounds__(64) void modelb_update_kernel(const WorkList wl, in
                 part[2] = ch[2];
             }
             for (int f = 0; f < ncons; f++) {
-                const double tot = wave_sum_down(part[f]);
+                const double tot = mb_block_sum(part[f]);
                 if (lane == 0) {
                     I.tpart[(int64_t)f * I.nt + b.t] = tot;
                     I.s_tile[((int64_t)f * 2 + (pself ^ 1)) * I.nt + b.t] = I.scal[8 + f];
@@ -551,245 +604,329 @@ __global__ __launch_bounds__(64) void modelb_update_kernel(const WorkList wl, in
     }
 }
 
-// ------------------------------------------------------------ Model B, superblocks
-// Steps of one 3D Model B instance (4x4x4 blocks, no conserved shift) in which
-// at least sb_from blocks are awake run on superblocks of 2 x 2 x SZ blocks: one
-// workgroup of 4 SZ waves stages the box of a superblock's 8 x 8 x 4SZ cells and
-// their 1-cell halo once (10 x 10 x (4SZ + 2) values per field; each block's own
-// box holds 216 values for 64 cells), and wave w computes block w of the
-// superblock if that block is awake. The arithmetic per cell is mb_mu_at /
-// mb_change_at, as in the block kernels, so both give the same doubles. Each
-// superblock kernel returns at once when the list is shorter than sb_from, and
-// the block kernels when it is not.
-
-// positions of the blocks around a superblock among the 4 x 4 x 4 blocks its box
-// can touch: bit (ox + 1) + 4 (oy + 1) + 16 (oz + 1), block offsets o in [-1, 2]
-__device__ __forceinline__ int sb_code(int w) { return 21 + (w & 1) + 4 * ((w >> 1) & 1) + 16 * (w >> 2); }
-
-template <int SZ>
-struct Sb {
-    static constexpr int W = 10, WZ = 4 * SZ + 2, A = W * W * WZ;  // box sides and size
-    static constexpr int NT = 256 * SZ;                            // 4 SZ waves
-    static constexpr int NE = (A + NT - 1) / NT;                   // box elements per thread
-    static constexpr uint64_t own() {
-        uint64_t m = 0;
-        for (int w = 0; w < 4 * SZ; w++) m |= 1ull << (21 + (w & 1) + 4 * ((w >> 1) & 1) + 16 * (w >> 2));
-        return m;
-    }
+// ------------------------------------------------------------ Model B, column march
+// Steps of one 3D Model B instance in which at least `from` blocks are awake take
+// one launch: a workgroup walks a column of 32 x 12 cells up `nl` layers of
+// blocks, plane by plane. Plane p of x, y, z (with a 2-cell halo) goes through
+// LDS once; every thread keeps the plane sums of its cell, so plane p completes
+// the Laplacians of plane p - 1 and with them its potentials (six waves the
+// cells, the other two the ring around them, whose potentials their neighbours
+// compute as well); the potentials pass through LDS the same way and complete
+// plane p - 2, which is written back. Against the two launches over 8 x 8 x 4
+// boxes this replaces, the potentials never go to memory (56 bytes per cell
+// instead of the 148 measured), a Laplacian adds 8 neighbours per plane instead
+// of 26, and no halo plane is staged twice. What bounds it: FP64 issue (four
+// logarithms, two exponentials and six Laplacians per cell, 1.33 x the
+// potentials for the ring and (4 nl + 2) / 4 nl for the ends of the strip).
+//
+// Sleeping blocks: a cell of one presents the potentials it stored when it last
+// ran (aux 0..2) and is not written. A block stores its potentials as long as it
+// has not fired: plane by plane until the vote of its four waves' cells says so,
+// so a block that fires in its first plane stores that plane at most, and one
+// that does not fire stores all four, which is all that a later step reads.
+// Conserved DBA (CONS): values less the pending shift of their block, and each
+// block's change sums (mb_block_sum's order: the block kernels give the same doubles).
+struct MbMarch {
+    static constexpr int TX = 32, TY = 12, NT = 512;
+    static constexpr int CW = TX + 4, CH = TY + 4, CA = CW * CH;  // x, y, z with a 2-cell halo
+    static constexpr int MW = TX + 2, MH = TY + 2, MA = MW * MH;  // potentials with their ring
+    static constexpr int NI = TX * TY;                            // threads with a cell (six waves)
+    static constexpr int NR = MA - NI;                            // threads with a ring cell (of the last two)
+    static constexpr int BW = TX / 4 + 2, BH = TY / 4 + 2, NB = BW * BH;  // blocks around a column's layer
+    static constexpr int ML = 16, MLC = 8;                        // layers per strip, at most (conserved)
+    static_assert(NB <= 64 && NR <= NT - NI && CA <= NT + 64, "one ballot, two ring waves, two loads per thread");
 };
 
-// A superblock as every wave of its workgroup sees it (all uniform).
-struct MbSuper {
-    int X0, Y0, Z0;  // first cell
-    int tw;          // this wave's block
-    uint64_t pm;     // parity of the blocks the box touches (bit 1: buf[1] is current)
-    uint64_t am;     // awake bits of the own blocks, at the same positions
-    bool interior;   // the box needs no periodic wrap, and its offsets fit an int
-};
-
-// Each wave reads the parity and awake words itself (lane l: block l of the
-// 4 x 4 x 4 around the superblock's corner block), so no barrier is needed
-// before the box loads.
-template <int SZ>
-__device__ __forceinline__ MbSuper sb_setup(CInst& I, int sb, bool regular) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int ntx = I.ntx, nty = I.nty, nsx = ntx >> 1, nsy = nty >> 1;
-    const int sx = sb % nsx, sy = (sb / nsx) % nsy, sz = sb / (nsx * nsy);
-    MbSuper s;
-    s.X0 = sx * 8;
-    s.Y0 = sy * 8;
-    s.Z0 = sz * 4 * SZ;
-    s.tw = (2 * sx + (w & 1)) + (2 * sy + ((w >> 1) & 1)) * ntx + (SZ * sz + (w >> 2)) * ntx * nty;
-    // a one-block-thick superblock's box reaches oz = 1 at most (lanes past it read that layer)
-    const int oz = min(lane >> 4, SZ + 1) - 1;
-    const int bx = wrap1(2 * sx + (lane & 3) - 1, ntx), by = wrap1(2 * sy + ((lane >> 2) & 3) - 1, nty),
-              bz = wrap1(SZ * sz + oz, I.ntz);
-    const int tt = bx + by * ntx + bz * ntx * nty;
-    const gu64 *par0 = I.par[0], *cur0 = I.a_cur[0];
-    asm volatile("" : "+s"(par0), "+s"(cur0));
-    const uint64_t wp = par0[tt >> 6], wa = cur0[tt >> 6];
-    constexpr uint64_t kOwn = Sb<SZ>::own();
-    s.pm = __ballot((int)((wp >> (tt & 63)) & 1ull));
-    s.am = regular ? kOwn : (__ballot((int)((wa >> (tt & 63)) & 1ull)) & kOwn);
-    s.interior = s.X0 > 0 && s.X0 + 8 < I.nx && s.Y0 > 0 && s.Y0 + 8 < I.ny && s.Z0 > 0 &&
-                 s.Z0 + 4 * SZ < I.nz && (int64_t)I.nx * I.ny < (1 << 27);
-    return s;
+// v modulo n for small overshoot of any small n
+__device__ __forceinline__ int wrap_any(int v, int n) {
+    v %= n;
+    return v < 0 ? v + n : v;
 }
 
-// The superblocks of this workgroup, k = 0, 1, ...: the band sweep of the block
-// kernels over superblock columns (XCD b mod 8 sweeps its band of columns
-// z-layer by z-layer), or plain grid-stride order where the counts do not allow it.
-template <int SZ>
-__device__ __forceinline__ int sb_of(CInst& I, int k) {
-    const int G = gridDim.x, nsb = I.nt / (4 * SZ), C = (I.ntx >> 1) * (I.nty >> 1);
-    if ((G & 7) == 0 && (C & 7) == 0) {
-        const int cx = C >> 3;
-        const int64_t i = (int64_t)(blockIdx.x >> 3) + (int64_t)k * (G >> 3);
-        if (i >= (nsb >> 3)) return -1;
-        return (int)(i / cx) * C + (int)(blockIdx.x & 7) * cx + (int)(i % cx);
-    }
-    const int64_t i = (int64_t)blockIdx.x + (int64_t)k * G;
-    return i < nsb ? (int)i : -1;
-}
-
-// The thread's box elements k = tid + e NT (the last round's slots past the box
-// hold element tid's coordinates and are neither loaded nor stored).
-template <int SZ>
-struct SbElems {
-    using S = Sb<SZ>;
-    int lx[S::NE], ly[S::NE], lz[S::NE], d[S::NE], off[S::NE];
-    __device__ __forceinline__ void init(int tid, int nx, int nxy) {
-#pragma unroll
-        for (int e = 0; e < S::NE; e++) {
-            const int k0 = tid + e * S::NT, k = k0 < S::A ? k0 : tid;
-            lx[e] = k % S::W;
-            ly[e] = (k / S::W) % S::W;
-            lz[e] = k / (S::W * S::W);
-            d[e] = ((lx[e] + 3) >> 2) + 4 * ((ly[e] + 3) >> 2) + 16 * ((lz[e] + 3) >> 2);
-            off[e] = lx[e] + ly[e] * nx + lz[e] * nxy;
-        }
-    }
-    // wrapped global index of element e of the box at (X0, Y0, Z0)
-    __device__ __forceinline__ int64_t index(CInst& I, const MbSuper& s, int e) const {
-        return wrap1(s.X0 + lx[e] - 1, I.nx) + (int64_t)wrap1(s.Y0 + ly[e] - 1, I.ny) * I.nx +
-               (int64_t)wrap1(s.Z0 + lz[e] - 1, I.nz) * ((int64_t)I.nx * I.ny);
-    }
+template <bool CONS>
+struct MbMarchLds {
+    using M = MbMarch;
+    static constexpr int NL = (CONS ? M::MLC : M::ML) + 2;
+    double c[3 * M::CA], mu[3 * M::MA];
+    uint64_t vote[M::NI / 64];
+    uint64_t par[NL], act[NL];                      // parity and awake bits of the blocks of each layer
+    double shift[CONS ? NL * M::NB * 3 : 1];        // pending shift of each block
+    double part[CONS ? 3 * (M::NI / 64) * 8 : 1];   // change sums of half blocks
 };
 
-// Calc_mu(_wakeup) + the detector on superblocks (see modelb_mu_kernel)
-// 4 waves per SIMD (128 VGPRs; left free the compiler takes 129 and 3 waves):
-// measured 0.945 ms per 256^3 step with the update kernel at 5, 1.04 ms at 3
-template <int SZ>
-__global__ __launch_bounds__(Sb<SZ>::NT) __attribute__((amdgpu_waves_per_eu(4))) void modelb_mu_sb_kernel(const WorkList wl, int sb_from) {
-    using S = Sb<SZ>;
-    constexpr int A = S::A, NT = S::NT, NE = S::NE;
-    __shared__ double sc[3 * A];
+template <bool CONS>
+__global__ __launch_bounds__(MbMarch::NT) __attribute__((amdgpu_waves_per_eu(CONS ? 2 : 4))) void modelb_march_kernel(
+    const WorkList wl, int from, int nl, int ncx, int ncy) {
+    using M = MbMarch;
+    __shared__ MbMarchLds<CONS> S;
     const int total = wl.offsets[wl.nseg];
-    if (total < sb_from) return;
+    if (total < from) return;
     CInst& I = *(CInst*)wl.insts;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int nx = I.nx, ny = I.ny, nz = I.nz, ntx = I.ntx, nty = I.nty, ntz = I.ntz;
+    const int64_t nxy = (int64_t)nx * ny;
     const bool regular = I.mode == 0;
-    const int nx = I.nx, nxy = I.nx * I.ny;
-    SbElems<SZ> el;
-    el.init(tid, nx, nxy);
-    const int cx = 4 * (w & 1) + (lane & 3), cy = 4 * ((w >> 1) & 1) + ((lane >> 2) & 3), cz = 4 * (w >> 2) + (lane >> 4);
-    const int code = sb_code(w);
-    for (int k = 0;; k++) {
-        const int sb = sb_of<SZ>(I, k);
-        if (sb < 0) break;
-        const MbSuper s = sb_setup<SZ>(I, sb, regular);
-        if (!s.am) continue;
-        const bool awake = (s.am >> code) & 1ull;
-        const int pw = (int)(s.pm >> code) & 1;
-        const int64_t own = (s.X0 + cx) + (int64_t)(s.Y0 + cy) * nx + (int64_t)(s.Z0 + cz) * nxy;
-        double h[NE][3];
-        if (s.interior && (s.pm == 0ull || s.pm == ~0ull)) {
-            // no wrap, and every block the box touches current in one buffer
-            const int p = (int)(s.pm & 1ull);
-            const int64_t base = (s.X0 - 1) + (int64_t)(s.Y0 - 1) * nx + (int64_t)(s.Z0 - 1) * nxy;
-            const gdouble *b0 = I.buf[p][0] + base, *b1 = I.buf[p][1] + base, *b2 = I.buf[p][2] + base;
+    const int item = xcd_deal(blockIdx.x, gridDim.x, 0, gridDim.x);
+    const int ncol = ncx * ncy, col = item % ncol;
+    const int l0 = (item / ncol) * nl, nlay = min(nl, ntz - l0);
+    const int x0 = (col % ncx) * M::TX, y0 = (col / ncx) * M::TY;
+    const double inv_dx2 = I.invdx2;
+
+    // parity and awake bits of the blocks around each layer l0 - 1 .. l0 + nlay
+    for (int k = wid; k < nlay + 2; k += M::NT / 64) {
+        const int l = lane < M::NB ? lane : 0;
+        const int tt = wrap_any(x0 / 4 + l % M::BW - 1, ntx) + wrap_any(y0 / 4 + l / M::BW - 1, nty) * ntx +
+                       wrap_any(l0 + k - 1, ntz) * ntx * nty;
+        const gu64 *par0 = I.par[0], *cur0 = I.a_cur[0];
+        asm volatile("" : "+s"(par0), "+s"(cur0));
+        const uint64_t wp = par0[tt >> 6], wa = cur0[tt >> 6];
+        const int pb = (int)((wp >> (tt & 63)) & 1ull);
+        const uint64_t pm = __ballot(pb);
+        const uint64_t am = regular ? ~0ull : __ballot((int)((wa >> (tt & 63)) & 1ull));
+        if (lane == 0) {
+            S.par[k] = pm;
+            S.act[k] = am;
+        }
+        if (CONS && lane < M::NB)
 #pragma unroll
-            for (int e = 0; e < NE; e++) {
-                if (e + 1 < NE || tid + e * NT < A) {
-                    h[e][0] = b0[el.off[e]];
-                    h[e][1] = b1[el.off[e]];
-                    h[e][2] = b2[el.off[e]];
-                }
-            }
+            for (int f = 0; f < 3; f++)
+                S.shift[(k * M::NB + lane) * 3 + f] =
+                    I.scal[8 + f] - I.s_tile[((int64_t)f * 2 + pb) * I.nt + tt];
+    }
+    __syncthreads();
+    // the blocks a column owns in a layer, and whether the strip has any to run
+    const int bw = min(M::TX, nx - x0) / 4, bh = min(M::TY, ny - y0) / 4;
+    uint64_t own = 0ull;
+    for (int j = 0; j < bh; j++) own |= ((1ull << bw) - 1ull) << (M::BW * (j + 1) + 1);
+    uint64_t run = 0ull;
+    for (int k = 1; k <= nlay; k++) run |= S.act[k] & own;
+    run = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(run >> 32)) << 32) |
+          (uint32_t)__builtin_amdgcn_readfirstlane((int)run);
+    if (run == 0ull) return;
+    // this thread's loads: region positions tid and, for the last wave, 512 + lane
+    const bool two = tid >= M::NT - 64;
+    int lbit[2];
+    unsigned loff[2];
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+        const int k = s == 0 ? tid : M::NT + lane, lx = k % M::CW, ly = k / M::CW;
+        lbit[s] = ((lx + 2) >> 2) + M::BW * ((ly + 2) >> 2);
+        loff[s] = (unsigned)(wrap_any(x0 + lx - 2, nx) + wrap_any(y0 + ly - 2, ny) * nx) * 8u;
+    }
+    // this thread's cell in the region of the potentials: a cell of the column, or of its ring
+    int mx, my;
+    if (tid < M::NI) {
+        mx = 1 + (tid & 31);
+        my = 1 + (tid >> 5);
+    } else {
+        const int r = min(tid - M::NI, M::NR - 1);
+        if (r < 2 * M::MW) {
+            mx = r < M::MW ? r : r - M::MW;
+            my = r < M::MW ? 0 : M::MH - 1;
         } else {
+            const int k = r - 2 * M::MW;
+            mx = k < M::TY ? 0 : M::MW - 1;
+            my = 1 + (k < M::TY ? k : k - M::TY);
+        }
+    }
+    const bool cell = tid < M::NI;
+    const bool mine = cell && mx - 1 < nx - x0 && my - 1 < ny - y0;  // a cell of the grid this column owns
+    const int mbit = ((mx + 3) >> 2) + M::BW * ((my + 3) >> 2);
+    const unsigned moff = (unsigned)(wrap_any(x0 + mx - 1, nx) + wrap_any(y0 + my - 1, ny) * nx) * 8u;
+    const double* sc = S.c + (mx + 1) + (my + 1) * M::CW;
+    double* sm = S.mu + mx + my * M::MW;
+
+    double v[2][3];
+    auto zof = [&](int p) {  // plane p of the strip (p from -2 to 4 nlay + 1), wrapped
+        int z = 4 * l0 + p;
+        z = z < 0 ? z + nz : z;
+        return z >= nz ? z - nz : z;
+    };
+    auto bits = [&](const uint64_t* m, int p) {
+        const uint64_t w = m[(p + 4) >> 2];
+        return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(w >> 32)) << 32) |
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)w);
+    };
+    // both buffers' plane of field f, and the one lane data picks: pointers held in
+    // registers, or the compiler makes a load of the pointer out of the choice
+    auto planes = [&](int f, int64_t zo, gdouble*& b0, gdouble*& b1) {
+        b0 = I.buf[0][f] + zo;
+        b1 = I.buf[1][f] + zo;
+        asm volatile("" : "+s"(b0), "+s"(b1));
+    };
+    auto load = [&](int p) {
+        const int64_t zo = (int64_t)zof(p) * nxy;
+        const uint64_t pm = bits(S.par, p);
+        const bool q0 = (pm >> lbit[0]) & 1ull, q1 = (pm >> lbit[1]) & 1ull;
 #pragma unroll
-            for (int e = 0; e < NE; e++) {
-                if (e + 1 < NE || tid + e * NT < A) {
-                    const int64_t gi = el.index(I, s, e);
-                    const int pp = (int)(s.pm >> el.d[e]) & 1;
-                    for (int f = 0; f < 3; f++) h[e][f] = I.buf[pp][f][gi];
-                }
+        for (int f = 0; f < 3; f++) {
+            gdouble *b0, *b1;
+            planes(f, zo, b0, b1);
+            v[0][f] = at_bytes(q0 ? b1 : b0, loff[0]);
+            if (two) v[1][f] = at_bytes(q1 ? b1 : b0, loff[1]);
+        }
+    };
+    auto deposit = [&](int p) {
+        if (CONS) {
+            const double* sh = S.shift + ((p + 4) >> 2) * M::NB * 3;
+#pragma unroll
+            for (int f = 0; f < 3; f++) {
+                v[0][f] -= sh[lbit[0] * 3 + f];
+                if (two) v[1][f] -= sh[lbit[1] * 3 + f];
             }
         }
+#pragma unroll
+        for (int f = 0; f < 3; f++) {
+            S.c[f * M::CA + tid] = v[0][f];
+            if (two) S.c[f * M::CA + M::NT + lane] = v[1][f];
+        }
+    };
+
+    // of the last plane of x, y, z (c) and of the potentials (m): the value, what it
+    // adds to its neighbour planes, its Laplacian without the plane above; and
+    // x, y, z of the plane before
+    double cv[3], cs[3], co[3], mv[3], ms[3], mo[3], c2[3];
+    double part[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int f = 0; f < 3; f++) cv[f] = cs[f] = co[f] = mv[f] = ms[f] = mo[f] = c2[f] = 0.0;
+    int fired = 0;
+    const int last = 4 * nlay + 1;
+    load(-2);
+    deposit(-2);
+#pragma unroll 1
+    for (int p = -2; p <= last; p++) {
+        lds_barrier();
         double phi = 0.0;
-        if (awake) phi = I.buf[pw][3][own];
+        if (p >= 0) {
+            const int64_t zo = (int64_t)zof(p - 1) * nxy;
+            gdouble *b0, *b1;
+            planes(3, zo, b0, b1);
+            phi = at_bytes((bits(S.par, p - 1) >> mbit) & 1ull ? b1 : b0, moff);
+        }
+        // on its way until the end of the iteration (after phi: loads return in order)
+        if (p < last) load(p + 1);
+        // the Laplacians of plane p - 1 and its potentials
+        double lap[3], df[3];
+        const bool up = p >= 0;
+        const bool wakes = (bits(S.act, p - 1 < -2 ? -2 : p - 1) >> mbit) & 1ull;  // this cell's block runs
 #pragma unroll
-        for (int e = 0; e < NE; e++)
-            if (tid + e * NT < A)
-                for (int f = 0; f < 3; f++) sc[f * A + tid + e * NT] = h[e][f];
-        __syncthreads();
-        if (awake) {
-            double df[3];
-            const double lz_ = mb_mu_at<S::W, S::W * S::W, A>(I, sc, cx + 1, cy + 1, cz + 1, phi, df);
-            I.aux[0][own] = df[0];
-            I.aux[1][own] = df[1];
-            I.aux[2][own] = df[2];
-            if (I.mode != 0) {
-                const int any = __ballot(fabs(lz_) > I.thresh_a) != 0ull;
-                if (lane == 0) I.nflag[0][s.tw] = (uint8_t)any;
+        for (int f = 0; f < 3; f++) {
+            const Plane3 n = plane_sums<M::CW>(sc + f * M::CA);
+            lap[f] = (co[f] + n.side) * inv_dx2;
+            co[f] = n.own + cs[f];
+            cs[f] = n.side;
+            df[f] = cv[f];
+            cv[f] = n.c;
+        }
+        const double X = df[0], Y = df[1], Z = df[2];
+        if (up) {
+            if (wakes) {
+                // one logarithm at a time: together they spill
+                const double B = 1.0 - X - Y - Z;
+                const double com = mb_shared(I, X, Y, Z, log_f64(B));
+                __builtin_amdgcn_sched_barrier(0);
+                df[0] = mb_mu_x(I, Y, Z, B, com, log_f64(X), lap[0]);
+                __builtin_amdgcn_sched_barrier(0);
+                df[1] = mb_mu_y(I, X, Z, B, com, log_f64(Y), lap[1]);
+                __builtin_amdgcn_sched_barrier(0);
+                df[2] = mb_mu_z(I, X, Y, B, com, log_f64(Z), lap[2], phi);
+                __builtin_amdgcn_sched_barrier(0);
+            } else {
+                const int64_t zo = (int64_t)zof(p - 1) * nxy;
+#pragma unroll
+                for (int f = 0; f < 3; f++) df[f] = at_bytes(I.aux[f] + zo, moff);
+            }
+            if (tid < M::NI + M::NR)
+#pragma unroll
+                for (int f = 0; f < 3; f++) sm[f * M::MA] = df[f];
+            if (cell && !regular) {
+                const uint64_t w = __ballot(mine && wakes && fabs(lap[2]) > I.thresh_a);
+                if (lane == 0) S.vote[wid] = w;
             }
         }
-        __syncthreads();
-    }
-}
-
-// Update(_wakeup) + copy-back on superblocks (see modelb_update_kernel)
-// 5 waves per SIMD (96 VGPRs, no spills; 4 left free)
-template <int SZ>
-__global__ __launch_bounds__(Sb<SZ>::NT) __attribute__((amdgpu_waves_per_eu(5))) void modelb_update_sb_kernel(const WorkList wl, int sb_from) {
-    using S = Sb<SZ>;
-    constexpr int A = S::A, NT = S::NT, NE = S::NE;
-    __shared__ double smu[3 * A];
-    const int total = wl.offsets[wl.nseg];
-    if (total < sb_from) return;
-    CInst& I = *(CInst*)wl.insts;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const bool regular = I.mode == 0;
-    const int nx = I.nx, nxy = I.nx * I.ny;
-    SbElems<SZ> el;
-    el.init(tid, nx, nxy);
-    const int cx = 4 * (w & 1) + (lane & 3), cy = 4 * ((w >> 1) & 1) + ((lane >> 2) & 3), cz = 4 * (w >> 2) + (lane >> 4);
-    const int code = sb_code(w);
-    for (int k = 0;; k++) {
-        const int sb = sb_of<SZ>(I, k);
-        if (sb < 0) break;
-        const MbSuper s = sb_setup<SZ>(I, sb, regular);
-        if (!s.am) continue;
-        const bool awake = (s.am >> code) & 1ull;
-        const int pw = (int)(s.pm >> code) & 1;
-        const int64_t own = (s.X0 + cx) + (int64_t)(s.Y0 + cy) * nx + (int64_t)(s.Z0 + cz) * nxy;
-        double h[NE][3];
-        if (s.interior) {
-            const int64_t base = (s.X0 - 1) + (int64_t)(s.Y0 - 1) * nx + (int64_t)(s.Z0 - 1) * nxy;
-            const gdouble *a0 = I.aux[0] + base, *a1 = I.aux[1] + base, *a2 = I.aux[2] + base;
+        lds_barrier();
+        if (cell && up) {
+            // plane p - 1 of the potentials: stored until the block is known to have fired
+            const int q = p - 1;
+            if (!regular && mine && q >= 0 && q < 4 * nlay) {
+                // the block's cells in this plane: four lanes in two rows, of this wave and its partner
+                const uint64_t w = S.vote[wid & ~1] | S.vote[wid | 1];
+                const uint64_t m = (0xFull | 0xFull << 32) << (tid & 28);
+                fired |= (w & m) != 0ull;
+                if (wakes && !fired) {
+                    const int64_t zo = (int64_t)zof(q) * nxy;
 #pragma unroll
-            for (int e = 0; e < NE; e++) {
-                if (e + 1 < NE || tid + e * NT < A) {
-                    h[e][0] = a0[el.off[e]];
-                    h[e][1] = a1[el.off[e]];
-                    h[e][2] = a2[el.off[e]];
+                    for (int f = 0; f < 3; f++) at_bytes(I.aux[f] + zo, moff) = df[f];
+                }
+                if ((q & 3) == 3) {
+                    if (wakes && (tid & 3) == 0 && ((tid >> 5) & 3) == 0)
+                        I.nflag[0][(x0 + mx - 1) / 4 + ((y0 + my - 1) / 4) * ntx + (l0 + q / 4) * ntx * nty] =
+                            (uint8_t)fired;
+                    fired = 0;
                 }
             }
-        } else {
+            // the changes of plane p - 2
 #pragma unroll
-            for (int e = 0; e < NE; e++) {
-                if (e + 1 < NE || tid + e * NT < A) {
-                    const int64_t gi = el.index(I, s, e);
-                    for (int f = 0; f < 3; f++) h[e][f] = I.aux[f][gi];
+            for (int f = 0; f < 3; f++) {
+                const Plane3 n = plane_sums<M::MW>(sm + f * M::MA);
+                lap[f] = (mo[f] + n.side) * inv_dx2;
+                mo[f] = n.own + ms[f];
+                ms[f] = n.side;
+                df[f] = mv[f];
+                mv[f] = n.c;
+            }
+            if (p >= 2) {
+                const int zr = p - 2;
+                const bool ran = mine && ((bits(S.act, zr) >> mbit) & 1ull);
+                double ch[3];
+                mb_change(I, df[0], df[1], df[2], lap[0], lap[1], lap[2], ch);
+                if (ran) {
+                    const int64_t zo = (int64_t)zof(zr) * nxy;
+                    const bool q = (bits(S.par, zr) >> mbit) & 1ull;
+#pragma unroll
+                    for (int f = 0; f < 3; f++) {
+                        gdouble *b0, *b1;
+                        planes(f, zo, b0, b1);
+                        at_bytes(q ? b0 : b1, moff) = c2[f] + ch[f];
+                    }
+                }
+                if (CONS) {
+#pragma unroll
+                    for (int f = 0; f < 3; f++) part[f] += ran ? ch[f] : 0.0;
+                    if ((zr & 3) == 3) {
+#pragma unroll
+                        for (int f = 0; f < 3; f++) {
+                            double s = part[f];
+                            s += __shfl_xor(s, 1, 64);
+                            s += __shfl_xor(s, 2, 64);
+                            s += __shfl_xor(s, 32, 64);
+                            if ((lane & 35) == 0) S.part[(f * (M::NI / 64) + wid) * 8 + (lane >> 2)] = s;
+                            part[f] = 0.0;
+                        }
+                    }
                 }
             }
         }
-        double v[3] = {0.0, 0.0, 0.0};
-        if (awake)
-            for (int f = 0; f < 3; f++) v[f] = I.buf[pw][f][own];
-#pragma unroll
-        for (int e = 0; e < NE; e++)
-            if (tid + e * NT < A)
-                for (int f = 0; f < 3; f++) smu[f * A + tid + e * NT] = h[e][f];
-        __syncthreads();
-        if (awake) {
-            double ch[3];
-            mb_change_at<S::W, S::W * S::W, A>(I, smu, cx + 1, cy + 1, cz + 1, ch);
-            I.buf[pw ^ 1][0][own] = v[0] + ch[0];
-            I.buf[pw ^ 1][1][own] = v[1] + ch[1];
-            I.buf[pw ^ 1][2][own] = v[2] + ch[2];
+        if (CONS && p >= 2 && ((p - 2) & 3) == 3) {
+            lds_barrier();
+            // a block's change sums: its two waves' halves
+            if (tid < 3 * (M::TY / 4) * 8) {
+                const int f = tid / (8 * (M::TY / 4)), r = tid % (8 * (M::TY / 4)), j = r / 8, i = r % 8;
+                const int bit = (i + 1) + M::BW * (j + 1), lay = (p - 2) / 4 + 1;
+                if (i < bw && j < bh && ((S.act[lay] >> bit) & 1ull)) {
+                    const int t = x0 / 4 + i + (y0 / 4 + j) * ntx + (l0 + lay - 1) * ntx * nty;
+                    const int b = (int)((S.par[lay] >> bit) & 1ull);
+                    const double* h = S.part + (f * (M::NI / 64) + 2 * j) * 8 + i;
+                    I.tpart[(int64_t)f * I.nt + t] = h[0] + h[8];
+                    I.s_tile[((int64_t)f * 2 + (b ^ 1)) * I.nt + t] = I.scal[8 + f];
+                }
+            }
         }
-        __syncthreads();
+        c2[0] = X;
+        c2[1] = Y;
+        c2[2] = Z;
+        // every read of plane p's sums was before the second barrier
+        if (p < last) deposit(p + 1);
     }
 }
 

@@ -415,13 +415,86 @@ struct WorkList {
     const uint64_t* solo_rec; // ... its neighbour records
     int solo_nt;              // ... and its tile count (0 otherwise)
     int one_inst;             // one instance: segment s holds its tiles from s kSegTiles on
+    // Folded merge (kFoldSegs): the segment counts, from which every workgroup makes
+    // the offsets itself; null otherwise
+    const int32_t* counts;
 };
+
+// Groups of several segments in which no step needs the merged sums of the one
+// before (a conserved shift, a CFL time step) go without a merge launch: the step kernel's workgroups scan the
+// segment counts themselves, and the instance sums of a step are merged by a wave
+// of the next step's finalize (the last ones of a run by the merge kernel). The
+// launch cost 4.2 to 6.6 us of every step. The 2D kernels keep one segment's
+// offset per lane (up to 64 segments), since 1 KB more of LDS took a workgroup
+// from each CU (KH on 8 x 8 tiles 26.4 -> 28.8 us per step); the 3D kernels, whose
+// grids have hundreds, a table in LDS.
+constexpr int kFoldLanes = 64, kFoldSegs = 256;
+
+struct FoldLds {
+    int o[kFoldSegs + 4];  // exclusive prefix of the counts; [kFoldSegs] the total
+};
+
+struct Fold {
+    int ex;        // lane k: the offset of segment k (at most 64 segments)
+    const int* o;  // the table, for kernels that have one
+};
+
+__device__ __forceinline__ int wave_scan_add(int v) {  // inclusive
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(v, off, 64);
+        if (lane >= off) v += y;
+    }
+    return v;
+}
+
+// The list length; with folded merges also the offsets (all threads call it). The
+// counts are padded with zeros to kFoldSegs.
+template <bool FOLD = true>
+__device__ __forceinline__ int work_open(const WorkList& w, Fold& F, FoldLds* L = nullptr) {
+    F.o = nullptr;
+    F.ex = 0;
+    if (!FOLD || !w.counts) return w.offsets[w.nseg];
+    if (!L) {
+        const int v = w.counts[threadIdx.x & 63], incl = wave_scan_add(v);
+        F.ex = incl - v;
+        return __builtin_amdgcn_readlane(incl, 63);
+    }
+    F.o = L->o;
+    if (threadIdx.x < 64) {
+        const int4 v = ((const int4*)w.counts)[threadIdx.x];
+        const int sum = v.x + v.y + v.z + v.w, incl = wave_scan_add(sum), ex = incl - sum;
+        ((int4*)L->o)[threadIdx.x] = int4{ex, ex + v.x, ex + v.x + v.y, ex + v.x + v.y + v.z};
+        if (threadIdx.x == 63) L->o[kFoldSegs] = incl;
+    }
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(L->o[kFoldSegs]);
+}
+
+// The segment of an item every lane of the wave holds (as find_slot_wave): the
+// number of segments k >= 1 that start at or below it. Segments past the last one
+// start at the total, above every item.
+__device__ __forceinline__ int find_slot_fold(const Fold& F, int item, int* off_s) {
+    const int lane = threadIdx.x & 63;
+    if (!F.o) {
+        const int cnt = __popcll(__ballot(lane > 0 && F.ex <= item));
+        *off_s = __builtin_amdgcn_readlane(F.ex, cnt);
+        return cnt;
+    }
+    const int4 v = ((const int4*)F.o)[lane];
+    const int cnt = __popcll(__ballot(lane > 0 && v.x <= item)) + __popcll(__ballot(v.y <= item)) +
+                    __popcll(__ballot(v.z <= item)) + __popcll(__ballot(v.w <= item));
+    *off_s = F.o[cnt];
+    return cnt;
+}
 
 // Item -> (instance, tile, neighbour record); false once the item is past the
 // list. `total` is offsets[nseg], loaded by the caller once per workgroup.
 // 3D models pass want_rec = false (their records are not written).
-__device__ __forceinline__ bool next_item(const WorkList& w, int item, int total, CInst** I, int* t,
-                                          uint64_t* rec, bool want_rec = true) {
+template <bool FOLD>
+__device__ __forceinline__ bool next_item(const WorkList& w, const Fold& F, int item, int total, CInst** I,
+                                          int* t, uint64_t* rec, bool want_rec = true) {
     if (w.solo_nt > 0) {
         if (item >= w.solo_nt) return false;
         // in bounds; loaded before the length check so all three loads overlap
@@ -436,7 +509,8 @@ __device__ __forceinline__ bool next_item(const WorkList& w, int item, int total
     }
     if (item >= total) return false;
     int s = 0, off = 0;
-    if (w.nseg > 1) s = find_slot_wave(w.offsets, w.nseg, item, &off);
+    if (FOLD && w.counts) s = find_slot_fold(F, item, &off);
+    else if (w.nseg > 1) s = find_slot_wave(w.offsets, w.nseg, item, &off);
     int inst = 0, tile0 = s * kSegTiles;
     if (!w.one_inst) {
         const Seg sg = w.segs[s];
@@ -487,8 +561,9 @@ __device__ __forceinline__ void work_begin(const WorkList& w, WorkCursor& c, boo
     }
 }
 
-__device__ __forceinline__ bool work_next(const WorkList& w, WorkCursor& c, int total, CInst** I, int* t,
-                                          uint64_t* rec, bool want_rec = true) {
+template <bool FOLD = true>
+__device__ __forceinline__ bool work_next(const WorkList& w, const Fold& F, WorkCursor& c, int total,
+                                          CInst** I, int* t, uint64_t* rec, bool want_rec = true) {
     const int G = gridDim.x;
     while (c.base < total) {
         const int item = xcd_deal(blockIdx.x, G, c.base, min(G, total - c.base));
@@ -502,7 +577,7 @@ __device__ __forceinline__ bool work_next(const WorkList& w, WorkCursor& c, int 
             c.spec_item = -1;
             return true;
         }
-        return next_item(w, item, total, I, t, rec, want_rec);
+        return next_item<FOLD>(w, F, item, total, I, t, rec, want_rec);
     }
     return false;
 }
@@ -516,7 +591,7 @@ struct RoundList {
     int t;           // lane j: that block
 };
 
-__device__ __forceinline__ RoundList round_list(const WorkList& w, int total, int round0) {
+__device__ __forceinline__ RoundList round_list(const WorkList& w, const Fold& F, int total, int round0) {
     const int G = gridDim.x, lane = threadIdx.x & 63;
     const int64_t base = (int64_t)(round0 + lane) * G;
     int item = -1;
@@ -528,10 +603,17 @@ __device__ __forceinline__ RoundList round_list(const WorkList& w, int total, in
         if (w.solo_nt > 0) {
             L.t = w.solo_seg[item];
         } else {
-            const int s = w.nseg == 1 ? 0 : find_slot(w.offsets, w.nseg, item);
+            int s = 0, off = 0;
+            if (w.counts) {
+                s = find_slot(F.o, w.nseg, item);
+                off = F.o[s];
+            } else if (w.nseg > 1) {
+                s = find_slot(w.offsets, w.nseg, item);
+                off = w.offsets[s];
+            }
             const Seg sg = w.segs[s];
             L.inst = sg.inst;
-            L.t = w.insts[sg.inst].seg[sg.tile0 + (item - w.offsets[s])];
+            L.t = w.insts[sg.inst].seg[sg.tile0 + (item - off)];
         }
     }
     L.valid = __ballot(item >= 0);

@@ -117,6 +117,7 @@ struct Group {
     int32_t* d_offsets = nullptr;
     int32_t* d_dmap = nullptr;    // single-launch steps of several instances or segments: instance << 24 | tile
     int nseg = 0;
+    bool fold = false;            // steps without a merge launch (WorkList::counts)
     int64_t total_tiles = 0;
     int grid = 0;
     uint64_t last_use = 0;
@@ -545,9 +546,25 @@ dba_status get_group(dba_ctx* ctx, const std::vector<int>& ids, Group** out) {
     HIP_TRY(hipMemcpyAsync(g->d_segs, segs.data(), sizeof(Seg) * ns, hipMemcpyHostToDevice, ctx->setup));
     HIP_TRY(hipMalloc(&g->d_isegs, sizeof(InstSegs) * n));
     HIP_TRY(hipMemcpyAsync(g->d_isegs, isegs.data(), sizeof(InstSegs) * n, hipMemcpyHostToDevice, ctx->setup));
-    HIP_TRY(hipMalloc(&g->d_parts, sizeof(SegPart) * ns));
-    HIP_TRY(hipMemsetAsync(g->d_parts, 0, sizeof(SegPart) * ns, ctx->setup));
-    HIP_TRY(hipMalloc(&g->d_counts, sizeof(int32_t) * ns));
+    // folded merges: as many segments as the kernels' offsets hold, and no instance
+    // whose step needs the merged sums of the one before (a conserved shift, a CFL
+    // time step). KH on 16 x 16 tiles keeps the merge launch: its kernel has no
+    // registers left for the offsets (2048^2 at a fixed time step 164.6 us per step
+    // with the merge launch, 168.2 folded; 8 x 8 tiles 26.4 and 24.8 us at 512^2)
+    const bool three_d = g->model == DBA_MODEL_DENDRITE_K94 || g->model == DBA_MODEL_MODELB;
+    g->fold = ns > 1 && ns <= (size_t)(three_d ? kFoldSegs : kFoldLanes) &&
+              !(g->model == DBA_MODEL_KH && g->tile != 8);
+    for (int id : ids) {
+        const dba_params& p = ctx->inst.at(id)->p;
+        if (p.mode == DBA_MODE_CONSERVED || (p.model == DBA_MODEL_KH && p.dt_mode == DBA_DT_CFL)) g->fold = false;
+    }
+    // two sets of partials (folded merges read one step's while the next one's are
+    // written); counts padded with zeros to a whole scan
+    const size_t nc = std::max<size_t>(ns, kFoldSegs);
+    HIP_TRY(hipMalloc(&g->d_parts, sizeof(SegPart) * 2 * ns));
+    HIP_TRY(hipMemsetAsync(g->d_parts, 0, sizeof(SegPart) * 2 * ns, ctx->setup));
+    HIP_TRY(hipMalloc(&g->d_counts, sizeof(int32_t) * nc));
+    HIP_TRY(hipMemsetAsync(g->d_counts, 0, sizeof(int32_t) * nc, ctx->setup));
     HIP_TRY(hipMalloc(&g->d_offsets, sizeof(int32_t) * (ns + 1)));
     HIP_TRY(hipMemsetAsync(g->d_offsets, 0, sizeof(int32_t) * (ns + 1), ctx->setup));
     std::vector<int32_t> dmap;
@@ -573,9 +590,12 @@ dba_status get_group(dba_ctx* ctx, const std::vector<int>& ids, Group** out) {
 
 // ---------------------------------------------------------------- launches
 
+// Segment partials of step `step` of a run (folded merges alternate between two sets).
+SegPart* parts_of(const Group* g, int step) { return g->d_parts + (g->fold && (step & 1) ? g->nseg : 0); }
+
 WorkList wl_of(const Group* g) {
     return WorkList{g->d_insts, g->d_segs, g->d_offsets, g->nseg, g->solo_seg, g->solo_rec, g->solo_nt,
-                    g->ids.size() == 1 ? 1 : 0};
+                    g->ids.size() == 1 ? 1 : 0, g->fold ? g->d_counts : nullptr};
 }
 
 template <int TB, int NT>
@@ -753,15 +773,19 @@ void launch_dense(const Group* g, hipStream_t s, int first, int step) {
     }
 }
 
-void launch_finalize(const Group* g, hipStream_t s, int rotate) {
+// The end of step `step` of a run (rotate), or the rebuilt worklists of the current
+// awake sets. last: no step follows, so the instance sums are merged here.
+void launch_finalize(const Group* g, hipStream_t s, int rotate, int step, bool last) {
+    SegPart* parts = parts_of(g, step);
+    const SegPart* pend = g->fold && rotate && step > 0 ? parts_of(g, step - 1) : nullptr;
     hipLaunchKernelGGL(finalize_kernel, dim3((unsigned)g->nseg), dim3(kFinNT), 0, s, g->d_insts, g->d_segs,
-                       g->nseg, g->d_parts, g->d_counts, g->d_offsets, rotate, g->ids.size() == 1 ? 1 : 0);
-    if (g->nseg > 1) {
+                       g->nseg, parts, g->d_counts, g->d_offsets, rotate, g->ids.size() == 1 ? 1 : 0, pend);
+    if (g->nseg > 1 && (!g->fold || last)) {
         // workgroup 0 scans the segment counts; the others reduce 16 instances each
         const int n_inst = (int)g->ids.size();
         const unsigned wgs = 1u + (unsigned)((n_inst + kFinNT / 64 - 1) / (kFinNT / 64));
         hipLaunchKernelGGL(finalize_merge_kernel, dim3(wgs), dim3(kFinNT), 0, s, g->d_insts, g->nseg, g->d_isegs,
-                           n_inst, g->d_parts, g->d_counts, g->d_offsets, rotate);
+                           n_inst, parts, g->d_counts, g->d_offsets, rotate);
     }
 }
 
@@ -847,7 +871,7 @@ dba_status enqueue_steps(dba_ctx* ctx, const std::vector<Group*>& gs, int n_step
             launch_step(g, ctx->stream);
             LAUNCH_CHECK();
             if (timed) (void)hipEventRecord(b, ctx->stream);
-            launch_finalize(g, ctx->stream, 1);
+            launch_finalize(g, ctx->stream, 1, s, s + 1 == n_steps);
             LAUNCH_CHECK();
             if (timed) {
                 (void)hipEventRecord(c, ctx->stream);
@@ -881,7 +905,7 @@ dba_status prepare_groups(dba_ctx* ctx, const int32_t* ids, int32_t n_ids, std::
     }
     // (re)build the worklists from the current awake sets
     for (Group* g : *gs) {
-        launch_finalize(g, ctx->stream, 0);
+        launch_finalize(g, ctx->stream, 0, 0, true);
         LAUNCH_CHECK();
     }
     return DBA_OK;

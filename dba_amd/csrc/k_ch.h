@@ -395,13 +395,14 @@ __global__ __launch_bounds__(NT) void ch_step_kernel(const WorkList wl) {
     __shared__ NbTable nb;
 
     WorkCursor cur;
+    Fold FO;
     work_begin(wl, cur, true);
-    const int total = wl.offsets[wl.nseg];
+    const int total = work_open(wl, FO);
     for (;;) {
         CInst* Ip;
         int t;
         uint64_t rec;
-        if (!work_next(wl, cur, total, &Ip, &t, &rec)) break;
+        if (!work_next(wl, FO, cur, total, &Ip, &t, &rec)) break;
         CInst& I = *Ip;
         if (ch_partial<TB, PART>(I, t)) {
             if (I.stencil != 5) ch_tile<TB, NT, true, true, PART>(I, t, rec, nb, sc, smu, sred, sflag);

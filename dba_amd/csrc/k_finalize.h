@@ -131,6 +131,49 @@ __device__ __forceinline__ void finish_instance(CInst& J, int64_t listlen, unsig
     if (J.model == 5 && J.dt_mode == 1) J.scal[1] = J.cfl * (J.dx / vmax);
 }
 
+// Merge of one instance's segment partials (segments [first, first + count)) by
+// one wave: lanes stride over the segments, then a fixed-shape shuffle tree (the
+// same order on every run, and for a one-segment instance exactly that segment's
+// partial). counts: null leaves the list length as it is.
+__device__ __forceinline__ void merge_instance(CInst& J, int first, int count, const SegPart* __restrict__ parts,
+                                               const int32_t* __restrict__ counts, int rotate) {
+    const int lane = threadIdx.x & 63;
+    // the instance's scalars and counters, loaded ahead of the reduction
+    double sc[16];
+    int64_t step = 0, upd = 0, len = 0;
+    if (lane == 0) {
+        for (int kk = 0; kk < 16; kk++) sc[kk] = J.scal[kk];
+        step = J.ctr[0];
+        upd = J.ctr[1];
+        len = J.ctr[2];
+    }
+    int64_t ll = 0;
+    unsigned long long q0 = 0, q1 = 0, qc = 0;
+    double cs[kMaxFields] = {0.0, 0.0, 0.0, 0.0};
+    double vm = 0.0;
+    const int ncs = J.ncons;
+    for (int q = first + lane; q < first + count; q += 64) {
+        if (counts) ll += counts[q];
+        if (rotate) {
+            q0 += parts[q].c0;
+            q1 += parts[q].c1;
+            qc += parts[q].cells;
+            for (int f = 0; f < ncs; f++) cs[f] += parts[q].csum[f];
+            vm = fmax(vm, parts[q].vmax);
+        }
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        ll += __shfl_down(ll, off, 64);
+        q0 += __shfl_down(q0, off, 64);
+        q1 += __shfl_down(q1, off, 64);
+        qc += __shfl_down(qc, off, 64);
+        for (int f = 0; f < kMaxFields; f++) cs[f] += __shfl_down(cs[f], off, 64);
+        vm = fmax(vm, __shfl_down(vm, off, 64));
+    }
+    if (lane == 0) finish_instance(J, counts ? ll : len, q0, q1, qc, cs, vm, step, upd, sc, rotate);
+}
+
 // LDS of the finalize body.
 struct FinLds {
     uint8_t s_pb[2][kSegTiles];     // per tile: parity the next step sees
@@ -151,7 +194,8 @@ template <int NT>
 __device__ __forceinline__ void finalize_body(const Inst* __restrict__ insts, const Seg* __restrict__ segs,
                                               int segi, int nseg, SegPart* __restrict__ parts,
                                               int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
-                                              int rotate, int one_inst, FinLds& F) {
+                                              int rotate, int one_inst, const SegPart* __restrict__ pend,
+                                              FinLds& F) {
     static_assert(NT == kSegTiles, "one thread per tile of a segment");
     auto& s_pb = F.s_pb;
     auto& s_ab = F.s_ab;
@@ -320,6 +364,9 @@ __device__ __forceinline__ void finalize_body(const Inst* __restrict__ insts, co
         }
         return;
     }
+    // folded merges: the instance sums of the step before this one, by the last wave
+    // of the instance's first segment
+    if (pend && wid == NT / 64 - 1 && t0 == 0) merge_instance(I, segi, (nt + kSegTiles - 1) / kSegTiles, pend, nullptr, 1);
     if (tid == 0) {
         counts[segi] = listlen;
         if (rotate) {
@@ -362,39 +409,7 @@ __device__ __forceinline__ void finalize_merge_body(const Inst* __restrict__ ins
         if (i >= i_hi) break;
         CInst& J = ((CInst*)insts)[i];
         const InstSegs r = n_inst == 1 ? InstSegs{0, nseg} : isegs[i];
-        // the instance's scalars and counters, loaded ahead of the reduction
-        double sc[16];
-        int64_t step = 0, upd = 0;
-        if (lane == 0) {
-            for (int kk = 0; kk < 16; kk++) sc[kk] = J.scal[kk];
-            step = J.ctr[0];
-            upd = J.ctr[1];
-        }
-        int64_t ll = 0;
-        unsigned long long q0 = 0, q1 = 0, qc = 0;
-        double cs[kMaxFields] = {0.0, 0.0, 0.0, 0.0};
-        double vm = 0.0;
-        const int ncs = J.ncons;
-        for (int q = r.first + lane; q < r.first + r.count; q += 64) {
-            ll += counts[q];
-            if (rotate) {
-                q0 += parts[q].c0;
-                q1 += parts[q].c1;
-                qc += parts[q].cells;
-                for (int f = 0; f < ncs; f++) cs[f] += parts[q].csum[f];
-                vm = fmax(vm, parts[q].vmax);
-            }
-        }
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-            ll += __shfl_down(ll, off, 64);
-            q0 += __shfl_down(q0, off, 64);
-            q1 += __shfl_down(q1, off, 64);
-            qc += __shfl_down(qc, off, 64);
-            for (int f = 0; f < kMaxFields; f++) cs[f] += __shfl_down(cs[f], off, 64);
-            vm = fmax(vm, __shfl_down(vm, off, 64));
-        }
-        if (lane == 0) finish_instance(J, ll, q0, q1, qc, cs, vm, step, upd, sc, rotate);
+        merge_instance(J, r.first, r.count, parts, counts, rotate);
     }
     if (!one && blockIdx.x != 0) return;
     int running = 0;
@@ -415,9 +430,9 @@ __global__ __launch_bounds__(kFinNT) void finalize_kernel(const Inst* __restrict
                                                           SegPart* __restrict__ parts,
                                                           int32_t* __restrict__ counts,
                                                           int32_t* __restrict__ offsets, int rotate,
-                                                          int one_inst) {
+                                                          int one_inst, const SegPart* __restrict__ pend) {
     __shared__ FinLds F;
-    finalize_body<kFinNT>(insts, segs, blockIdx.x, nseg, parts, counts, offsets, rotate, one_inst, F);
+    finalize_body<kFinNT>(insts, segs, blockIdx.x, nseg, parts, counts, offsets, rotate, one_inst, pend, F);
 }
 
 __global__ __launch_bounds__(kFinNT) void finalize_merge_kernel(const Inst* __restrict__ insts, int nseg,

@@ -231,13 +231,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k9
     __shared__ NbTable nb;
 
     WorkCursor cur;
+    Fold FO;
     work_begin(wl, cur, true);
-    const int total = wl.offsets[wl.nseg];
+    const int total = work_open(wl, FO);
     for (;;) {
         CInst* Ip;
         int t;
         uint64_t rec;
-        if (!work_next(wl, cur, total, &Ip, &t, &rec)) break;
+        if (!work_next(wl, FO, cur, total, &Ip, &t, &rec)) break;
         if (k93_partial<TB, PART>(*Ip, t)) k93_tile<TB, NT, true, true>(*Ip, t, rec, nb, L, sflag);
         else k93_tile<TB, NT, true>(*Ip, t, rec, nb, L, sflag);
     }

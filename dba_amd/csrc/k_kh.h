@@ -604,8 +604,10 @@ template <int TB, bool P2>
 __global__ __launch_bounds__(TB* TB) __attribute__((amdgpu_waves_per_eu(4))) void kh_step_kernel(const WorkList wl) {
     __shared__ KhLds<TB> S;
     WorkCursor cur;
+    Fold FO;
     work_begin(wl, cur, true);
-    const int total = wl.offsets[wl.nseg];
+    constexpr bool FOLD = TB == 8;
+    const int total = work_open<FOLD>(wl, FO);
     // opaque to the compiler, so that what follows from the thread index alone is
     // worked out per tile instead of being kept in registers across the tiles
     auto thread = [] {
@@ -616,7 +618,7 @@ __global__ __launch_bounds__(TB* TB) __attribute__((amdgpu_waves_per_eu(4))) voi
     for (;;) {
         KhItem it;
         uint64_t rec;
-        if (!work_next(wl, cur, total, &it.I, &it.t, &rec)) break;
+        if (!work_next<FOLD>(wl, FO, cur, total, &it.I, &it.t, &rec)) break;
         CInst& I = *it.I;
         const int ntx = I.ntx, lane = threadIdx.x & 63;
         it.tj = it.t / ntx;

@@ -387,12 +387,14 @@ __global__ __launch_bounds__(64) void modelb_mu_kernel(const WorkList wl, int fr
         if (lane < C) ph = I.buf[(int)(q.pm >> 13) & 1][3][mb_own_index<TB, TZ>(q, lane)];
     };
 
-    const int total = wl.offsets[wl.nseg];
+    __shared__ FoldLds FL;
+    Fold FO;
+    const int total = work_open(wl, FO, &FL);
     // a list of at least `from` blocks is the march's step
     if (total >= from) return;
     const BandSweep bs = band_sweep_setup(wl, total);
     for (int round0 = 0; (int64_t)round0 * gridDim.x < total; round0 += 64) {
-        const RoundList L = bs.cx ? band_sweep_round(bs, round0) : round_list(wl, total, round0);
+        const RoundList L = bs.cx ? band_sweep_round(bs, round0) : round_list(wl, FO, total, round0);
         uint64_t todo = L.valid;
         if (!todo) continue;
         MbBlock b = mb_take<TB, TZ>(wl, L, todo);
@@ -523,12 +525,14 @@ __global__ __launch_bounds__(64) void modelb_update_kernel(const WorkList wl, in
         for (int f = 0; f < I.ncons; f++) eq[f] = I.s_tile[((int64_t)f * 2 + pq) * I.nt + q.t];
     };
 
-    const int total = wl.offsets[wl.nseg];
+    __shared__ FoldLds FL;
+    Fold FO;
+    const int total = work_open(wl, FO, &FL);
     // a list of at least `from` blocks is the march's step
     if (total >= from) return;
     const BandSweep bs = band_sweep_setup(wl, total);
     for (int round0 = 0; (int64_t)round0 * gridDim.x < total; round0 += 64) {
-        const RoundList L = bs.cx ? band_sweep_round(bs, round0) : round_list(wl, total, round0);
+        const RoundList L = bs.cx ? band_sweep_round(bs, round0) : round_list(wl, FO, total, round0);
         uint64_t todo = L.valid;
         if (!todo) continue;
         MbBlock b = mb_take<TB, TZ>(wl, L, todo);
@@ -659,7 +663,9 @@ __global__ __launch_bounds__(MbMarch::NT) __attribute__((amdgpu_waves_per_eu(CON
     const WorkList wl, int from, int nl, int ncx, int ncy) {
     using M = MbMarch;
     __shared__ MbMarchLds<CONS> S;
-    const int total = wl.offsets[wl.nseg];
+    __shared__ FoldLds FL;
+    Fold FO;
+    const int total = work_open(wl, FO, &FL);
     if (total < from) return;
     CInst& I = *(CInst*)wl.insts;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -943,13 +949,15 @@ __global__ __launch_bounds__(64) void k94_step_kernel(const WorkList wl) {
 
     WorkCursor cur;
     work_begin(wl, cur, false);
-    const int total = wl.offsets[wl.nseg];
+    __shared__ FoldLds FL;
+    Fold FO;
+    const int total = work_open(wl, FO, &FL);
     const int tid = threadIdx.x;
     for (;;) {
         CInst* Ip;
         int t;
         uint64_t rec;
-        if (!work_next(wl, cur, total, &Ip, &t, &rec, false)) break;
+        if (!work_next(wl, FO, cur, total, &Ip, &t, &rec, false)) break;
         CInst& I = *Ip;
         const int nx = I.nx, ny = I.ny, nz = I.nz;
         const int x0 = (t % I.ntx) * TB, y0 = ((t / I.ntx) % I.nty) * TB, z0 = (t / (I.ntx * I.nty)) * TZ;

@@ -16,6 +16,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -23,6 +24,7 @@
 #include "common.h"
 #include "k_finalize.h"
 #include "k_ch.h"
+#include "k_resident.h"
 #include "k_k93.h"
 #include "k_kh.h"
 #include "k_ref3d.h"
@@ -109,6 +111,7 @@ struct Group {
     int march_from = 0;           // Model B: lists of at least this many blocks take the column march (0: never)
     int mb_nl = 1, mb_ncx = 0, mb_ncy = 0, mb_ntz = 0;  // ... layers per strip, columns in x and y, layers
     bool nine = true;             // CH 9-point stencil (the march kernel is instanced on it)
+    int res_gx = 0, res_gy = 0, res_threads = 0, res_per_tile = 0;  // resident steps (k_resident.h): region, workgroup, threads per tile (0: not taken)
     Inst* d_insts = nullptr;
     Seg* d_segs = nullptr;
     InstSegs* d_isegs = nullptr;
@@ -166,6 +169,12 @@ struct dba_ctx {
     std::vector<hipEvent_t> ev_pool;
     hipEvent_t markers[8] = {};
     unsigned char* scratch = nullptr;  // this device's address of the scratch array
+    // exchange of the resident steps: one workspace for every instance (its launches
+    // follow each other on the one stream; sequence numbers never repeat)
+    uint64_t* xbuf = nullptr;
+    size_t xwords = 0;
+    uint32_t xseq = 1;
+    int* stuck = nullptr;          // pinned host word: a resident step's wait ran out
 };
 
 namespace {
@@ -431,6 +440,8 @@ dba_status kh_prime(dba_ctx* ctx, Instance* in) {
     return DBA_OK;
 }
 
+void resident_choose(const dba_ctx* ctx, Group* g, const Inst& h);  // below, with the launches
+
 dba_status get_group(dba_ctx* ctx, const std::vector<int>& ids, Group** out) {
     auto it = ctx->groups.find(ids);
     if (it != ctx->groups.end()) {
@@ -486,6 +497,9 @@ dba_status get_group(dba_ctx* ctx, const std::vector<int>& ids, Group** out) {
                 break;
             }
     }
+    // Resident steps: one CH instance (regular or DBA) whose tiles fit the chip at once
+    if (ids.size() == 1 && g->model == DBA_MODEL_CH && first->p.mode != DBA_MODE_CONSERVED && first->p.threads == 0)
+        resident_choose(ctx, g, first->h);
     // Speculative staging in single-launch K93 steps (k93_dense_kernel SPEC):
     // one instance of up to 1024 full 16 x 16 tiles at 512 threads (measured on
     // 512^2: 7.2 -> 6.7 us per step with the run-counter prefetch); larger grids
@@ -829,6 +843,158 @@ dba_status partition(dba_ctx* ctx, const int32_t* ids, int32_t n_ids, std::vecto
     return DBA_OK;
 }
 
+// The state-restoring launches after n_steps single-launch or resident steps.
+dba_status launch_canon(dba_ctx* ctx, const Group* g, int n_steps) {
+    if (!g->d_dmap) {
+        hipLaunchKernelGGL(dense_canon_kernel, dim3(1), dim3(kFinNT), 0, ctx->stream, g->d_insts, n_steps);
+    } else {
+        hipLaunchKernelGGL(dense_canon_seg_kernel, dim3((unsigned)g->nseg), dim3(kFinNT), 0, ctx->stream, g->d_insts,
+                           g->d_segs, g->d_parts, g->d_counts, n_steps);
+        LAUNCH_CHECK();
+        hipLaunchKernelGGL(dense_canon_merge_kernel, dim3(1), dim3(kFinNT), 0, ctx->stream, g->d_insts, g->d_isegs,
+                           (int)g->ids.size(), g->d_parts, g->d_counts, n_steps);
+    }
+    LAUNCH_CHECK();
+    return DBA_OK;
+}
+
+// ---- resident steps (k_resident.h)
+
+// The cooperative launch costs about 15 us more than the launches it replaces have
+// around them (256^2: 41 us + 2.7 us per step against 28 + 4.4; 1024^2: 54 + 4.4
+// against 36 + 7.0), so calls of fewer steps keep single-launch steps.
+constexpr int kResidentMinSteps = 12;
+
+template <int TB, int NT>
+const void* ch_resident_fn(bool nine) {
+    return nine ? (const void*)ch_resident_kernel<TB, NT, true> : (const void*)ch_resident_kernel<TB, NT, false>;
+}
+
+// The kernel of a group's tile with `per_tile` threads on each tile.
+const void* resident_kernel(const Group* g, int per_tile) {
+    switch (g->tile) {
+        case 8: return ch_resident_fn<8, 64>(g->nine);
+        case 16: return ch_resident_fn<16, 128>(g->nine);
+        default: return per_tile == 1024 ? ch_resident_fn<32, 1024>(g->nine) : ch_resident_fn<32, 256>(g->nine);
+    }
+}
+
+// Whether `wgs` workgroups of the kernel are certainly resident at once. The
+// occupancy the runtime computes does not count the scalar registers the trap
+// handler takes from every wave (measured: 28 one-wave workgroups per CU promised,
+// 24 resident), so at most 24 waves per CU; and a sixteenth is kept free where
+// several share a CU (27 promised by their LDS, 26.7 resident).
+bool all_resident(const dba_ctx* ctx, const void* f, int threads, size_t lds, int64_t wgs) {
+    constexpr size_t kLdsPerCu = 160 * 1024;
+    if (lds + 2048 > kLdsPerCu) return false;
+    if (lds > 64 * 1024 && hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    int blocks = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, f, threads, lds) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    blocks = std::min(blocks, 24 / (threads / 64));
+    const int64_t all = (int64_t)blocks * ctx->n_cu;
+    return wgs <= (blocks > 1 ? all - all / 16 : all);
+}
+
+// Region and workgroup of a CH group's resident steps, if the grid fits the chip.
+void resident_choose(const dba_ctx* ctx, Group* g, const Inst& h) {
+    int coop = 0;
+    if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device) != hipSuccess || !coop) return;
+    struct Shape {
+        int gx, gy, threads, per_tile;
+    };
+    // smallest regions first: per step a region waits for one exchange whatever its
+    // size, so a grid that leaves room takes more threads per cell, and a larger one
+    // larger regions (fewer frames). us per step over 1000 steps, single-launch
+    // steps -> this: 32 x 32 tiles 256^2 4.4 -> 2.7 (512 or 1024 threads per tile; 256: 3.5),
+    // 1024^2 7.1 -> 4.4 (one tile per workgroup: 7.0, two: 7.1), 1200 x 1100
+    // 15.2 -> 6.5; 16 x 16 tiles 512^2 4.5 -> 2.8, 1024^2 8.4 -> 5.1; 8 x 8 tiles
+    // 512^2 5.7 -> 3.2
+    std::vector<Shape> shapes = {{1, 1, 1024, 1024}, {2, 2, 1024, 256}, {3, 2, 768, 256}};
+    if (g->tile == 16) shapes = {{2, 2, 512, 128}, {4, 4, 1024, 128}};
+    if (g->tile == 8) shapes = {{4, 2, 512, 64}, {4, 4, 1024, 64}};
+    for (const Shape& s : shapes) {
+        const void* f = resident_kernel(g, s.per_tile);
+        const size_t lds = ch_resident_bytes(g->tile * s.gx, g->tile * s.gy);
+        const int64_t wgs = (int64_t)((h.ntx + s.gx - 1) / s.gx) * ((h.nty + s.gy - 1) / s.gy);
+        if (!all_resident(ctx, f, s.threads, lds, wgs)) continue;
+        g->res_gx = s.gx;
+        g->res_gy = s.gy;
+        g->res_threads = s.threads;
+        g->res_per_tile = s.per_tile;
+        return;
+    }
+}
+
+// The exchange buffer of `words`, cleared when the sequence numbers start over.
+bool resident_buffer(dba_ctx* ctx, size_t words, int n_steps) {
+    if (!ctx->stuck) {
+        if (hipHostMalloc((void**)&ctx->stuck, sizeof(int)) != hipSuccess) return false;
+        *ctx->stuck = 0;
+    }
+    const bool wrap = ctx->xseq > 0xffffffffu - (uint32_t)n_steps - 2u;
+    if (words <= ctx->xwords && !wrap) return true;
+    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
+    if (words > ctx->xwords) {
+        if (ctx->xbuf) (void)hipFree(ctx->xbuf);
+        ctx->xbuf = nullptr;
+        ctx->xwords = 0;
+        if (hipMalloc(&ctx->xbuf, words * sizeof(uint64_t)) != hipSuccess) return false;
+        ctx->xwords = words;
+    }
+    ctx->xseq = 1;
+    return hipMemsetAsync(ctx->xbuf, 0, ctx->xwords * sizeof(uint64_t), ctx->stream) == hipSuccess;
+}
+
+// The process's contexts on a device, after adding `d`. A context alone on its device
+// takes resident launches. Where there are others it does not: two such launches, each
+// half resident, would wait for ever, and single-launch steps of two contexts overlap,
+// so they finish sooner than resident ones after each other (two contexts of 1024^2,
+// 2000 steps: 18.5 ms against 22).
+int live_contexts(int device, int d) {
+    static std::mutex m;
+    static std::map<int, int>* live = new std::map<int, int>();  // kept until the process ends
+    std::lock_guard<std::mutex> lock(m);
+    return (*live)[device] += d;
+}
+
+// n_steps of one group as a resident launch and its canonicalising kernels; *taken is
+// false where the launch could not be had (the other paths need less) or must not be.
+dba_status enqueue_resident(dba_ctx* ctx, Group* g, int n_steps, bool* taken) {
+    *taken = false;
+    if (!g->res_gx || ctx->single_launch == 0 || ctx->timing || n_steps < kResidentMinSteps) return DBA_OK;
+    if (live_contexts(ctx->device, 0) > 1) return DBA_OK;
+    const Inst& h = ctx->inst.at(g->ids[0])->h;
+    const int nt = h.nt, gx = g->res_gx, gy = g->res_gy;
+    const unsigned wgs = (unsigned)(((h.ntx + gx - 1) / gx) * ((h.nty + gy - 1) / gy));
+    const int slots = frame_slots(gx * g->tile, gy * g->tile);
+    const size_t words = 2 * (size_t)wgs * (size_t)slots * 2 + 2 * (size_t)nt;
+    bool ok = resident_buffer(ctx, words, n_steps);
+    if (ok) {
+        const void* f = resident_kernel(g, g->res_per_tile);
+        const size_t lds = ch_resident_bytes(gx * g->tile, gy * g->tile);
+        Exchange X{ctx->xbuf, ctx->xbuf + (words - 2 * (size_t)nt), ctx->stuck, ctx->xseq, slots};
+        const Inst* insts = g->d_insts;
+        int n = n_steps, ax = gx, ay = gy;
+        void* args[] = {(void*)&insts, (void*)&X, (void*)&n, (void*)&ax, (void*)&ay};
+        ok = hipLaunchCooperativeKernel(f, dim3(wgs), dim3((unsigned)g->res_threads), args, (unsigned)lds,
+                                        ctx->stream) == hipSuccess;
+    }
+    if (!ok) {  // too little memory, or no such launch here: the other paths from now on
+        (void)hipGetLastError();
+        g->res_gx = 0;
+        return DBA_OK;
+    }
+    ctx->xseq += (uint32_t)n_steps + 1u;
+    *taken = true;
+    return launch_canon(ctx, g, n_steps);
+}
+
 dba_status enqueue_steps(dba_ctx* ctx, const std::vector<Group*>& gs, int n_steps, bool timed) {
     // single-launch groups: n steps, then one canonicalisation
     for (Group* g : gs) {
@@ -842,14 +1008,9 @@ dba_status enqueue_steps(dba_ctx* ctx, const std::vector<Group*>& gs, int n_step
             }
             if (s < n_steps) {
                 launch_dense(g, ctx->stream, s == 0, s);
-            } else if (!g->d_dmap) {
-                hipLaunchKernelGGL(dense_canon_kernel, dim3(1), dim3(kFinNT), 0, ctx->stream, g->d_insts, n_steps);
             } else {
-                hipLaunchKernelGGL(dense_canon_seg_kernel, dim3((unsigned)g->nseg), dim3(kFinNT), 0, ctx->stream,
-                                   g->d_insts, g->d_segs, g->d_parts, g->d_counts, n_steps);
-                LAUNCH_CHECK();
-                hipLaunchKernelGGL(dense_canon_merge_kernel, dim3(1), dim3(kFinNT), 0, ctx->stream, g->d_insts,
-                                   g->d_isegs, (int)g->ids.size(), g->d_parts, g->d_counts, n_steps);
+                const dba_status st = launch_canon(ctx, g, n_steps);
+                if (st != DBA_OK) return st;
             }
             LAUNCH_CHECK();
             if (timed) {
@@ -928,6 +1089,22 @@ dba_status ensure_staging(dba_ctx* ctx, size_t n) {
 
 }  // namespace
 
+// Waits for the compute stream; an error if a resident step's wait ran out.
+namespace {
+dba_status wait_stream(dba_ctx* ctx) {
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    if (ctx->stuck && *(volatile int*)ctx->stuck)
+        return fail(DBA_ERR_HIP, "a resident step waited too long for another workgroup: the fields are not valid");
+    return DBA_OK;
+}
+}  // namespace
+
+#define WAIT_STREAM(ctx)                              \
+    do {                                              \
+        const dba_status w_ = wait_stream(ctx);       \
+        if (w_ != DBA_OK) return w_;                  \
+    } while (0)
+
 // ===================================================================== C ABI
 
 namespace {
@@ -987,6 +1164,7 @@ dba_status dba_init(int32_t device, dba_ctx** out) {
     HIP_TRY(hipMalloc(&ctx->d_diag, sizeof(double) * (3 * kDiagBlocks + kMaxFrontCols + 8)));
     HIP_TRY(hipMalloc(&ctx->d_cols, sizeof(int32_t) * kMaxFrontCols));
     for (auto& m : ctx->markers) HIP_TRY(hipEventCreate(&m));
+    live_contexts(device, 1);
     *out = ctx;
     return DBA_OK;
 }
@@ -995,6 +1173,7 @@ dba_status dba_finalize(dba_ctx* ctx) {
     if (!ctx) return DBA_OK;
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
+    live_contexts(ctx->device, -1);
     std::vector<int> ids;
     for (auto& kv : ctx->inst) ids.push_back(kv.first);
     for (int id : ids) dba_instance_destroy(ctx, id);
@@ -1003,6 +1182,8 @@ dba_status dba_finalize(dba_ctx* ctx) {
     for (auto e : ctx->ev_pool) (void)hipEventDestroy(e);
     for (auto m : ctx->markers) (void)hipEventDestroy(m);
     if (ctx->staging) (void)hipFree(ctx->staging);
+    if (ctx->xbuf) (void)hipFree(ctx->xbuf);
+    if (ctx->stuck) (void)hipHostFree(ctx->stuck);
     if (ctx->d_flag) (void)hipFree(ctx->d_flag);
     if (ctx->d_diag) (void)hipFree(ctx->d_diag);
     if (ctx->d_cols) (void)hipFree(ctx->d_cols);
@@ -1142,7 +1323,7 @@ dba_status dba_instance_info(dba_ctx* ctx, int32_t id, dba_info* out) {
     if (!ctx || !out) return fail(DBA_ERR_INVALID, "null argument");
     Instance* in = find(ctx, id);
     if (!in) return fail(DBA_ERR_NOTFOUND, "unknown instance %d", id);
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    WAIT_STREAM(ctx);
     double scal[16];
     int64_t ctr[4];
     HIP_TRY(hipMemcpy(scal, in->h.scal, sizeof(scal), hipMemcpyDeviceToHost));
@@ -1197,7 +1378,7 @@ dba_status dba_download(dba_ctx* ctx, int32_t id, int32_t field, double* host, s
                        ctx->staging);
     LAUNCH_CHECK();
     HIP_TRY(hipMemcpyAsync(host, ctx->staging, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    WAIT_STREAM(ctx);
     return DBA_OK;
 }
 
@@ -1207,6 +1388,9 @@ dba_status dba_step(dba_ctx* ctx, const int32_t* ids, int32_t n_ids, int32_t n_s
     std::vector<Group*> gs;
     dba_status st = prepare_groups(ctx, ids, n_ids, &gs);
     if (st != DBA_OK) return st;
+    bool taken = false;
+    if (gs.size() == 1) st = enqueue_resident(ctx, gs[0], n_steps, &taken);
+    if (st != DBA_OK || taken) return st;
     return enqueue_steps(ctx, gs, n_steps, ctx->timing);
 }
 
@@ -1216,6 +1400,9 @@ dba_status dba_step_graph(dba_ctx* ctx, const int32_t* ids, int32_t n_ids, int32
     std::vector<Group*> gs;
     dba_status st = prepare_groups(ctx, ids, n_ids, &gs);
     if (st != DBA_OK) return st;
+    bool taken = false;
+    if (gs.size() == 1) st = enqueue_resident(ctx, gs[0], n_steps, &taken);
+    if (st != DBA_OK || taken) return st;
     int reps = n_steps / chunk, rem = n_steps % chunk;
     if (reps > 0) {
         GraphKey key{std::vector<int>(ids, ids + n_ids), chunk, ctx->single_launch};
@@ -1252,7 +1439,7 @@ dba_status dba_set_single_launch(dba_ctx* ctx, int32_t mode) {
 
 dba_status dba_sync(dba_ctx* ctx) {
     if (!ctx) return fail(DBA_ERR_INVALID, "null ctx");
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    WAIT_STREAM(ctx);
     return DBA_OK;
 }
 
@@ -1261,7 +1448,7 @@ dba_status dba_active_tiles(dba_ctx* ctx, int32_t id, int32_t set, int32_t* coun
     Instance* in = find(ctx, id);
     if (!in) return fail(DBA_ERR_NOTFOUND, "unknown instance %d", id);
     if (set < 0 || set >= in->h.nsets) return fail(DBA_ERR_INVALID, "set %d invalid", set);
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    WAIT_STREAM(ctx);
     int nt = in->h.nt;
     std::vector<uint64_t> w((size_t)in->h.nwords);
     HIP_TRY(hipMemcpy(w.data(), in->h.a_cur[set], sizeof(uint64_t) * w.size(), hipMemcpyDeviceToHost));
@@ -1283,7 +1470,7 @@ dba_status dba_worklist(dba_ctx* ctx, int32_t id, int32_t* tiles, int32_t cap, i
     std::vector<Group*> gs;
     dba_status st = prepare_groups(ctx, &id, 1, &gs);
     if (st != DBA_OK) return st;
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    WAIT_STREAM(ctx);
     int64_t ctr[4];
     HIP_TRY(hipMemcpy(ctr, in->h.ctr, sizeof(ctr), hipMemcpyDeviceToHost));
     *count = (int32_t)ctr[2];
@@ -1298,7 +1485,7 @@ dba_status dba_active_history(dba_ctx* ctx, int32_t id, int32_t* counts, int32_t
     if (!ctx || !n_steps) return fail(DBA_ERR_INVALID, "null argument");
     Instance* in = find(ctx, id);
     if (!in) return fail(DBA_ERR_NOTFOUND, "unknown instance %d", id);
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    WAIT_STREAM(ctx);
     int64_t ctr[4];
     HIP_TRY(hipMemcpy(ctr, in->h.ctr, sizeof(ctr), hipMemcpyDeviceToHost));
     int n = (int)std::min<int64_t>(std::min<int64_t>(ctr[0], in->h.hist_cap), max_steps);
@@ -1309,7 +1496,7 @@ dba_status dba_active_history(dba_ctx* ctx, int32_t id, int32_t* counts, int32_t
 
 dba_status dba_timing_enable(dba_ctx* ctx, int32_t enable) {
     if (!ctx) return fail(DBA_ERR_INVALID, "null ctx");
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    WAIT_STREAM(ctx);
     ctx->ev_pool.insert(ctx->ev_pool.end(), ctx->ev_used.begin(), ctx->ev_used.end());
     ctx->ev_used.clear();
     ctx->ev_step.clear();
@@ -1320,7 +1507,7 @@ dba_status dba_timing_enable(dba_ctx* ctx, int32_t enable) {
 
 dba_status dba_timing_query(dba_ctx* ctx, double* step_ms, int64_t* step_n, double* fin_ms, int64_t* fin_n) {
     if (!ctx) return fail(DBA_ERR_INVALID, "null ctx");
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    WAIT_STREAM(ctx);
     double a = 0.0, b = 0.0;
     for (auto& e : ctx->ev_step) {
         float ms = 0.f;
@@ -1364,7 +1551,7 @@ dba_status dba_check_finite(dba_ctx* ctx, int32_t id) {
     LAUNCH_CHECK();
     int bad = 0;
     HIP_TRY(hipMemcpyAsync(&bad, ctx->d_flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    WAIT_STREAM(ctx);
     if (bad) return fail(DBA_ERR_NUMERIC, "instance %d holds non-finite values", id);
     return DBA_OK;
 }
@@ -1382,7 +1569,7 @@ dba_status dba_field_sum(dba_ctx* ctx, int32_t id, int32_t field, double* sum) {
     hipLaunchKernelGGL(reduce_parts_kernel, dim3(1), dim3(64), 0, ctx->stream, part, 1, res);
     LAUNCH_CHECK();
     HIP_TRY(hipMemcpyAsync(sum, res, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    WAIT_STREAM(ctx);
     return DBA_OK;
 }
 
@@ -1403,7 +1590,7 @@ dba_status dba_growth_front(dba_ctx* ctx, int32_t id, const int32_t* xs, int32_t
                        ctx->d_cols, n, res);
     LAUNCH_CHECK();
     HIP_TRY(hipMemcpyAsync(front, res, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    WAIT_STREAM(ctx);
     return DBA_OK;
 }
 
@@ -1439,7 +1626,7 @@ dba_status dba_droplets(dba_ctx* ctx, int32_t id, int32_t field, double* avg, in
     int64_t cnt[2];
     HIP_TRY(hipMemcpyAsync(cnt, counters, sizeof(cnt), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipMemcpyAsync(avg, d_avg, sizeof(double), hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    WAIT_STREAM(ctx);
     *n_droplets = cnt[0];
     *volume = cnt[1];
     if (cap == 0 || cnt[0] == 0) return DBA_OK;
@@ -1504,7 +1691,7 @@ dba_status dba_droplets_noalloc(dba_ctx* ctx, int32_t id, int32_t field, double*
     int64_t cnt[2];
     HIP_TRY(hipMemcpyAsync(cnt, counters, sizeof(cnt), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipMemcpyAsync(avg, d_avg, sizeof(double), hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    WAIT_STREAM(ctx);
     *n_droplets = cnt[0];
     *volume = cnt[1];
     if (cap == 0 || cnt[0] == 0) return DBA_OK;
@@ -1536,7 +1723,7 @@ dba_status dba_kh_vy_mode(dba_ctx* ctx, int32_t id, double* amplitude) {
     LAUNCH_CHECK();
     double s[3];
     HIP_TRY(hipMemcpyAsync(s, res, sizeof(s), hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    WAIT_STREAM(ctx);
     *amplitude = 2.0 * std::sqrt(s[0] * s[0] / (s[2] * s[2]) + s[1] * s[1] / (s[2] * s[2]));
     return DBA_OK;
 }

@@ -1,0 +1,449 @@
+// k_resident.h - many DBA steps of one instance in one cooperative launch, the
+// fields in LDS from the first step to the last.
+//
+// A step of a grid that fits the chip is bound by latency, not by bytes or
+// arithmetic: with one launch per step a 1024^2 Cahn-Hilliard step takes 7 us, of
+// which a copy of the grid would take 3 and the arithmetic 2; the rest is the gap
+// between launches, the tables every workgroup builds first and the trip of every
+// cell through the caches. Here each workgroup owns a region of gx x gy tiles for
+// the whole call, keeps its cells in LDS, and per step exchanges only the two-cell
+// frame its neighbours read.
+//
+// Exchange: every published value travels as two 8-byte words, each holding half
+// of the double and the step's sequence number, written and read with relaxed
+// atomics of agent scope (they bypass the per-XCD caches). A word is valid when its
+// number is the expected one, so there is no flag to wait for after the data and
+// no fence. Two generations (step parity) suffice: a tile publishes generation
+// s + 2 only after step s + 1, for which it has received every neighbour's word of
+// step s, and those were sent after the neighbour had read generation s.
+//
+// Progress: the launch is cooperative, so all workgroups are resident; a workgroup
+// waits only for words of the step before, which their owners send without waiting
+// for anything of this step, so by induction over the steps every wait ends. Each
+// wait is bounded all the same: past the bound, or once any other wait has passed
+// it, a workgroup says so in *stuck and ends its steps, and the host returns an error.
+#pragma once
+#include "common.h"
+#include "k_ch.h"
+#include "k_finalize.h"
+
+namespace dba {
+
+struct Exchange {
+    uint64_t* frame;   // [parity][region][slot][2]
+    uint64_t* flag;    // [parity][tile]: sequence number << 32 | detector bit
+    int* stuck;        // host memory: a wait ran out
+    uint32_t base;     // sequence number of the launch's first step
+    int slots;         // frame slots of a whole region
+};
+
+__device__ __forceinline__ void xput(uint64_t* p, uint64_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t xget(const uint64_t* p) {
+    return __hip_atomic_load((uint64_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ void put_double(uint64_t* p, double v, uint32_t seq) {
+    const uint64_t b = (uint64_t)__double_as_longlong(v), s = (uint64_t)seq << 32;
+    xput(p, s | (uint32_t)b);
+    xput(p + 1, s | (uint32_t)(b >> 32));
+}
+
+// Bound of a wait: about a second of polls (each is a trip to memory).
+constexpr int kWaitPolls = 1 << 20;
+
+// Called while polling: true when the wait must be given up.
+__device__ __forceinline__ bool wait_over(int polls, int* stuck) {
+    if ((polls & 1023) != 1023) return false;
+    if (polls >= kWaitPolls) __hip_atomic_store(stuck, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return __hip_atomic_load(stuck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0;
+}
+
+__device__ __forceinline__ double wait_double(const uint64_t* p, uint32_t seq, int* stuck, int* gone) {
+    uint64_t a, b;
+    for (int k = 0;; k++) {
+        a = xget(p);
+        b = xget(p + 1);
+        if ((uint32_t)(a >> 32) == seq && (uint32_t)(b >> 32) == seq) break;
+        if (wait_over(k, stuck)) {
+            *gone = 1;
+            break;
+        }
+    }
+    return __longlong_as_double((long long)((uint64_t)(uint32_t)b << 32 | (uint32_t)a));
+}
+
+__device__ __forceinline__ int wait_flag(const uint64_t* p, uint32_t seq, int* stuck, int* gone) {
+    uint64_t a;
+    for (int k = 0;; k++) {
+        a = xget(p);
+        if ((uint32_t)(a >> 32) == seq) break;
+        if (wait_over(k, stuck)) {
+            *gone = 1;
+            break;
+        }
+    }
+    return (int)(a & 1ull);
+}
+
+// The published cells of a w x h region: two cells deep on each side, every cell
+// one slot (rows first, so the cells of a region two or three cells thick have one).
+__host__ __device__ __forceinline__ int frame_slots(int w, int h) { return 4 * w + 4 * h; }  // at most
+
+__device__ __forceinline__ int frame_slot(int lx, int ly, int w, int h) {
+    if (ly < 2) return ly * w + lx;
+    if (ly >= h - 2) return 2 * w + (ly - (h - 2)) * w + lx;
+    if (lx < 2) return 4 * w + (ly - 2) * 2 + lx;
+    if (lx >= w - 2) return 4 * w + 2 * (h - 4) + (ly - 2) * 2 + (lx - (w - 2));
+    return -1;
+}
+
+// cell k of the ring of thickness T around a w x h region (coordinates from -T):
+// the rows below, the rows above, then the columns
+template <int T>
+__device__ __forceinline__ void outer_cell(int k, int w, int h, int* x, int* y) {
+    const int W = w + 2 * T;
+    if (k < 2 * T * W) {
+        const int r = k / W;
+        *y = r < T ? r - T : h + r - T;
+        *x = k - r * W - T;
+    } else {
+        const int q = k - 2 * T * W, c = q % (2 * T);
+        *y = q / (2 * T);
+        *x = c < T ? c - T : w + c - T;
+    }
+}
+
+constexpr int kResMaxTiles = 16;  // tiles of a region, at most (with their surroundings two deep: 64, one ballot)
+
+struct ResTile {
+    int t, x, y, w, h, par, runs, last;  // tile, window position, extent, buffer, steps run, bit of the last of them
+    int pos;                             // position among the awake bits
+};
+
+// LDS bytes of a region of w x h cells.
+constexpr size_t ch_resident_bytes(int w, int h) {
+    return sizeof(double) * ((size_t)(w + 4) * (h + 4) + (size_t)(w + 2) * (h + 2)) +
+           sizeof(int) * (2 * (size_t)(4 * (w + h) + 16) + (size_t)(4 * (w + h)));
+}
+
+// n steps of one CH instance (regular or DBA). The region's c (with a two-cell
+// halo) and mu (with a one-cell ring) stay in LDS windows for the whole launch; per
+// tile and step the arithmetic, its order and the detector are ch_tile's, so results
+// are bit-identical to the other paths. A sleeping tile's mu is what the window
+// still holds from the last step it ran, and a sleeping outside tile's ring is what
+// this region computed for it then (the same doubles from the same cells); only at
+// the end of the launch do tiles that did not fire when they last ran store their
+// ring. The canonicalising kernels follow, as after single-launch steps.
+//
+// A step: 1. mu of the tiles that fired in the step before (they run whatever their
+// neighbours did), all but the region's edge, while the frames of the other regions
+// are on their way; 2. the halo and the outside detector bits; 3. mu of tiles only a
+// neighbour woke, of the edge and of the ring; 4. c' and the frame.
+// NT threads work on a tile: R = TB TB / NT rows of one column each.
+template <int TB, int NT, bool NINE>
+__global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restrict__ insts, Exchange X, int n, int gx,
+                                                           int gy) {
+    constexpr int R = TB * TB / NT;
+    extern __shared__ __align__(16) double lds[];
+    __shared__ ResTile tiles[kResMaxTiles];
+    __shared__ int fire[3][kResMaxTiles];  // detector bits of step s in fire[s % 3]
+    __shared__ int gone;                   // a wait ran out
+    __shared__ uint64_t sact[2];           // awake tiles of step s: positions of the region and two tiles around it
+    CInst& I = ((CInst*)insts)[0];
+    const int tid = threadIdx.x, lane = tid & 63, nthr = blockDim.x;
+    const int nx = I.nx, ny = I.ny, ntx = I.ntx, nty = I.nty, bcx = I.bc_x, bcy = I.bc_y;
+    const bool regular = I.mode == 0;
+    const double kappa = I.kappa, eps = I.thresh_a, inv = NINE ? I.inv6dx2 : I.invdx2;
+    const double dt = I.dt, mob = I.mobility, rg = I.react_gamma, cbar = I.cbar;
+    gdouble* mu_store = I.aux[0];
+    const int nrx = (ntx + gx - 1) / gx;
+    const int rgn = blockIdx.x, rx = rgn % nrx, ry = rgn / nrx;
+    const int ti0 = rx * gx, tj0 = ry * gy;
+    const int kx = min(gx, ntx - ti0), ky = min(gy, nty - tj0), nk = kx * ky;  // the region's tiles
+    const int x0 = ti0 * TB, y0 = tj0 * TB;
+    const int w = min(kx * TB, nx - x0), h = min(ky * TB, ny - y0);
+    const int W2 = w + 4, W1 = w + 2;
+    const int nh = W2 * (h + 4) - w * h, nr = W1 * (h + 2) - w * h, ne = 2 * w + 2 * h - 4;
+    double* sc = lds;                         // c at (x, y): sc[x + 2 + (y + 2) W2]
+    double* smu = sc + (size_t)W2 * (h + 4);  // mu at (x, y): smu[x + 1 + (y + 1) W1]
+    int* ht = (int*)(smu + (size_t)W1 * (h + 2));
+    int* hc = ht + nh;  // window index of the halo cells
+    int* rt = hc + nh;
+    const int PW = kx + 4, np = PW * (ky + 4);  // positions: tile (i, j) of the region at (i + 2) + (j + 2) PW
+    const int64_t plane = (int64_t)gridDim.x * X.slots * 2;
+
+    // the tile at position p (this lane's), or -1 outside a closed boundary
+    int near = -1;
+    if (lane < np) {
+        int i = ti0 + lane % PW - 2, j = tj0 + lane / PW - 2;
+        if (bcx == 0) i = ((i % ntx) + ntx) % ntx;
+        if (bcy == 0) j = ((j % nty) + nty) % nty;
+        if (i >= 0 && i < ntx && j >= 0 && j < nty) near = i + j * ntx;
+    }
+    // position of the tile that holds mapped cell (mx, my), seen from a cell (x, y)
+    // outside the region: mirrored cells belong to the region's own tiles
+    auto pos_of = [&](int x, int y) {
+        const int gxx = x0 + x, gyy = y0 + y;
+        int i, j;
+        if (bcx != 0 && (gxx < 0 || gxx >= nx)) i = map_index(gxx, nx, bcx) / TB - ti0;
+        else i = x < 0 ? -1 : (x >= w ? kx : x / TB);
+        if (bcy != 0 && (gyy < 0 || gyy >= ny)) j = map_index(gyy, ny, bcy) / TB - tj0;
+        else j = y < 0 ? -1 : (y >= h ? ky : y / TB);
+        return (i + 2) + (j + 2) * PW;
+    };
+
+    // ---- tables and the state the launch starts from
+    if (tid < nk) {
+        const int i = tid % kx, j = tid / kx;
+        ResTile& T = tiles[tid];
+        T.t = (ti0 + i) + (tj0 + j) * ntx;
+        T.x = i * TB;
+        T.y = j * TB;
+        T.w = min(TB, w - T.x);
+        T.h = min(TB, h - T.y);
+        T.par = bit_of(I.par[0], T.t);
+        T.runs = 0;
+        T.last = 1;
+        T.pos = (i + 2) + (j + 2) * PW;
+        for (int q = 0; q < 3; q++) fire[q][tid] = 0;
+    }
+    if (tid < 64) {
+        const int a = near >= 0 && (regular || bit_of(I.a_cur[0], near));
+        const uint64_t m = __ballot(a);
+        if (lane == 0) {
+            sact[0] = m;
+            sact[1] = 0ull;
+            gone = 0;
+        }
+    }
+    for (int k = tid; k < w * h; k += nthr) {
+        const int x = k % w, y = k / w, t = (ti0 + x / TB) + (tj0 + y / TB) * ntx;
+        sc[(x + 2) + (y + 2) * W2] = I.buf[bit_of(I.par[0], t)][0][(x0 + x) + (int64_t)(y0 + y) * nx];
+    }
+    for (int k = tid; k < nh; k += nthr) {
+        int x, y;
+        outer_cell<2>(k, w, h, &x, &y);
+        const int mx = map_index(x0 + x, nx, bcx), my = map_index(y0 + y, ny, bcy);
+        const int oi = mx / TB, oj = my / TB, ox = oi / gx, oy = oj / gy, bx = ox * gx * TB, by = oy * gy * TB;
+        const int slot = frame_slot(mx - bx, my - by, min(gx * TB, nx - bx), min(gy * TB, ny - by));
+        ht[k] = ((ox + oy * nrx) * X.slots + slot) << 6 | pos_of(x, y);
+        hc[k] = (x + 2) + (y + 2) * W2;
+        sc[hc[k]] = I.buf[bit_of(I.par[0], oi + oj * ntx)][0][mx + (int64_t)my * nx];
+    }
+    for (int k = tid; k < nr + ne; k += nthr) {
+        int x, y, own = 0, p;
+        if (k < nr) {
+            outer_cell<1>(k, w, h, &x, &y);
+            p = pos_of(x, y);
+        } else {
+            int lx, ly;
+            TileRing<TB>::cell(k - nr, &lx, &ly, w, h);
+            x = lx;
+            y = ly;
+            own = 1 + x / TB + y / TB * kx;
+            p = (x / TB + 2) + (y / TB + 2) * PW;
+        }
+        rt[k] = (x + 1) | (y + 1) << 9 | p << 18 | own << 24;
+        if (!own && !regular) {  // a sleeping owner's stored potential
+            const int mx = map_index(x0 + x, nx, bcx), my = map_index(y0 + y, ny, bcy);
+            smu[(x + 1) + (y + 1) * W1] = TileRing<TB>::stale(mu_store, mx / TB + (my / TB) * ntx, mx, my, nx, ny);
+        }
+    }
+    __syncthreads();
+    if (!regular)  // the stored rings of the region's own tiles (read while they sleep)
+        for (int j = 0; j < nk; j++) {
+            const ResTile& T = tiles[j];
+            for (int k = tid; k < TileRing<TB>::size(T.w, T.h); k += nthr) {
+                int lx, ly;
+                TileRing<TB>::cell(k, &lx, &ly, T.w, T.h);
+                smu[(T.x + lx + 1) + (T.y + ly + 1) * W1] = mu_store[(int64_t)T.t * TileRing<TB>::N + k];
+            }
+        }
+    __syncthreads();
+
+    const int grp = tid / NT, gn = nthr / NT;  // NT threads work on a tile at a time
+    const int tx = (tid % NT) % TB, ty = (tid % NT) / TB;
+    auto strip = [&](const double* s, int stride, int x, int y, double (&out)[R], double (&c)[R]) {
+        double L[R + 2], M[R + 2], Rt[R + 2];
+#pragma unroll
+        for (int r = 0; r < R + 2; r++) {
+            const double* q = s + x + (y - 1 + r) * stride;
+            L[r] = q[-1];
+            M[r] = q[0];
+            Rt[r] = q[1];
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const double s1 = (Rt[r + 1] + L[r + 1]) + (M[r + 2] + M[r]);
+            if (NINE) {
+                const double s2 = (Rt[r + 2] + L[r + 2]) + (Rt[r] + L[r]);
+                out[r] = ((4.0 * s1 + s2) - 20.0 * M[r + 1]) * inv;
+            } else {
+                out[r] = (s1 - 4.0 * M[r + 1]) * inv;
+            }
+            c[r] = M[r + 1];
+        }
+    };
+    // mu of tile j but for the region's edge cells (their halo may be on its way)
+    auto tile_mu = [&](int j, int* f) {
+        const ResTile& T = tiles[j];
+        double lc[R], c[R];
+        int flag = 0;
+        // rows past a partial tile read other window rows, and are not used
+        const int yb = T.y + ty * R;
+        if (tx < T.w && ty * R < T.h) {
+            strip(sc, W2, T.x + tx + 2, yb + 2, lc, c);
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const int x = T.x + tx, y = yb + r;
+                if (ty * R + r < T.h && x > 0 && x < w - 1 && y > 0 && y < h - 1) {
+                    smu[(x + 1) + (y + 1) * W1] = (c[r] * c[r] * c[r] - c[r]) - kappa * lc[r];
+                    flag |= fabs(lc[r]) > eps;
+                }
+            }
+        }
+        const unsigned long long v = __ballot(flag);
+        if (lane == 0 && v) f[j] = 1;
+    };
+
+    // frame slots of the thread's cells of the group's first tile (-1: not published)
+    int slot0[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        slot0[r] = -1;
+        if (grp < nk) {
+            const ResTile& T = tiles[grp];
+            if (tx < T.w && ty * R + r < T.h) slot0[r] = frame_slot(T.x + tx, T.y + ty * R + r, w, h);
+        }
+    }
+
+#pragma unroll 1
+    for (int s = 0; s < n; s++) {
+        const uint32_t seq = X.base + (uint32_t)s;
+        const uint64_t* fin = X.frame + (s & 1) * plane;
+        uint64_t* fout = X.frame + ((s & 1) ^ 1) * plane;
+        int* f = fire[s % 3];
+        const int* fp = fire[(s + 2) % 3];
+        // 1. mu of the tiles that certainly run
+        for (int j = grp; j < nk; j += gn)
+            if (regular || (s > 0 && fp[j])) tile_mu(j, f);
+        // 2. the frames of the tiles outside that ran, the detector bits around
+        if (s > 0) {
+            const uint64_t ran = sact[(s & 1) ^ 1];
+            for (int k = tid; k < nh; k += nthr) {
+                const int e = ht[k];
+                if (!((ran >> (e & 63)) & 1ull)) continue;
+                sc[hc[k]] = wait_double(fin + 2 * (int64_t)(e >> 6), seq, X.stuck, &gone);
+            }
+            if (tid >= nthr - 64) {
+                uint64_t m = ~0ull;
+                if (!regular) {
+                    const uint64_t* fl = X.flag + (int64_t)((s & 1) ^ 1) * I.nt;
+                    const int px = lane % PW, py = lane / PW;
+                    const bool inside = px >= 2 && px < kx + 2 && py >= 2 && py < ky + 2;
+                    int b = 0;
+                    if (inside && lane < np) b = fp[(px - 2) + (py - 2) * kx];
+                    else if (near >= 0) b = wait_flag(fl + near, seq, X.stuck, &gone);
+                    m = __ballot(b);
+                    m |= m << 1 | m >> 1 | m << PW | m >> PW;  // (rows touch only past the positions in use)
+                    m &= __ballot(near >= 0);
+                } else {
+                    m = __ballot(near >= 0);
+                }
+                if (lane == 0) sact[s & 1] = m;
+            }
+        }
+        if (tid < kResMaxTiles) fire[(s + 1) % 3][tid] = 0;
+        lds_barrier();
+        const uint64_t act = sact[s & 1];
+        auto runs = [&](int j) { return (act >> tiles[j].pos) & 1ull; };
+        // 3. mu of tiles a neighbour woke, of the region's edge, of the ring of running tiles outside
+        for (int j = grp; j < nk; j += gn)
+            if (!regular && !(s > 0 && fp[j]) && runs(j)) tile_mu(j, f);
+        for (int k = tid; k < nr + ne; k += nthr) {
+            const int e = rt[k], x = (e & 511), y = (e >> 9) & 511, p = (e >> 18) & 63;
+            if (!((act >> p) & 1ull)) continue;
+            const double* q = sc + (x + 1) + (y + 1) * W2;
+            const double s1 = (q[1] + q[-1]) + (q[W2] + q[-W2]);
+            double lc;
+            if (NINE) {
+                const double s2 = (q[W2 + 1] + q[W2 - 1]) + (q[-W2 + 1] + q[-W2 - 1]);
+                lc = ((4.0 * s1 + s2) - 20.0 * q[0]) * inv;
+            } else {
+                lc = (s1 - 4.0 * q[0]) * inv;
+            }
+            const double cv = q[0];
+            smu[x + y * W1] = (cv * cv * cv - cv) - kappa * lc;
+            if ((e >> 24) && fabs(lc) > eps) f[(e >> 24) - 1] = 1;
+        }
+        lds_barrier();
+        // 4. c' into the window, the region's frame to the others
+        for (int j = grp; j < nk; j += gn) {
+            if (!runs(j)) continue;
+            const ResTile& T = tiles[j];
+            if (tx < T.w && ty * R < T.h) {
+                double lm[R], mu[R];
+                const int yb = T.y + ty * R, x = T.x + tx;
+                strip(smu, W1, x + 1, yb + 1, lm, mu);
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const int y = yb + r;
+                    if (ty * R + r < T.h) {
+                        double* q = sc + (x + 2) + (y + 2) * W2;
+                        const double cv = *q, change = dt * (mob * lm[r] - rg * (cv - cbar)), cn = cv + change;
+                        *q = cn;
+                        const int slot = j == grp ? slot0[r] : frame_slot(x, y, w, h);
+                        if (slot >= 0 && s + 1 < n) put_double(fout + 2 * ((int64_t)rgn * X.slots + slot), cn, seq + 1);
+                    }
+                }
+            }
+        }
+        if (tid < nk) {
+            ResTile& T = tiles[tid];
+            const bool ran = runs(tid);
+            const int any = !regular && ran ? f[tid] : 0;
+            if (!regular && s + 1 < n)
+                xput(X.flag + (int64_t)(s & 1) * I.nt + T.t, (uint64_t)(seq + 1) << 32 | (uint32_t)any);
+            f[tid] = any;
+            if (ran) {
+                T.runs++;
+                T.last = any;
+                if (I.hist_cap > 0) {
+                    const int64_t step = I.ctr[0] + s;
+                    if (step < I.hist_cap) atomicAdd((int*)&I.hist[2 * step], 1);
+                }
+            }
+        }
+        lds_barrier();
+        if (gone) break;
+    }
+
+    // ---- the state the other paths read: the cells into the buffer that was not
+    //      current (others may still read this launch's start from that one), the
+    //      rings, the per-tile bytes of the last step, the update counts
+    for (int j = 0; j < nk; j++) {
+        const ResTile& T = tiles[j];
+        if (T.runs > 0) {
+            gdouble* out = I.buf[T.par ^ 1][0];
+            for (int k = tid; k < T.w * T.h; k += nthr) {
+                const int x = T.x + k % T.w, y = T.y + k / T.w;
+                out[(x0 + x) + (int64_t)(y0 + y) * nx] = sc[(x + 2) + (y + 2) * W2];
+            }
+            if (!regular && !T.last)
+                for (int k = tid; k < TileRing<TB>::size(T.w, T.h); k += nthr) {
+                    int lx, ly;
+                    TileRing<TB>::cell(k, &lx, &ly, T.w, T.h);
+                    mu_store[(int64_t)T.t * TileRing<TB>::N + k] = smu[(T.x + lx + 1) + (T.y + ly + 1) * W1];
+                }
+        }
+        if (tid == 0) {
+            I.dF[n & 1][T.t] = (uint8_t)fire[(n + 2) % 3][j];
+            I.dP[n & 1][T.t] = (uint8_t)(T.par ^ (T.runs > 0));
+            I.druns[T.t] = T.runs;
+        }
+    }
+}
+
+}  // namespace dba

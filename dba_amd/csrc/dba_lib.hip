@@ -913,15 +913,16 @@ void resident_choose(const dba_ctx* ctx, Group* g, const Inst& h) {
     // larger regions (fewer frames). us per step over 1000 steps, single-launch
     // steps -> this: 32 x 32 tiles 256^2 4.4 -> 2.7 (512 or 1024 threads per tile; 256: 3.5),
     // 1024^2 7.1 -> 4.4 (one tile per workgroup: 7.0, two: 7.1), 1200 x 1100
-    // 15.2 -> 6.5; 16 x 16 tiles 512^2 4.5 -> 2.8, 1024^2 8.4 -> 5.1; 8 x 8 tiles
-    // 512^2 5.7 -> 3.2
-    std::vector<Shape> shapes = {{1, 1, 1024, 1024}, {2, 2, 1024, 256}, {3, 2, 768, 256}};
+    // 15.2 -> 6.2, 1571 x 1390 15.8 -> 7.7; 16 x 16 tiles 512^2 4.5 -> 2.6, 1024^2 8.4 -> 5.0; 8 x 8 tiles
+    // 512^2 5.7 -> 3.1
+    std::vector<Shape> shapes = {{1, 1, 1024, 1024}, {2, 2, 1024, 256}, {3, 2, 768, 256}, {3, 3, 1024, 256}};
     if (g->tile == 16) shapes = {{2, 2, 512, 128}, {4, 4, 1024, 128}};
     if (g->tile == 8) shapes = {{4, 2, 512, 64}, {4, 4, 1024, 64}};
     for (const Shape& s : shapes) {
         const void* f = resident_kernel(g, s.per_tile);
         const size_t lds = ch_resident_bytes(g->tile * s.gx, g->tile * s.gy);
         const int64_t wgs = (int64_t)((h.ntx + s.gx - 1) / s.gx) * ((h.nty + s.gy - 1) / s.gy);
+        if (s.threads < ch_resident_threads(g->tile * s.gx, g->tile * s.gy)) continue;
         if (!all_resident(ctx, f, s.threads, lds, wgs)) continue;
         g->res_gx = s.gx;
         g->res_gy = s.gy;

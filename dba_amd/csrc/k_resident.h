@@ -124,9 +124,12 @@ struct ResTile {
 
 // LDS bytes of a region of w x h cells.
 constexpr size_t ch_resident_bytes(int w, int h) {
-    return sizeof(double) * ((size_t)(w + 4) * (h + 4) + (size_t)(w + 2) * (h + 2)) +
-           sizeof(int) * (2 * (size_t)(4 * (w + h) + 16) + (size_t)(4 * (w + h)));
+    return sizeof(double) * ((size_t)(w + 4) * (h + 4) + (size_t)(w + 2) * (h + 2));
 }
+
+// Threads a region of w x h cells needs at least: one for each cell of its halo (and
+// of its mu ring and edge), whose place and owner that thread keeps in registers.
+constexpr int ch_resident_threads(int w, int h) { return 4 * (w + h) + 16; }
 
 // n steps of one CH instance (regular or DBA). The region's c (with a two-cell
 // halo) and mu (with a one-cell ring) stay in LDS windows for the whole launch; per
@@ -168,9 +171,6 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
     const int nh = W2 * (h + 4) - w * h, nr = W1 * (h + 2) - w * h, ne = 2 * w + 2 * h - 4;
     double* sc = lds;                         // c at (x, y): sc[x + 2 + (y + 2) W2]
     double* smu = sc + (size_t)W2 * (h + 4);  // mu at (x, y): smu[x + 1 + (y + 1) W1]
-    int* ht = (int*)(smu + (size_t)W1 * (h + 2));
-    int* hc = ht + nh;  // window index of the halo cells
-    int* rt = hc + nh;
     const int PW = kx + 4, np = PW * (ky + 4);  // positions: tile (i, j) of the region at (i + 2) + (j + 2) PW
     const int64_t plane = (int64_t)gridDim.x * X.slots * 2;
 
@@ -222,33 +222,36 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
         const int x = k % w, y = k / w, t = (ti0 + x / TB) + (tj0 + y / TB) * ntx;
         sc[(x + 2) + (y + 2) * W2] = I.buf[bit_of(I.par[0], t)][0][(x0 + x) + (int64_t)(y0 + y) * nx];
     }
-    for (int k = tid; k < nh; k += nthr) {
+    // this thread's cell of the halo: where it is published, the tile position of its owner, its place
+    int hslot = 0, hpos = -1, hcell = 0;
+    if (tid < nh) {
         int x, y;
-        outer_cell<2>(k, w, h, &x, &y);
+        outer_cell<2>(tid, w, h, &x, &y);
         const int mx = map_index(x0 + x, nx, bcx), my = map_index(y0 + y, ny, bcy);
         const int oi = mx / TB, oj = my / TB, ox = oi / gx, oy = oj / gy, bx = ox * gx * TB, by = oy * gy * TB;
         const int slot = frame_slot(mx - bx, my - by, min(gx * TB, nx - bx), min(gy * TB, ny - by));
-        ht[k] = ((ox + oy * nrx) * X.slots + slot) << 6 | pos_of(x, y);
-        hc[k] = (x + 2) + (y + 2) * W2;
-        sc[hc[k]] = I.buf[bit_of(I.par[0], oi + oj * ntx)][0][mx + (int64_t)my * nx];
+        hslot = 2 * ((ox + oy * nrx) * X.slots + slot);
+        hpos = pos_of(x, y);
+        hcell = (x + 2) + (y + 2) * W2;
+        sc[hcell] = I.buf[bit_of(I.par[0], oi + oj * ntx)][0][mx + (int64_t)my * nx];
     }
-    for (int k = tid; k < nr + ne; k += nthr) {
-        int x, y, own = 0, p;
-        if (k < nr) {
-            outer_cell<1>(k, w, h, &x, &y);
-            p = pos_of(x, y);
+    // ... and of the ring outside or the edge inside: its owner (own: region tile + 1, 0 outside), its place
+    int rpos = -1, rx1 = 0, ry1 = 0, own = 0;
+    if (tid < nr + ne) {
+        int x, y;
+        if (tid < nr) {
+            outer_cell<1>(tid, w, h, &x, &y);
+            rpos = pos_of(x, y);
         } else {
-            int lx, ly;
-            TileRing<TB>::cell(k - nr, &lx, &ly, w, h);
-            x = lx;
-            y = ly;
+            TileRing<TB>::cell(tid - nr, &x, &y, w, h);
             own = 1 + x / TB + y / TB * kx;
-            p = (x / TB + 2) + (y / TB + 2) * PW;
+            rpos = (x / TB + 2) + (y / TB + 2) * PW;
         }
-        rt[k] = (x + 1) | (y + 1) << 9 | p << 18 | own << 24;
+        rx1 = x + 1;
+        ry1 = y + 1;
         if (!own && !regular) {  // a sleeping owner's stored potential
             const int mx = map_index(x0 + x, nx, bcx), my = map_index(y0 + y, ny, bcy);
-            smu[(x + 1) + (y + 1) * W1] = TileRing<TB>::stale(mu_store, mx / TB + (my / TB) * ntx, mx, my, nx, ny);
+            smu[rx1 + ry1 * W1] = TileRing<TB>::stale(mu_store, mx / TB + (my / TB) * ntx, mx, my, nx, ny);
         }
     }
     __syncthreads();
@@ -332,11 +335,7 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
         // 2. the frames of the tiles outside that ran, the detector bits around
         if (s > 0) {
             const uint64_t ran = sact[(s & 1) ^ 1];
-            for (int k = tid; k < nh; k += nthr) {
-                const int e = ht[k];
-                if (!((ran >> (e & 63)) & 1ull)) continue;
-                sc[hc[k]] = wait_double(fin + 2 * (int64_t)(e >> 6), seq, X.stuck, &gone);
-            }
+            if (hpos >= 0 && ((ran >> hpos) & 1ull)) sc[hcell] = wait_double(fin + hslot, seq, X.stuck, &gone);
             if (tid >= nthr - 64) {
                 uint64_t m = ~0ull;
                 if (!regular) {
@@ -362,10 +361,8 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
         // 3. mu of tiles a neighbour woke, of the region's edge, of the ring of running tiles outside
         for (int j = grp; j < nk; j += gn)
             if (!regular && !(s > 0 && fp[j]) && runs(j)) tile_mu(j, f);
-        for (int k = tid; k < nr + ne; k += nthr) {
-            const int e = rt[k], x = (e & 511), y = (e >> 9) & 511, p = (e >> 18) & 63;
-            if (!((act >> p) & 1ull)) continue;
-            const double* q = sc + (x + 1) + (y + 1) * W2;
+        if (rpos >= 0 && ((act >> rpos) & 1ull)) {
+            const double* q = sc + (rx1 + 1) + (ry1 + 1) * W2;
             const double s1 = (q[1] + q[-1]) + (q[W2] + q[-W2]);
             double lc;
             if (NINE) {
@@ -375,8 +372,8 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
                 lc = (s1 - 4.0 * q[0]) * inv;
             }
             const double cv = q[0];
-            smu[x + y * W1] = (cv * cv * cv - cv) - kappa * lc;
-            if ((e >> 24) && fabs(lc) > eps) f[(e >> 24) - 1] = 1;
+            smu[rx1 + ry1 * W1] = (cv * cv * cv - cv) - kappa * lc;
+            if (own && fabs(lc) > eps) f[own - 1] = 1;
         }
         lds_barrier();
         // 4. c' into the window, the region's frame to the others

@@ -53,7 +53,7 @@ def same(a, b):
 @pytest.mark.parametrize("mode", [abi.MODE_REGULAR, abi.MODE_DBA])
 @pytest.mark.parametrize("nx,ny,tile,stencil,bc", [
     (32, 32, 32, 9, 0), (64, 66, 32, 5, 0), (8, 10, 8, 9, 0), (40, 24, 8, 5, 1), (70, 130, 16, 9, 1),
-    (1024, 1024, 32, 9, 0), (1000, 996, 32, 9, 1), (1200, 1100, 32, 5, 0), (514, 480, 8, 9, 0), (900, 700, 16, 5, 0)])
+    (1024, 1024, 32, 9, 0), (1000, 996, 32, 9, 1), (1200, 1100, 32, 5, 0), (1534, 1310, 32, 9, 0), (514, 480, 8, 9, 0), (900, 700, 16, 5, 0)])
 def test_resident_equals_worklist(ctx, mode, nx, ny, tile, stencil, bc):
     p = configs.ch_params(n=nx, ny=ny, tile=tile, mode=mode, stencil=stencil, eps=1e-3, react_gamma=0.01, cbar=0.05,
                           history_cap=128)

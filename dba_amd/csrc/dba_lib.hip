@@ -26,6 +26,7 @@
 #include "k_ch.h"
 #include "k_resident.h"
 #include "k_k93.h"
+#include "k_resident_k93.h"
 #include "k_kh.h"
 #include "k_ref3d.h"
 #include "k_diag.h"
@@ -497,8 +498,9 @@ dba_status get_group(dba_ctx* ctx, const std::vector<int>& ids, Group** out) {
                 break;
             }
     }
-    // Resident steps: one CH instance (regular or DBA) whose tiles fit the chip at once
-    if (ids.size() == 1 && g->model == DBA_MODEL_CH && first->p.mode != DBA_MODE_CONSERVED && first->p.threads == 0)
+    // Resident steps: one CH or K93 instance (regular or DBA) whose tiles fit the chip at once
+    if (ids.size() == 1 && first->p.mode != DBA_MODE_CONSERVED && first->p.threads == 0 &&
+        (g->model == DBA_MODEL_CH || g->model == DBA_MODEL_DENDRITE_K93))
         resident_choose(ctx, g, first->h);
     // Speculative staging in single-launch K93 steps (k93_dense_kernel SPEC):
     // one instance of up to 1024 full 16 x 16 tiles at 512 threads (measured on
@@ -870,13 +872,22 @@ const void* ch_resident_fn(bool nine) {
     return nine ? (const void*)ch_resident_kernel<TB, NT, true> : (const void*)ch_resident_kernel<TB, NT, false>;
 }
 
-// The kernel of a group's tile with `per_tile` threads on each tile.
+// The kernel of a group's tile: `per_tile` threads on each tile (K93: one per cell).
 const void* resident_kernel(const Group* g, int per_tile) {
+    if (g->model == DBA_MODEL_DENDRITE_K93) switch (g->tile) {
+            case 8: return (const void*)k93_resident_kernel<8>;
+            case 16: return (const void*)k93_resident_kernel<16>;
+            default: return (const void*)k93_resident_kernel<32>;
+        }
     switch (g->tile) {
         case 8: return ch_resident_fn<8, 64>(g->nine);
         case 16: return ch_resident_fn<16, 128>(g->nine);
         default: return per_tile == 1024 ? ch_resident_fn<32, 1024>(g->nine) : ch_resident_fn<32, 256>(g->nine);
     }
+}
+
+size_t resident_bytes(const Group* g, int w, int h) {
+    return g->model == DBA_MODEL_DENDRITE_K93 ? k93_resident_bytes(w, h) : ch_resident_bytes(w, h);
 }
 
 // Whether `wgs` workgroups of the kernel are certainly resident at once. The
@@ -918,9 +929,20 @@ void resident_choose(const dba_ctx* ctx, Group* g, const Inst& h) {
     std::vector<Shape> shapes = {{1, 1, 1024, 1024}, {2, 2, 1024, 256}, {3, 2, 768, 256}, {3, 3, 1024, 256}};
     if (g->tile == 16) shapes = {{2, 2, 512, 128}, {4, 4, 1024, 128}};
     if (g->tile == 8) shapes = {{4, 2, 512, 64}, {4, 4, 1024, 64}};
+    // K93: one cell per thread. Several cells per thread (4 x 4 tiles of 16 x 16) make a
+    // larger grid fit, but one dendrite's awake tiles then crowd on few CUs: 1000^2
+    // 16.5 us per step against 7.9. Smaller regions with several on a CU exchange more:
+    // 512^2 4.3 - 5.2 against 4.0. us per step over 1000 steps, single-launch steps ->
+    // this: 16 x 16 tiles 256^2 4.9 -> 3.5, 512^2 5.8 -> 4.0 (regular mode 9.2 -> 3.4);
+    // 8 x 8 tiles 512^2 6.9 -> 4.4; 32 x 32 tiles 512^2 7.6 -> 4.2
+    if (g->model == DBA_MODEL_DENDRITE_K93) {
+        shapes = {{1, 1, 1024, 1024}};
+        if (g->tile == 16) shapes = {{1, 1, 256, 256}, {2, 2, 1024, 256}};
+        if (g->tile == 8) shapes = {{2, 2, 256, 64}, {4, 4, 1024, 64}};
+    }
     for (const Shape& s : shapes) {
         const void* f = resident_kernel(g, s.per_tile);
-        const size_t lds = ch_resident_bytes(g->tile * s.gx, g->tile * s.gy);
+        const size_t lds = resident_bytes(g, g->tile * s.gx, g->tile * s.gy);
         const int64_t wgs = (int64_t)((h.ntx + s.gx - 1) / s.gx) * ((h.nty + s.gy - 1) / s.gy);
         if (s.threads < ch_resident_threads(g->tile * s.gx, g->tile * s.gy)) continue;
         if (!all_resident(ctx, f, s.threads, lds, wgs)) continue;
@@ -974,12 +996,14 @@ dba_status enqueue_resident(dba_ctx* ctx, Group* g, int n_steps, bool* taken) {
     const int nt = h.nt, gx = g->res_gx, gy = g->res_gy;
     const unsigned wgs = (unsigned)(((h.ntx + gx - 1) / gx) * ((h.nty + gy - 1) / gy));
     const int slots = frame_slots(gx * g->tile, gy * g->tile);
-    const size_t words = 2 * (size_t)wgs * (size_t)slots * 2 + 2 * (size_t)nt;
+    const size_t flags = 2 * (size_t)nt;
+    const int fields = g->model == DBA_MODEL_DENDRITE_K93 ? 2 : 1;
+    const size_t words = 2 * (size_t)wgs * (size_t)slots * 2 * fields + flags;
     bool ok = resident_buffer(ctx, words, n_steps);
     if (ok) {
         const void* f = resident_kernel(g, g->res_per_tile);
-        const size_t lds = ch_resident_bytes(gx * g->tile, gy * g->tile);
-        Exchange X{ctx->xbuf, ctx->xbuf + (words - 2 * (size_t)nt), ctx->stuck, ctx->xseq, slots};
+        const size_t lds = resident_bytes(g, gx * g->tile, gy * g->tile);
+        Exchange X{ctx->xbuf, ctx->xbuf + (words - flags), ctx->stuck, ctx->xseq, slots};
         const Inst* insts = g->d_insts;
         int n = n_steps, ax = gx, ay = gy;
         void* args[] = {(void*)&insts, (void*)&X, (void*)&n, (void*)&ax, (void*)&ay};

@@ -30,8 +30,8 @@
 namespace dba {
 
 struct Exchange {
-    uint64_t* frame;   // [parity][region][slot][2]
-    uint64_t* flag;    // [parity][tile]: sequence number << 32 | detector bit
+    uint64_t* frame;   // [parity][region][slot][2 words per field]
+    uint64_t* flag;    // [parity][tile]: sequence number << 32 | detector bits
     int* stuck;        // host memory: a wait ran out
     uint32_t base;     // sequence number of the launch's first step
     int slots;         // frame slots of a whole region
@@ -84,7 +84,7 @@ __device__ __forceinline__ int wait_flag(const uint64_t* p, uint32_t seq, int* s
             break;
         }
     }
-    return (int)(a & 1ull);
+    return (int)(a & 3ull);
 }
 
 // The published cells of a w x h region: two cells deep on each side, every cell
@@ -131,6 +131,66 @@ constexpr size_t ch_resident_bytes(int w, int h) {
 // of its mu ring and edge), whose place and owner that thread keeps in registers.
 constexpr int ch_resident_threads(int w, int h) { return 4 * (w + h) + 16; }
 
+// A workgroup's region: gx x gy tiles of TB x TB (fewer at the grid's end), its cells
+// from (x0, y0), and the positions of its tiles and the two tiles around it on every
+// side: tile (i, j) of the region at (i + 2) + (j + 2) PW.
+template <int TB>
+struct Region {
+    int nx, ny, ntx, nty, bcx, bcy, gx, gy, nrx, rgn, ti0, tj0, kx, ky, nk, x0, y0, w, h, PW;
+
+    __device__ __forceinline__ Region(CInst& I, int gx_, int gy_)
+        : nx(I.nx), ny(I.ny), ntx(I.ntx), nty(I.nty), bcx(I.bc_x), bcy(I.bc_y), gx(gx_), gy(gy_),
+          nrx((I.ntx + gx_ - 1) / gx_), rgn(blockIdx.x) {
+        ti0 = rgn % nrx * gx;
+        tj0 = rgn / nrx * gy;
+        kx = min(gx, ntx - ti0);
+        ky = min(gy, nty - tj0);
+        nk = kx * ky;
+        x0 = ti0 * TB;
+        y0 = tj0 * TB;
+        w = min(kx * TB, nx - x0);
+        h = min(ky * TB, ny - y0);
+        PW = kx + 4;
+    }
+    // the tile at position p, or -1 outside a closed boundary or past the positions
+    __device__ __forceinline__ int near(int p) const {
+        if (p >= PW * (ky + 4)) return -1;
+        int i = ti0 + p % PW - 2, j = tj0 + p / PW - 2;
+        if (bcx == 0) i = ((i % ntx) + ntx) % ntx;
+        if (bcy == 0) j = ((j % nty) + nty) % nty;
+        return i >= 0 && i < ntx && j >= 0 && j < nty ? i + j * ntx : -1;
+    }
+    // the region's tile (i + j kx) at position p, or -1
+    __device__ __forceinline__ int inside(int p) const {
+        const int i = p % PW - 2, j = p / PW - 2;
+        return i >= 0 && i < kx && j >= 0 && j < ky ? i + j * kx : -1;
+    }
+    // position of the tile that holds the mapped cell of (x, y), a cell outside the
+    // region: mirrored cells belong to the region's own tiles
+    __device__ __forceinline__ int pos_of(int x, int y) const {
+        const int gxx = x0 + x, gyy = y0 + y;
+        int i, j;
+        if (bcx != 0 && (gxx < 0 || gxx >= nx)) i = map_index(gxx, nx, bcx) / TB - ti0;
+        else i = x < 0 ? -1 : (x >= w ? kx : x / TB);
+        if (bcy != 0 && (gyy < 0 || gyy >= ny)) j = map_index(gyy, ny, bcy) / TB - tj0;
+        else j = y < 0 ? -1 : (y >= h ? ky : y / TB);
+        return (i + 2) + (j + 2) * PW;
+    }
+    // mapped cell of (x, y): its tile, and its slot among the frames of all regions
+    __device__ __forceinline__ void source(int x, int y, int slots, int* mx, int* my, int* tile, int* slot) const {
+        *mx = map_index(x0 + x, nx, bcx);
+        *my = map_index(y0 + y, ny, bcy);
+        const int oi = *mx / TB, oj = *my / TB, ox = oi / gx, oy = oj / gy, bx = ox * gx * TB, by = oy * gy * TB;
+        *tile = oi + oj * ntx;
+        *slot = (ox + oy * nrx) * slots +
+                frame_slot(*mx - bx, *my - by, min(gx * TB, nx - bx), min(gy * TB, ny - by));
+    }
+    // awake positions of a step from the detector bits of the step before
+    __device__ __forceinline__ uint64_t dilate(uint64_t m, uint64_t exist) const {
+        return (m | m << 1 | m >> 1 | m << PW | m >> PW) & exist;  // (rows touch only past the positions in use)
+    }
+};
+
 // n steps of one CH instance (regular or DBA). The region's c (with a two-cell
 // halo) and mu (with a one-cell ring) stay in LDS windows for the whole launch; per
 // tile and step the arithmetic, its order and the detector are ch_tile's, so results
@@ -156,43 +216,20 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
     __shared__ uint64_t sact[2];           // awake tiles of step s: positions of the region and two tiles around it
     CInst& I = ((CInst*)insts)[0];
     const int tid = threadIdx.x, lane = tid & 63, nthr = blockDim.x;
-    const int nx = I.nx, ny = I.ny, ntx = I.ntx, nty = I.nty, bcx = I.bc_x, bcy = I.bc_y;
+    const Region<TB> G(I, gx, gy);
+    const int nx = G.nx, ny = G.ny, ntx = G.ntx, ti0 = G.ti0, tj0 = G.tj0, kx = G.kx, nk = G.nk;
+    const int x0 = G.x0, y0 = G.y0, w = G.w, h = G.h, PW = G.PW, rgn = G.rgn;
     const bool regular = I.mode == 0;
     const double kappa = I.kappa, eps = I.thresh_a, inv = NINE ? I.inv6dx2 : I.invdx2;
     const double dt = I.dt, mob = I.mobility, rg = I.react_gamma, cbar = I.cbar;
     gdouble* mu_store = I.aux[0];
-    const int nrx = (ntx + gx - 1) / gx;
-    const int rgn = blockIdx.x, rx = rgn % nrx, ry = rgn / nrx;
-    const int ti0 = rx * gx, tj0 = ry * gy;
-    const int kx = min(gx, ntx - ti0), ky = min(gy, nty - tj0), nk = kx * ky;  // the region's tiles
-    const int x0 = ti0 * TB, y0 = tj0 * TB;
-    const int w = min(kx * TB, nx - x0), h = min(ky * TB, ny - y0);
     const int W2 = w + 4, W1 = w + 2;
     const int nh = W2 * (h + 4) - w * h, nr = W1 * (h + 2) - w * h, ne = 2 * w + 2 * h - 4;
     double* sc = lds;                         // c at (x, y): sc[x + 2 + (y + 2) W2]
     double* smu = sc + (size_t)W2 * (h + 4);  // mu at (x, y): smu[x + 1 + (y + 1) W1]
-    const int PW = kx + 4, np = PW * (ky + 4);  // positions: tile (i, j) of the region at (i + 2) + (j + 2) PW
     const int64_t plane = (int64_t)gridDim.x * X.slots * 2;
 
-    // the tile at position p (this lane's), or -1 outside a closed boundary
-    int near = -1;
-    if (lane < np) {
-        int i = ti0 + lane % PW - 2, j = tj0 + lane / PW - 2;
-        if (bcx == 0) i = ((i % ntx) + ntx) % ntx;
-        if (bcy == 0) j = ((j % nty) + nty) % nty;
-        if (i >= 0 && i < ntx && j >= 0 && j < nty) near = i + j * ntx;
-    }
-    // position of the tile that holds mapped cell (mx, my), seen from a cell (x, y)
-    // outside the region: mirrored cells belong to the region's own tiles
-    auto pos_of = [&](int x, int y) {
-        const int gxx = x0 + x, gyy = y0 + y;
-        int i, j;
-        if (bcx != 0 && (gxx < 0 || gxx >= nx)) i = map_index(gxx, nx, bcx) / TB - ti0;
-        else i = x < 0 ? -1 : (x >= w ? kx : x / TB);
-        if (bcy != 0 && (gyy < 0 || gyy >= ny)) j = map_index(gyy, ny, bcy) / TB - tj0;
-        else j = y < 0 ? -1 : (y >= h ? ky : y / TB);
-        return (i + 2) + (j + 2) * PW;
-    };
+    const int near = G.near(lane);  // the tile at this lane's position
 
     // ---- tables and the state the launch starts from
     if (tid < nk) {
@@ -227,13 +264,12 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
     if (tid < nh) {
         int x, y;
         outer_cell<2>(tid, w, h, &x, &y);
-        const int mx = map_index(x0 + x, nx, bcx), my = map_index(y0 + y, ny, bcy);
-        const int oi = mx / TB, oj = my / TB, ox = oi / gx, oy = oj / gy, bx = ox * gx * TB, by = oy * gy * TB;
-        const int slot = frame_slot(mx - bx, my - by, min(gx * TB, nx - bx), min(gy * TB, ny - by));
-        hslot = 2 * ((ox + oy * nrx) * X.slots + slot);
-        hpos = pos_of(x, y);
+        int mx, my, tile;
+        G.source(x, y, X.slots, &mx, &my, &tile, &hslot);
+        hslot *= 2;
+        hpos = G.pos_of(x, y);
         hcell = (x + 2) + (y + 2) * W2;
-        sc[hcell] = I.buf[bit_of(I.par[0], oi + oj * ntx)][0][mx + (int64_t)my * nx];
+        sc[hcell] = I.buf[bit_of(I.par[0], tile)][0][mx + (int64_t)my * nx];
     }
     // ... and of the ring outside or the edge inside: its owner (own: region tile + 1, 0 outside), its place
     int rpos = -1, rx1 = 0, ry1 = 0, own = 0;
@@ -241,7 +277,7 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
         int x, y;
         if (tid < nr) {
             outer_cell<1>(tid, w, h, &x, &y);
-            rpos = pos_of(x, y);
+            rpos = G.pos_of(x, y);
         } else {
             TileRing<TB>::cell(tid - nr, &x, &y, w, h);
             own = 1 + x / TB + y / TB * kx;
@@ -250,7 +286,7 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
         rx1 = x + 1;
         ry1 = y + 1;
         if (!own && !regular) {  // a sleeping owner's stored potential
-            const int mx = map_index(x0 + x, nx, bcx), my = map_index(y0 + y, ny, bcy);
+            const int mx = map_index(x0 + x, nx, G.bcx), my = map_index(y0 + y, ny, G.bcy);
             smu[rx1 + ry1 * W1] = TileRing<TB>::stale(mu_store, mx / TB + (my / TB) * ntx, mx, my, nx, ny);
         }
     }
@@ -337,19 +373,15 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
             const uint64_t ran = sact[(s & 1) ^ 1];
             if (hpos >= 0 && ((ran >> hpos) & 1ull)) sc[hcell] = wait_double(fin + hslot, seq, X.stuck, &gone);
             if (tid >= nthr - 64) {
-                uint64_t m = ~0ull;
+                const uint64_t exist = __ballot(near >= 0);
+                uint64_t m = exist;
                 if (!regular) {
-                    const uint64_t* fl = X.flag + (int64_t)((s & 1) ^ 1) * I.nt;
-                    const int px = lane % PW, py = lane / PW;
-                    const bool inside = px >= 2 && px < kx + 2 && py >= 2 && py < ky + 2;
+                    const int own_tile = G.inside(lane);
                     int b = 0;
-                    if (inside && lane < np) b = fp[(px - 2) + (py - 2) * kx];
-                    else if (near >= 0) b = wait_flag(fl + near, seq, X.stuck, &gone);
-                    m = __ballot(b);
-                    m |= m << 1 | m >> 1 | m << PW | m >> PW;  // (rows touch only past the positions in use)
-                    m &= __ballot(near >= 0);
-                } else {
-                    m = __ballot(near >= 0);
+                    if (near >= 0)
+                        b = own_tile >= 0 ? fp[own_tile]
+                                          : wait_flag(X.flag + (int64_t)((s & 1) ^ 1) * I.nt + near, seq, X.stuck, &gone);
+                    m = G.dilate(__ballot(b), exist);
                 }
                 if (lane == 0) sact[s & 1] = m;
             }

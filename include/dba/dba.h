@@ -215,7 +215,7 @@ dba_status dba_sync(dba_ctx* ctx);
  * than 1024 tiles) at the end of each dba_step / graph chunk restores the
  * bitmaps, counters and time. Sleeping tiles still take a workgroup each, so a
  * sparse batch can run faster on the worklist path.
- * A call of 12 steps or more for one reactive CH instance (threads 0, no timing) whose
+ * A call of 12 steps or more for one reactive CH or K93 instance (threads 0, no timing) whose
  * tiles fit the GPU at once, by a context alone on its device in this process, takes
  * resident steps in modes 1 and 2: all its steps in one cooperative launch that keeps
  * the fields on chip. Processes that share a GPU take turns with such launches; set

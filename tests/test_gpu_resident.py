@@ -28,16 +28,20 @@ def patchy(nx, ny, tile, seed=7):
 
 
 def run(ctx, p, c0, mode, plan=PLAN):
+    """c0: one field, or the list of fields."""
+    fields = c0 if isinstance(c0, list) else [c0]
     ctx.set_single_launch(mode)
     try:
         inst = ctx.create(p)
-        inst.upload(0, c0)
+        for f, v in enumerate(fields):
+            inst.upload(f, v)
         out = []
         for n in plan:
             inst.step(n, graph_chunk=16)
             info = inst.info()
-            out.append((inst.download(0), inst.active(0)[1], inst.history(), info.cell_updates, info.steps_done,
-                        info.sim_time))
+            out.append((np.stack([inst.download(f) for f in range(len(fields))]),
+                        np.stack([inst.active(f)[1] for f in range(len(fields))]), inst.history(), info.cell_updates,
+                        info.field_updates, info.steps_done, info.sim_time))
         inst.destroy()
         return out
     finally:
@@ -73,8 +77,25 @@ def test_resident_matches_oracle(ctx):
     o = OracleSim(p)
     o.set_field(0, c0)
     o.step(60)
-    assert np.array_equal(got[0], o.get_field(0))
-    assert np.array_equal(got[1], o.awake(0))
+    assert np.array_equal(got[0][0], o.get_field(0))
+    assert np.array_equal(got[1][0], o.awake(0))
+
+
+# K93: one tile a workgroup (256^2 at 16 x 16) and two by two (and larger grids, which
+# do not fit and keep single-launch steps); closed boundaries as in its configuration, and periodic
+@pytest.mark.parametrize("mode", [abi.MODE_REGULAR, abi.MODE_DBA])
+@pytest.mark.parametrize("nx,ny,tile,bc", [
+    (16, 16, 16, 0), (32, 34, 16, 1), (256, 256, 16, 1), (250, 310, 16, 0), (512, 512, 16, 1), (700, 1000, 16, 1),
+    (40, 56, 8, 1), (514, 480, 8, 0), (32, 66, 32, 1), (500, 530, 32, 1), (900, 1024, 32, 0)])
+def test_resident_k93_equals_worklist(ctx, mode, nx, ny, tile, bc):
+    p = configs.dendrite_k93_params(n=nx, ny=ny, tile=tile, mode=mode, history_cap=128, bc=bc)
+    seeds = [(nx // 2, ny // 3), (nx // 8, ny // 8)] if nx > 100 else [(nx // 2, ny // 2)]
+    fields = list(configs.dendrite_k93_ic(nx, ny, seeds=seeds))
+    a = run(ctx, p, fields, 1)
+    same(a, run(ctx, p, fields, 0))
+    if mode == abi.MODE_DBA and nx > 200:
+        awake = a[-1][1]
+        assert 0 < awake[0].sum() < awake[0].size and not np.array_equal(awake[0], awake[1])
 
 
 def test_resident_two_contexts(ctx):

@@ -812,12 +812,14 @@ void launch_dense(const Group* g, hipStream_t s, int first, int step) {
 void launch_finalize(const Group* g, hipStream_t s, int rotate, int step, bool last) {
     SegPart* parts = parts_of(g, step);
     const SegPart* pend = g->fold && rotate && step > 0 ? parts_of(g, step - 1) : nullptr;
-    hipLaunchKernelGGL(finalize_kernel, dim3((unsigned)g->nseg), dim3(kFinNT), 0, s, g->d_insts, g->d_segs,
-                       g->nseg, parts, g->d_counts, g->d_offsets, rotate, g->ids.size() == 1 ? 1 : 0, pend);
+    const int n_inst = (int)g->ids.size();
+    const unsigned per_inst = (unsigned)((n_inst + kFinNT / 64 - 1) / (kFinNT / 64));  // workgroups, a wave per instance
+    hipLaunchKernelGGL(finalize_kernel, dim3((unsigned)g->nseg + (pend ? per_inst : 0u)), dim3(kFinNT), 0, s,
+                       g->d_insts, g->d_segs, g->nseg, parts, g->d_counts, g->d_offsets, rotate, n_inst == 1 ? 1 : 0,
+                       pend, g->d_isegs, n_inst);
     if (g->nseg > 1 && (!g->fold || last)) {
         // workgroup 0 scans the segment counts; the others reduce 16 instances each
-        const int n_inst = (int)g->ids.size();
-        const unsigned wgs = 1u + (unsigned)((n_inst + kFinNT / 64 - 1) / (kFinNT / 64));
+        const unsigned wgs = 1u + per_inst;
         hipLaunchKernelGGL(finalize_merge_kernel, dim3(wgs), dim3(kFinNT), 0, s, g->d_insts, g->nseg, g->d_isegs,
                            n_inst, parts, g->d_counts, g->d_offsets, rotate);
     }

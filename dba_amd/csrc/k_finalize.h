@@ -35,28 +35,6 @@ __device__ __forceinline__ int64_t tile_cells(CInst& I, int t) {
     return (int64_t)wx * wy * wz;
 }
 
-// Awake flag of tile t for the next step: OR of the detector bytes over the
-// tile and its neighbours (kind 0: faces; kind 1: 3x3 in-plane + z faces),
-// wrapping where the instance is periodic and clamping elsewhere. A neighbour
-// clamped away reads the tile itself (or, for an in-plane corner, the edge
-// neighbour that exists), which the OR already holds: no load waits on a branch.
-__device__ __forceinline__ int dilated3d(CInst& I, const gu8* N, int t, int kind) {
-    const int ntx = I.ntx, nty = I.nty, ntz = I.ntz, nxy = ntx * nty;
-    const int ti = t % ntx, tj = (t / ntx) % nty, tk = t / nxy;
-    auto nb = [](int i, int d, int n, int bc) {
-        const int j = i + d;
-        return (j >= 0 && j < n) ? j : (bc == 0 ? (j + n) % n : i);
-    };
-    const int xm = nb(ti, -1, ntx, I.bc_x), xp = nb(ti, 1, ntx, I.bc_x);
-    const int ym = nb(tj, -1, nty, I.bc_y) * ntx, yp = nb(tj, 1, nty, I.bc_y) * ntx;
-    const int zm = nb(tk, -1, ntz, I.bc_z) * nxy, zp = nb(tk, 1, ntz, I.bc_z) * nxy;
-    const int row = tj * ntx, pl = tk * nxy;
-    int r = N[t] | N[xm + row + pl] | N[xp + row + pl] | N[ti + ym + pl] | N[ti + yp + pl] | N[ti + row + zm] |
-            N[ti + row + zp];
-    if (kind == 1) r |= N[xm + ym + pl] | N[xp + ym + pl] | N[xm + yp + pl] | N[xp + yp + pl];
-    return r != 0;
-}
-
 // 2D tile grid: neighbour columns/rows resolved once (-1 = clamped away).
 struct Nb2 {
     int xm, xp, ym, yp;  // tile-grid column / row indices
@@ -71,6 +49,8 @@ __device__ __forceinline__ Nb2 nb2_of(int ti, int tj, int ntx, int nty, int bcx,
     return n;
 }
 
+// Awake flag of tile (ti, tj) for the next step: OR of the detector bytes over the
+// tile and its neighbours (kind 0: faces; kind 1: 3x3).
 __device__ __forceinline__ int dilated2d(const gu8* N, int ti, int tj, int ntx, const Nb2& n, int kind) {
     // A missing neighbour (zero-flux or wall boundary) reads the tile itself
     // instead, which the OR already holds (a missing corner falls back to the
@@ -138,244 +118,294 @@ __device__ __forceinline__ void finish_instance(CInst& J, int64_t listlen, unsig
 __device__ __forceinline__ void merge_instance(CInst& J, int first, int count, const SegPart* __restrict__ parts,
                                                const int32_t* __restrict__ counts, int rotate) {
     const int lane = threadIdx.x & 63;
-    // the instance's scalars and counters, loaded ahead of the reduction
-    double sc[16];
-    int64_t step = 0, upd = 0, len = 0;
-    if (lane == 0) {
-        for (int kk = 0; kk < 16; kk++) sc[kk] = J.scal[kk];
-        step = J.ctr[0];
-        upd = J.ctr[1];
-        len = J.ctr[2];
-    }
-    int64_t ll = 0;
-    unsigned long long q0 = 0, q1 = 0, qc = 0;
+    // the descriptor's fields in one batch, then the instance's scalars and counters
+    // with the partials: no load waits for another
+    const int ncs = J.ncons, model = J.model, dt_mode = J.dt_mode, nsets = J.nsets, hist_cap = J.hist_cap;
+    gdouble* scal = J.scal;
+    gi64* ctr = J.ctr;
+    gi32* hist = J.hist;
+    const double ntotal = J.ntotal, cfl_n = J.cfl, dx = J.dx;
+    asm volatile("" ::"s"(ncs), "s"(model), "s"(dt_mode), "s"(nsets), "s"(hist_cap), "s"(scal), "s"(ctr), "s"(hist),
+                 "s"(ntotal), "s"(cfl_n), "s"(dx));
+    const bool cfl = rotate && model == 5 && dt_mode == 1;
+    double sc[16] = {0.0};
+    sc[1] = scal[1];
+    sc[2] = scal[2];
+#pragma unroll
+    for (int f = 0; f < kMaxFields; f++) sc[8 + f] = scal[8 + f];
+    const int64_t step = ctr[0], upd = ctr[1], len = ctr[2];
+    int ll = 0;
+    unsigned long long q01 = 0, qc = 0;  // tiles that ran set 0, set 1 << 32; their cells
     double cs[kMaxFields] = {0.0, 0.0, 0.0, 0.0};
     double vm = 0.0;
-    const int ncs = J.ncons;
+#pragma unroll 2
     for (int q = first + lane; q < first + count; q += 64) {
         if (counts) ll += counts[q];
         if (rotate) {
-            q0 += parts[q].c0;
-            q1 += parts[q].c1;
+            q01 += parts[q].c0 | parts[q].c1 << 32;
             qc += parts[q].cells;
-            for (int f = 0; f < ncs; f++) cs[f] += parts[q].csum[f];
-            vm = fmax(vm, parts[q].vmax);
+#pragma unroll
+            for (int f = 0; f < kMaxFields; f++)
+                if (f < ncs) cs[f] += parts[q].csum[f];
+            if (cfl) vm = fmax(vm, parts[q].vmax);
         }
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
         ll += __shfl_down(ll, off, 64);
-        q0 += __shfl_down(q0, off, 64);
-        q1 += __shfl_down(q1, off, 64);
+        q01 += __shfl_down(q01, off, 64);
         qc += __shfl_down(qc, off, 64);
-        for (int f = 0; f < kMaxFields; f++) cs[f] += __shfl_down(cs[f], off, 64);
-        vm = fmax(vm, __shfl_down(vm, off, 64));
     }
-    if (lane == 0) finish_instance(J, counts ? ll : len, q0, q1, qc, cs, vm, step, upd, sc, rotate);
+#pragma unroll
+    for (int f = 0; f < kMaxFields; f++)
+        if (f < ncs) cs[f] = wave_sum_down(cs[f]);
+    if (cfl) vm = wave_max_down(vm);
+    if (lane == 0)
+        finish_instance(J, counts ? (int64_t)ll : len, q01 & 0xffffffffull, q01 >> 32, qc, cs, vm, step, upd, sc, rotate);
 }
 
 // LDS of the finalize body.
 struct FinLds {
-    uint8_t s_pb[2][kSegTiles];     // per tile: parity the next step sees
-    uint8_t s_ab[2][kSegTiles];     // per tile: awake in the next step
-    int s_wcnt[kSegWords];          // per 64-tile word: tiles in the next worklist
-    unsigned long long s_wran[kSegWords][3];  // per word: tiles that ran (set 0, set 1), their cells
-    double sd[kFinNT / 64 + 1];
-    double s_cs[kMaxFields];
-    double s_scal[16];
-    int64_t s_step;
-    int64_t s_upd;
+    uint8_t bits[kSegTiles];        // per tile: awake in the next step (bits 0, 1: sets), parity it sees (2, 3)
+    alignas(16) int listed[kSegWords];  // per 64-tile word: tiles in the next worklist
+    alignas(16) uint32_t ran[kSegWords];    // ... tiles that ran: set 0, set 1 << 16
+    alignas(16) uint32_t cells[kSegWords];  // ... and their cells
+    double csum[kMaxFields][kSegWords];     // ... conserved change sums
+    double vmax[kSegWords];                 // ... KH wave speed
 };
 
-// One thread per tile of the segment, one wave per 64-tile bitmap word, so the
-// whole bookkeeping needs a single workgroup barrier (plus the reductions of
-// the conserved and CFL variants).
+// One thread per tile of the segment, one wave per 64-tile bitmap word, one
+// workgroup barrier.
+//
+// What bounds it: the chain of dependent loads (a segment has 30 KB of state). The
+// descriptor's fields come in one batch of scalar loads, then every vector load of
+// both sets goes out before the first is waited for; past the barrier everything is
+// read from LDS at fixed addresses, and folded merges have a workgroup of their own.
+// With loads waited for branch by branch and LDS loops of the segment's length, us per
+// launch before -> now: 16 dendrites in 30 segments 8.5 -> 5.4, a 256^3 dendrite (256
+// segments) 7.7 -> 5.8, KH 2048^2 (16 segments) 7.9 -> 5.3, 96 x 80 x 64
+// conserved Model B 7.3 -> 5.0.
 template <int NT>
 __device__ __forceinline__ void finalize_body(const Inst* __restrict__ insts, const Seg* __restrict__ segs,
                                               int segi, int nseg, SegPart* __restrict__ parts,
                                               int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
-                                              int rotate, int one_inst, const SegPart* __restrict__ pend,
-                                              FinLds& F) {
+                                              int rotate, int one_inst, FinLds& F) {
     static_assert(NT == kSegTiles, "one thread per tile of a segment");
-    auto& s_pb = F.s_pb;
-    auto& s_ab = F.s_ab;
-    auto& s_wcnt = F.s_wcnt;
-    auto& s_wran = F.s_wran;
-    auto& sd = F.sd;
-    auto& s_cs = F.s_cs;
-    auto& s_scal = F.s_scal;
-    auto& s_step = F.s_step;
-    auto& s_upd = F.s_upd;
-
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     // one segment: instance 0, all of its tiles (no dependent load of the segment table)
     // one instance: segment segi holds its tiles from segi kSegTiles on, so the
     // segment table is not read (its load would come before the descriptor's)
-    const bool one = nseg == 1 || one_inst;
-    const int inst = one ? 0 : __builtin_amdgcn_readfirstlane(segs[segi].inst);
+    const bool solo = nseg == 1, one = solo || one_inst;
+    int inst = 0, t0 = solo ? 0 : segi * kSegTiles, seg_n = 0;
+    if (!one) {
+        const Seg sg = segs[segi];
+        inst = __builtin_amdgcn_readfirstlane(sg.inst);
+        t0 = __builtin_amdgcn_readfirstlane(sg.tile0);
+        seg_n = __builtin_amdgcn_readfirstlane(sg.ntile);
+    }
     CInst& I = ((CInst*)insts)[inst];
-    const int t0 = nseg == 1 ? 0 : (one_inst ? segi * kSegTiles : __builtin_amdgcn_readfirstlane(segs[segi].tile0));
-    const int nts = nseg == 1 ? I.nt
-                              : (one_inst ? min(kSegTiles, I.nt - t0)
-                                          : __builtin_amdgcn_readfirstlane(segs[segi].ntile));
+    const int nt = I.nt, ntx = I.ntx, nty = I.nty, ntz = I.ntz, bcx = I.bc_x, bcy = I.bc_y, bcz = I.bc_z;
+    const int mode = I.mode, nsets = I.nsets, model = I.model, ncons = I.ncons, dt_mode = I.dt_mode;
+    const int tile_n = I.tx * I.ty * I.tz, full_tiles = I.full_tiles;
+    gu64 *cur0p = I.a_cur[0], *cur1p = I.a_cur[1], *par0p = I.par[0], *par1p = I.par[1];
+    const gu8 *nf0 = I.nflag[0], *nf1 = I.nflag[1];
+    const gdouble *tpart = I.tpart, *tspeed = I.tspeed;
+    gi32* seg = I.seg;
+    gu64* nbrec = I.nbrec;
+    asm volatile("" ::"s"(nt), "s"(ntx), "s"(nty), "s"(ntz), "s"(bcx), "s"(bcy), "s"(bcz), "s"(mode), "s"(nsets),
+                 "s"(model), "s"(ncons), "s"(dt_mode), "s"(tile_n), "s"(full_tiles), "s"(cur0p), "s"(cur1p),
+                 "s"(par0p), "s"(par1p), "s"(nf0), "s"(nf1), "s"(tpart), "s"(tspeed), "s"(seg), "s"(nbrec));
+    const int nts = solo ? nt : (one_inst ? min(kSegTiles, nt - t0) : seg_n);
     const int w0 = t0 >> 6, nws = (nts + 63) >> 6;
-    const bool regular = I.mode == 0;
-    const int nsets = I.nsets;
-    const int nt = I.nt;
-    const int kind = I.model == 5 ? 1 : 0;
-    const bool solo = nseg == 1;
-    const int k = tid, t = t0 + k;
-    const bool valid = k < nts;
+    const bool regular = mode == 0, dilate = rotate && !regular, cfl = rotate && model == 5 && dt_mode == 1;
+    const int t = t0 + tid, tc = tid < nts ? t : t0;
+    const bool valid = tid < nts;
     const bool wvalid = wid < nws;  // this wave's word exists
 
-    // ---- prologue: every independent global load, issued together
-    uint64_t cur0 = 0ull, cur1 = 0ull, par0 = 0ull, par1 = 0ull;
-    if (wvalid) {
-        cur0 = regular ? full_word(w0 + wid, nt) : I.a_cur[0][w0 + wid];
-        par0 = I.par[0][w0 + wid];
+    // ---- every global load, issued together (past the segment: tile t0's, not used)
+    const int wc = w0 + (wvalid ? wid : 0);
+    uint64_t cur0 = regular ? full_word(wc, nt) : cur0p[wc], par0 = par0p[wc], cur1 = 0ull, par1 = 0ull;
+    if (nsets > 1) {
+        cur1 = regular ? full_word(wc, nt) : cur1p[wc];
+        par1 = par1p[wc];
+    }
+    const int q = tc / ntx, ti = tc - q * ntx, tk = ntz == 1 ? 0 : q / nty, tj = q - tk * nty;
+    // neighbour columns, rows and planes; one clamped away is the tile's own
+    const int xm = ti > 0 ? ti - 1 : (bcx == 0 ? ntx - 1 : ti), xp = ti < ntx - 1 ? ti + 1 : (bcx == 0 ? 0 : ti);
+    const int ym = tj > 0 ? tj - 1 : (bcy == 0 ? nty - 1 : tj), yp = tj < nty - 1 ? tj + 1 : (bcy == 0 ? 0 : tj);
+    int f0[11], f1[7];
+#pragma unroll
+    for (int k = 0; k < 11; k++) f0[k] = 0;
+#pragma unroll
+    for (int k = 0; k < 7; k++) f1[k] = 0;
+    if (dilate) {
+        const int nxy = ntx * nty, pl = tk * nxy, row = tj * ntx + pl, rm = ym * ntx + pl, rp = yp * ntx + pl;
+        const int o[5] = {tc, xm + row, xp + row, ti + rm, ti + rp};
+        const int zm = tk > 0 ? tk - 1 : (bcz == 0 ? ntz - 1 : tk), zp = tk < ntz - 1 ? tk + 1 : (bcz == 0 ? 0 : tk);
+        const int om = zm * nxy + tj * ntx + ti, op = zp * nxy + tj * ntx + ti;
+#pragma unroll
+        for (int k = 0; k < 5; k++) f0[k] = nf0[o[k]];
+        if (ntz > 1) {
+            f0[5] = nf0[om];
+            f0[6] = nf0[op];
+        }
+        if (model == 5) {  // 3x3 in the plane
+            f0[7] = nf0[xm + rm];
+            f0[8] = nf0[xp + rm];
+            f0[9] = nf0[xm + rp];
+            f0[10] = nf0[xp + rp];
+        }
         if (nsets > 1) {
-            cur1 = regular ? full_word(w0 + wid, nt) : I.a_cur[1][w0 + wid];
-            par1 = I.par[1][w0 + wid];
+#pragma unroll
+            for (int k = 0; k < 5; k++) f1[k] = nf1[o[k]];
+            if (ntz > 1) {
+                f1[5] = nf1[om];
+                f1[6] = nf1[op];
+            }
         }
     }
-    int a0 = 0, a1 = 0;
-    if (valid && rotate && !regular) {
-        if (I.ntz == 1) {
-            const int ntx = I.ntx;
-            const int tj = t / ntx, ti = t - tj * ntx;
-            const Nb2 n = nb2_of(ti, tj, ntx, I.nty, I.bc_x, I.bc_y);
-            a0 = dilated2d(I.nflag[0], ti, tj, ntx, n, kind);
-            if (nsets > 1) a1 = dilated2d(I.nflag[1], ti, tj, ntx, n, kind);
-        } else {
-            a0 = dilated3d(I, I.nflag[0], t, kind);
-            if (nsets > 1) a1 = dilated3d(I, I.nflag[1], t, kind);
-        }
+    double part[kMaxFields] = {0.0, 0.0, 0.0, 0.0};
+    if (rotate)
+#pragma unroll
+        for (int f = 0; f < kMaxFields; f++)
+            if (f < ncons) part[f] = tpart[(int64_t)f * nt + tc];
+    double fresh = 0.0, stale = 0.0;
+    if (cfl) {
+        fresh = tspeed[tc];
+        stale = tspeed[nt + tc];
     }
-    if (solo && tid < 16) s_scal[tid] = I.scal[tid];
-    if (solo && tid == 16) s_step = I.ctr[0];
-    if (solo && tid == 17) s_upd = I.ctr[1];
+
+    double sc[16] = {0.0};
+    int64_t step = 0, upd = 0;
+    if (solo) {  // what finish_instance needs
+        sc[1] = I.scal[1];
+        sc[2] = I.scal[2];
+#pragma unroll
+        for (int f = 0; f < kMaxFields; f++) sc[8 + f] = I.scal[8 + f];
+        step = I.ctr[0];
+        upd = I.ctr[1];
+    }
 
     // ---- this tile: ran in the executed step?  awake in the next?  parity next?
+    if (!wvalid) cur0 = cur1 = par0 = par1 = 0ull;
     const int ran0 = (int)((cur0 >> lane) & 1ull), ran1 = (int)((cur1 >> lane) & 1ull);
-    int b0, b1;
-    if (rotate && !regular) {
-        b0 = a0;
-        b1 = a1;
-    } else {
-        // regular: every tile every step; rebuild (rotate = 0): the current sets
-        b0 = valid && ran0;
-        b1 = valid && ran1;
+    int b0 = ran0, b1 = ran1;  // regular: every tile every step; rebuild (rotate = 0): the current sets
+    if (dilate) {
+        b0 = (f0[0] | f0[1] | f0[2] | f0[3] | f0[4] | f0[5] | f0[6] | f0[7] | f0[8] | f0[9] | f0[10]) != 0;
+        b1 = (f1[0] | f1[1] | f1[2] | f1[3] | f1[4] | f1[5] | f1[6]) != 0;
     }
+    if (!valid) b0 = b1 = 0;
     const uint64_t pn0 = rotate ? (par0 ^ cur0) : par0;
     const uint64_t pn1 = rotate ? (par1 ^ cur1) : par1;
     const uint64_t nw0 = __ballot(b0);
     const uint64_t nw1 = __ballot(b1);
     const uint64_t uni = nw0 | nw1;
-    s_ab[0][k] = (uint8_t)b0;
-    s_ab[1][k] = (uint8_t)b1;
-    s_pb[0][k] = (uint8_t)((pn0 >> lane) & 1ull);
-    s_pb[1][k] = (uint8_t)((pn1 >> lane) & 1ull);
+    F.bits[tid] = (uint8_t)(b0 | b1 << 1 | (int)((pn0 >> lane) & 1ull) << 2 | (int)((pn1 >> lane) & 1ull) << 3);
     if (rotate && wvalid && lane == 0) {
-        I.par[0][w0 + wid] = pn0;
-        if (nsets > 1) I.par[1][w0 + wid] = pn1;
+        par0p[w0 + wid] = pn0;
+        if (nsets > 1) par1p[w0 + wid] = pn1;
         if (!regular) {
-            I.a_cur[0][w0 + wid] = nw0;
-            if (nsets > 1) I.a_cur[1][w0 + wid] = nw1;
+            cur0p[w0 + wid] = nw0;
+            if (nsets > 1) cur1p[w0 + wid] = nw1;
         }
     }
     // per-word statistics of the executed step
     // field-set updates: set 0's fields over the tiles that ran it; the second
     // set's field (dendrite T) over the tiles that ran either set, since a
     // p-awake tile writes T too
-    unsigned long long cells = 0ull;
-    if (rotate && valid && (ran0 | ran1)) {
-        const unsigned long long tc = I.full_tiles ? (unsigned long long)(I.tx * I.ty * I.tz)
-                                                   : (unsigned long long)tile_cells(I, t);
-        cells = tc * (unsigned long long)(nsets > 1 ? 1 + (ran0 ? 1 : 0) : 1);
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) cells += __shfl_down(cells, off, 64);
-    if (lane == 0) {
-        s_wcnt[wid] = __popcll(uni);
-        s_wran[wid][0] = (unsigned long long)__popcll(cur0);
-        s_wran[wid][1] = (unsigned long long)__popcll(cur1);
-        s_wran[wid][2] = cells;
-    }
-    // conserved change sums of the tiles that ran (sleeping tiles contribute 0)
+    uint32_t cells = 0;
     if (rotate) {
-        for (int f = 0; f < I.ncons; f++) {
-            const double csum = (valid && ran0) ? I.tpart[(int64_t)f * nt + t] : 0.0;
-            const double tot = block_sum<NT>(csum, sd);
-            if (tid == 0) s_cs[f] = tot;
+        if (full_tiles) {
+            cells = (uint32_t)tile_n * (uint32_t)(__popcll(cur0 | cur1) + (nsets > 1 ? __popcll(cur0) : 0));
+        } else {
+            if (valid && (ran0 | ran1)) cells = (uint32_t)tile_cells(I, t) * (uint32_t)(nsets > 1 ? 1 + ran0 : 1);
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) cells += __shfl_down(cells, off, 64);
         }
     }
+    if (lane == 0) {
+        F.listed[wid] = __popcll(uni);
+        F.ran[wid] = (uint32_t)__popcll(cur0) | (uint32_t)__popcll(cur1) << 16;
+        F.cells[wid] = cells;
+    }
+    // conserved change sums of the tiles that ran (sleeping tiles contribute 0):
+    // block_sum's tree, its words added in order below
+    if (rotate)
+#pragma unroll
+        for (int f = 0; f < kMaxFields; f++)
+            if (f < ncons) {
+                const double s = wave_sum_down(valid && ran0 ? part[f] : 0.0);
+                if (lane == 0) F.csum[f][wid] = s;
+            }
     // KH: max wave speed the next step's CFL sees (fresh for awake tiles, stale otherwise)
-    double vmax = 0.0;
-    if (rotate && I.model == 5 && I.dt_mode == 1) {
-        if (valid) vmax = b0 ? I.tspeed[t] : I.tspeed[nt + t];
-        vmax = block_max<NT>(vmax, sd);
+    if (cfl) {
+        const double v = wave_max_down(valid ? (b0 ? fresh : stale) : 0.0);
+        if (lane == 0) F.vmax[wid] = v;
     }
     __syncthreads();
 
     // ---- compaction of the union set (ascending tiles) and the neighbour records
     int base = 0, listlen = 0;
-    for (int w = 0; w < nws; w++) {
-        const int c = s_wcnt[w];
+#pragma unroll
+    for (int w = 0; w < kSegWords; w++) {
+        const int c = F.listed[w];
         if (w < wid) base += c;
         listlen += c;
     }
     if ((uni >> lane) & 1ull) {
         const int pos = t0 + base + __popcll(uni & ((1ull << lane) - 1ull));
-        I.seg[pos] = t;
-        if (I.ntz == 1) {
+        seg[pos] = t;
+        if (ntz == 1) {
             // resolved here when all nine owners are in this segment
             uint64_t rec = kRecValid;
-            const int tj = t / I.ntx, ti = t - tj * I.ntx;
+            bool all = true;
+#pragma unroll
             for (int d = 0; d < 9; d++) {
-                const int o = nb_owner2d(I, ti, tj, d) - t0;
-                if (o < 0 || o >= nts) {
-                    rec = 0ull;
-                    break;
-                }
-                for (int s2 = 0; s2 < nsets; s2++) {
-                    rec |= (uint64_t)s_pb[s2][o] << (s2 * 18 + d);
-                    rec |= (uint64_t)s_ab[s2][o] << (s2 * 18 + 9 + d);
-                }
+                const int o = (d % 3 == 0 ? xm : (d % 3 == 1 ? ti : xp)) +
+                              (d / 3 == 0 ? ym : (d / 3 == 1 ? tj : yp)) * ntx - t0;
+                const bool here = o >= 0 && o < nts;
+                all = all && here;
+                const uint32_t v = F.bits[here ? o : 0];
+                rec |= (uint64_t)((v >> 2) & 1u) << d | (uint64_t)(v & 1u) << (9 + d) |
+                       (uint64_t)(v >> 3) << (18 + d) | (uint64_t)((v >> 1) & 1u) << (27 + d);
             }
-            I.nbrec[pos] = rec;
+            nbrec[pos] = all ? rec : 0ull;
         }
     }
-    unsigned long long c0 = 0, c1 = 0, ccells = 0;
-    if (tid == 0) {
-        for (int w = 0; w < nws; w++) {
-            c0 += s_wran[w][0];
-            c1 += s_wran[w][1];
-            ccells += s_wran[w][2];
-        }
-    }
+    if (tid != 0) return;
 
-    // ---- per-instance reductions and merged offsets
+    // ---- the segment's sums
+    uint32_t ran = 0, ncell = 0;
+#pragma unroll
+    for (int w = 0; w < kSegWords; w++) {
+        ran += F.ran[w];  // (at most 1024 of each set: no carry)
+        ncell += F.cells[w];
+    }
+    double cs[kMaxFields] = {0.0, 0.0, 0.0, 0.0};
+    if (rotate)
+#pragma unroll
+        for (int f = 0; f < kMaxFields; f++)
+            if (f < ncons)
+                for (int w = 0; w < kSegWords; w++) cs[f] += F.csum[f][w];
+    double vmax = 0.0;
+    if (cfl) {
+        vmax = F.vmax[0];
+        for (int w = 1; w < kSegWords; w++) vmax = fmax(vmax, F.vmax[w]);
+    }
+    const unsigned long long c0 = ran & 0xffffu, c1 = ran >> 16;
     if (solo) {
-        if (tid == 0) {
-            double cs[kMaxFields] = {s_cs[0], s_cs[1], s_cs[2], s_cs[3]};
-            finish_instance(I, listlen, c0, c1, ccells, cs, vmax, s_step, s_upd, s_scal, rotate);
-            offsets[0] = 0;
-            offsets[1] = listlen;
-        }
+        finish_instance(I, listlen, c0, c1, ncell, cs, vmax, step, upd, sc, rotate);
+        offsets[0] = 0;
+        offsets[1] = listlen;
         return;
     }
-    // folded merges: the instance sums of the step before this one, by the last wave
-    // of the instance's first segment
-    if (pend && wid == NT / 64 - 1 && t0 == 0) merge_instance(I, segi, (nt + kSegTiles - 1) / kSegTiles, pend, nullptr, 1);
-    if (tid == 0) {
-        counts[segi] = listlen;
-        if (rotate) {
-            parts[segi].c0 = c0;
-            parts[segi].c1 = c1;
-            parts[segi].cells = ccells;
-            for (int f = 0; f < kMaxFields; f++) parts[segi].csum[f] = f < I.ncons ? s_cs[f] : 0.0;
-            parts[segi].vmax = vmax;
-        }
+    counts[segi] = listlen;
+    if (rotate) {
+        parts[segi].c0 = c0;
+        parts[segi].c1 = c1;
+        parts[segi].cells = ncell;
+        for (int f = 0; f < kMaxFields; f++) parts[segi].csum[f] = cs[f];
+        parts[segi].vmax = vmax;
     }
 }
 
@@ -425,14 +455,24 @@ __device__ __forceinline__ void finalize_merge_body(const Inst* __restrict__ ins
 }
 
 
+// Workgroups past the segments (folded merges): the instance sums of the step
+// before this one, a wave per instance.
 __global__ __launch_bounds__(kFinNT) void finalize_kernel(const Inst* __restrict__ insts,
                                                           const Seg* __restrict__ segs, int nseg,
                                                           SegPart* __restrict__ parts,
                                                           int32_t* __restrict__ counts,
                                                           int32_t* __restrict__ offsets, int rotate,
-                                                          int one_inst, const SegPart* __restrict__ pend) {
+                                                          int one_inst, const SegPart* __restrict__ pend,
+                                                          const InstSegs* __restrict__ isegs, int n_inst) {
     __shared__ FinLds F;
-    finalize_body<kFinNT>(insts, segs, blockIdx.x, nseg, parts, counts, offsets, rotate, one_inst, pend, F);
+    if ((int)blockIdx.x >= nseg) {
+        const int i = ((int)blockIdx.x - nseg) * (kFinNT / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        if (i >= n_inst) return;
+        const InstSegs r = n_inst == 1 ? InstSegs{0, nseg} : isegs[i];
+        merge_instance(((CInst*)insts)[i], r.first, r.count, pend, nullptr, 1);
+        return;
+    }
+    finalize_body<kFinNT>(insts, segs, blockIdx.x, nseg, parts, counts, offsets, rotate, one_inst, F);
 }
 
 __global__ __launch_bounds__(kFinNT) void finalize_merge_kernel(const Inst* __restrict__ insts, int nseg,

@@ -63,6 +63,7 @@ struct Inst {
     double ntotal;               // number of cells (conserved mean)
     // derived constants, computed on the host with the same expressions as the oracle
     double invdx2, inv6dx2, inv2dx, dt_tau, alpha_pi, cos_jt0, sin_jt0, k_epsp;
+    double k94_f0, k94_f1, k94_f2, k94_f3;  // K94: 1 / (2 dx), 1 / dx / dx, -alpha / 3.14159, 1 / tau
     double mb_cx, mb_cy, mb_cz, mb_lk;  // Model B: -1 + 1/r_x.., log(k_eq)/r_z
     double mb_irx, mb_iry, mb_irz, mb_hiomz;  // ... 1/r_x.., 1 / (2 (1 - z_crit))
     // model constants
@@ -169,6 +170,10 @@ __device__ __forceinline__ double wave_sum_down(double v) {
     v += dpp_row_down<1>(v);
     return v;
 }
+
+// LDS written by one lane and read by another of the same wave, in a kernel whose
+// waves do not wait for each other.
+__device__ __forceinline__ void wave_lds_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // Deterministic workgroup sum: per-wave shift reduction in a fixed order, then
 // wave totals added in wave order by thread 0.
@@ -533,6 +538,7 @@ __device__ __forceinline__ bool next_item(const WorkList& w, const Fold& F, int 
 // single-instance list, the first item of a full round is read before the list
 // length arrives (it is the same item either way), so both loads overlap.
 struct WorkCursor {
+    int b, G;       // this taker's index and their number (workgroups; waves in kernels that deal to waves)
     int base;       // first item of the next round
     int spec_item;  // item whose entry was read ahead (-1: none)
     int spec_t;
@@ -547,12 +553,13 @@ __device__ __forceinline__ int xcd_deal(int b, int G, int base, int cnt) {
     return item < base + cnt ? item : -1;
 }
 
-__device__ __forceinline__ void work_begin(const WorkList& w, WorkCursor& c, bool want_rec) {
+__device__ __forceinline__ void work_begin(const WorkList& w, WorkCursor& c, bool want_rec, int b, int G) {
+    c.b = b;
+    c.G = G;
     c.base = 0;
     c.spec_item = -1;
     if (w.solo_nt > 0) {
-        const int G = gridDim.x;
-        const int item = xcd_deal(blockIdx.x, G, 0, G);  // the item of a full first round
+        const int item = xcd_deal(b, G, 0, G);  // the item of a full first round
         if (item >= 0 && item < w.solo_nt) {
             c.spec_item = item;
             c.spec_t = w.solo_seg[item];
@@ -561,12 +568,16 @@ __device__ __forceinline__ void work_begin(const WorkList& w, WorkCursor& c, boo
     }
 }
 
+__device__ __forceinline__ void work_begin(const WorkList& w, WorkCursor& c, bool want_rec) {
+    work_begin(w, c, want_rec, blockIdx.x, gridDim.x);
+}
+
 template <bool FOLD = true>
 __device__ __forceinline__ bool work_next(const WorkList& w, const Fold& F, WorkCursor& c, int total,
                                           CInst** I, int* t, uint64_t* rec, bool want_rec = true) {
-    const int G = gridDim.x;
+    const int G = c.G;
     while (c.base < total) {
-        const int item = xcd_deal(blockIdx.x, G, c.base, min(G, total - c.base));
+        const int item = xcd_deal(c.b, G, c.base, min(G, total - c.base));
         c.base += G;
         if (item < 0) continue;
         if (item == c.spec_item) {

@@ -197,6 +197,10 @@ void derive_constants(const dba_params& p, Inst& h) {
         h.mb_cz = -1.0 + 1.0 / p.r_z;
         h.mb_lk = std::log(p.k_eq) / p.r_z;
     }
+    h.k94_f0 = 1. / (2 * p.dx);
+    h.k94_f1 = 1. / p.dx / p.dx;
+    h.k94_f2 = -p.alpha / 3.14159;
+    h.k94_f3 = 1. / p.tau;
     h.mb_irx = 1.0 / p.r_x;
     h.mb_iry = 1.0 / p.r_y;
     h.mb_irz = 1.0 / p.r_z;
@@ -541,8 +545,11 @@ dba_status get_group(dba_ctx* ctx, const std::vector<int>& ids, Group** out) {
         }
     }
     // Model B: 65536 workgroups (4 blocks each on a fully awake 256^3 field)
-    // measured faster than 16384 or 3072 with longer pipelines per wave
-    int64_t cap = g->model == DBA_MODEL_MODELB ? 65536 : (g->model == DBA_MODEL_DENDRITE_K94 ? 16384 : 4096);
+    // measured faster than 16384 or 3072 with longer pipelines per wave. K94: the
+    // waves that are resident at once (5 on each SIMD by registers), since a list is
+    // mostly shorter and the dispatch of further ones costs: 256^3 dendrite, us per
+    // step with 16, 20, 32, 64, 128 waves per CU: 22.3, 21.7, 22.4, 23.9, 27.0
+    int64_t cap = g->model == DBA_MODEL_MODELB ? 65536 : (g->model == DBA_MODEL_DENDRITE_K94 ? 20 * ctx->n_cu : 4096);
     g->grid = (int)std::max<int64_t>(1, std::min<int64_t>(g->total_tiles, cap));
     // Model B column march (modelb_march_kernel): one 3D instance, steps with at
     // least a quarter of the blocks awake. DBA_MODELB_SUPERBLOCKS=0 turns it off and
@@ -702,10 +709,12 @@ void launch_step(const Group* g, hipStream_t s) {
                 hipLaunchKernelGGL((modelb_update_kernel<4, 1>), grid, block, 0, s, wl_of(g), from);
             }
         } else {
+            // a wave per block; a multiple of 8 workgroups, so every XCD has as many
+            const unsigned wgs = ((unsigned)(g->grid + 8 * kK94Waves - 1) / (8 * kK94Waves)) * 8;
             if (g->tile_z == 4)
-                hipLaunchKernelGGL((k94_step_kernel<4, 4>), grid, block, 0, s, wl_of(g));
+                hipLaunchKernelGGL((k94_step_kernel<4, 4>), dim3(wgs), dim3(64 * kK94Waves), 0, s, wl_of(g));
             else
-                hipLaunchKernelGGL((k94_step_kernel<4, 1>), grid, block, 0, s, wl_of(g));
+                hipLaunchKernelGGL((k94_step_kernel<4, 1>), dim3(wgs), dim3(64 * kK94Waves), 0, s, wl_of(g));
         }
         return;
     }

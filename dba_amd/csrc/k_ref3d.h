@@ -827,16 +827,23 @@ __global__ __launch_bounds__(MbMarch::NT) __attribute__((amdgpu_waves_per_eu(CON
         const double X = df[0], Y = df[1], Z = df[2];
         if (up) {
             if (wakes) {
-                // one logarithm at a time: together they spill
                 const double B = 1.0 - X - Y - Z;
-                const double com = mb_shared(I, X, Y, Z, log_f64(B));
-                __builtin_amdgcn_sched_barrier(0);
-                df[0] = mb_mu_x(I, Y, Z, B, com, log_f64(X), lap[0]);
-                __builtin_amdgcn_sched_barrier(0);
-                df[1] = mb_mu_y(I, X, Z, B, com, log_f64(Y), lap[1]);
-                __builtin_amdgcn_sched_barrier(0);
-                df[2] = mb_mu_z(I, X, Y, B, com, log_f64(Z), lap[2], phi);
-                __builtin_amdgcn_sched_barrier(0);
+                if (X > 0.0 && Y > 0.0 && Z > 0.0 && B > 0.0) {  // (so all of them are below 1)
+                    // one logarithm at a time: together they spill
+                    const double com = mb_shared(I, X, Y, Z, log_positive(B));
+                    __builtin_amdgcn_sched_barrier(0);
+                    df[0] = mb_mu_x(I, Y, Z, B, com, log_positive(X), lap[0]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    df[1] = mb_mu_y(I, X, Z, B, com, log_positive(Y), lap[1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    df[2] = mb_mu_z(I, X, Y, B, com, log_positive(Z), lap[2], phi);
+                    __builtin_amdgcn_sched_barrier(0);
+                } else {
+                    const double com = mb_shared(I, X, Y, Z, log_f64(B));
+                    df[0] = mb_mu_x(I, Y, Z, B, com, log_f64(X), lap[0]);
+                    df[1] = mb_mu_y(I, X, Z, B, com, log_f64(Y), lap[1]);
+                    df[2] = mb_mu_z(I, X, Y, B, com, log_f64(Z), lap[2], phi);
+                }
             } else {
                 const int64_t zo = (int64_t)zof(p - 1) * nxy;
 #pragma unroll

@@ -57,3 +57,23 @@ def test_march_matches_block_kernels(ctx, mode, shape, monkeypatch):
         assert np.array_equal(a[-1][3], o.awake(0))
         if nx >= 64:
             assert ha[:, 0].min() < nx * ny * nz // 64   # some blocks slept
+
+
+@pytest.mark.parametrize("shape", [(36, 28, 8)])
+def test_logarithms_outside_their_domain(ctx, shape, monkeypatch):
+    """Cells with a concentration of 0, below 0 or infinite, and no solvent left: the
+    march's logarithms for such lanes give what the block kernels' do (NaN, infinities)."""
+    nx, ny, nz = shape
+    X = list(configs.modelb_ic(nx, ny, nz)) + [np.zeros((nz, ny, nx))]
+    X[0][4, 5, 6] = 0.0
+    X[1][1, 20, 30] = -0.01
+    X[2][6, 14, 17] = np.inf
+    X[0][3, 25, 2], X[1][3, 25, 2] = 0.6, 0.4 - X[2][3, 25, 2]
+    p = configs.modelb_params(n=nx, nz=nz, mode=abi.MODE_REGULAR)
+    p.ny = ny
+    a, _ = run(ctx, p, X, "1", monkeypatch)
+    b, _ = run(ctx, p, X, "0", monkeypatch)
+    for sa, sb in zip(a, b):
+        for f in range(3):
+            assert np.array_equal(sa[f], sb[f], equal_nan=True), f
+    assert np.isnan(a[0][0]).any() and np.isfinite(a[0][0]).any()

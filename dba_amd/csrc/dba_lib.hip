@@ -109,7 +109,7 @@ struct Group {
     int march = 0;                // column-march single-launch steps: tiles per strip (0: off)
     bool spec = false;            // K93 single-launch steps with speculative staging
     bool kh_p2 = false;           // KH: dx, dy and the cell area of every instance are powers of two
-    int march_from = 0;           // Model B: lists of at least this many blocks take the column march (0: never)
+    int march_from = 0;           // Model B: lists of at least this many blocks take the column march (0: never, 1: the block kernels are not launched)
     int mb_nl = 1, mb_ncx = 0, mb_ncy = 0, mb_ntz = 0;  // ... layers per strip, columns in x and y, layers
     bool nine = true;             // CH 9-point stencil (the march kernel is instanced on it)
     int res_gx = 0, res_gy = 0, res_threads = 0, res_per_tile = 0;  // resident steps (k_resident.h): region, workgroup, threads per tile (0: not taken)
@@ -551,32 +551,50 @@ dba_status get_group(dba_ctx* ctx, const std::vector<int>& ids, Group** out) {
     // step with 16, 20, 32, 64, 128 waves per CU: 22.3, 21.7, 22.4, 23.9, 27.0
     int64_t cap = g->model == DBA_MODEL_MODELB ? 65536 : (g->model == DBA_MODEL_DENDRITE_K94 ? 20 * ctx->n_cu : 4096);
     g->grid = (int)std::max<int64_t>(1, std::min<int64_t>(g->total_tiles, cap));
-    // Model B column march (modelb_march_kernel): one 3D instance, steps with at
-    // least a quarter of the blocks awake. DBA_MODELB_SUPERBLOCKS=0 turns it off and
-    // =1 uses it for every non-empty list (without conserved DBA both give the same
-    // doubles). Layers per strip: the fewest rounds of resident workgroups, each
-    // round 4 nl + 4 planes long.
-    if (g->model == DBA_MODEL_MODELB && ids.size() == 1 && g->tile == 4 && g->tile_z == 4) {
+    // Model B column march (modelb_march_kernel, nz == 1: modelb_plane_kernel): one
+    // instance, steps whose list is long enough. DBA_MODELB_SUPERBLOCKS=0 turns it off
+    // and =1 uses it for every non-empty list (both give the same doubles). Layers per
+    // strip: the fewest rounds of resident workgroups, each round 4 nl + 4 planes long.
+    if (g->model == DBA_MODEL_MODELB && ids.size() == 1 && g->tile == 4) {
         const Inst& h = first->h;
-        if (h.full_tiles && h.nz > 1 && (int64_t)h.nx * h.ny < (1 << 28)) {
+        if (h.full_tiles && (h.nz > 1) == (g->tile_z == 4) && (int64_t)h.nx * h.ny < (1 << 28)) {
             const char* env = std::getenv("DBA_MODELB_SUPERBLOCKS");
             const std::string e = env ? env : "";
-            g->march_from = e == "0" ? 0 : (e == "1" ? 1 : (int)((h.nt + 3) / 4));
             g->mb_ntz = h.ntz;
             g->mb_ncx = (h.nx + MbMarch::TX - 1) / MbMarch::TX;
             g->mb_ncy = (h.ny + MbMarch::TY - 1) / MbMarch::TY;
             const int64_t cols = (int64_t)g->mb_ncx * g->mb_ncy, slots = (g->conserved ? 1 : 2) * (int64_t)ctx->n_cu;
-            int64_t best = INT64_MAX;
+            int64_t planes = INT64_MAX;
             for (int nl = 1; nl <= (g->conserved ? MbMarch::MLC : MbMarch::ML) && nl <= h.ntz; nl++) {
                 const int64_t wgs = cols * ((h.ntz + nl - 1) / nl), cost = (wgs + slots - 1) / slots * (4 * nl + 4);
-                if (cost < best) {
-                    best = cost;
+                if (cost < planes) {
+                    planes = cost;
                     g->mb_nl = nl;
                 }
             }
-            // the block kernels then only take lists shorter than march_from
-            if (g->march_from > 0)
-                g->grid = (int)std::max<int64_t>(1, std::min<int64_t>(g->grid, (g->march_from + 7) / 8));
+            // A plane of the march costs as much as about 1000 blocks of the block kernels
+            // (conserved 550: one workgroup per CU). us per step, block kernels and march:
+            // 64^3 30 and 32 (all 4096 awake); 128^3 (16 planes) 73 and 92 at 31% awake,
+            // 105 and 95 at 62%; 160 x 160 x 100 (20) 84 and 110 at 30%, 123 and 112 at
+            // 60%; 256^3 (136) 339 and 386 at 25%, 655 and 586 at 56%; conserved
+            // 96 x 80 x 64 (12) 51 and 55 at 67%, 59 and 52 all awake. A list no grid of
+            // this size can have: the march is not launched.
+            // One plane: the block kernels fill 16 of a wave's 64 lanes and lose wherever
+            // a march's workgroup has something to do (300^2 37 and 13, 43% awake 20 and
+            // 12; 700^2 118 and 26, 25% awake 49 and 17); only on large grids with next to
+            // nothing awake does its one workgroup per column cost more (2048^2 at 1% 63
+            // and 42, 4096^2 at 0.6% 79 and 109, at 5% 214 and 122).
+            int64_t from = h.nz > 1 ? planes * (g->conserved ? 550 : 1000) : (cols <= 8 * slots ? 1 : cols * 2 / 5);
+            if (e == "0" || from > h.nt) from = 0;
+            if (e == "1") from = 1;
+            g->march_from = (int)from;
+            // the block kernels then only take lists shorter than that, and return at once
+            // from the others (160 x 160 x 100, all awake: 20000 workgroups 4 us more per
+            // step than 5000; 30% awake: 71 us with 17000, 93 with 8500, 101 with 4250;
+            // conserved 96 x 80 x 64, all awake: 58 with 6600 and 56.5 with 3300, 67%
+            // awake 53 and 52, 59 with 1650)
+            if (from > 0)
+                g->grid = (int)std::max<int64_t>(1, std::min<int64_t>({g->grid, g->conserved ? (from + 1) / 2 : from, 12288}));
         }
     }
     size_t n = ids.size();
@@ -702,11 +720,24 @@ void launch_step(const Group* g, hipStream_t s) {
                         hipLaunchKernelGGL(modelb_march_kernel<false>, mgrid, dim3(MbMarch::NT), 0, s, wl_of(g), from,
                                            g->mb_nl, g->mb_ncx, g->mb_ncy);
                 }
-                hipLaunchKernelGGL((modelb_mu_kernel<4, 4>), grid, block, 0, s, wl_of(g), from);
-                hipLaunchKernelGGL((modelb_update_kernel<4, 4>), grid, block, 0, s, wl_of(g), from);
+                if (g->march_from != 1) {
+                    hipLaunchKernelGGL((modelb_mu_kernel<4, 4>), grid, block, 0, s, wl_of(g), from);
+                    hipLaunchKernelGGL((modelb_update_kernel<4, 4>), grid, block, 0, s, wl_of(g), from);
+                }
             } else {
-                hipLaunchKernelGGL((modelb_mu_kernel<4, 1>), grid, block, 0, s, wl_of(g), from);
-                hipLaunchKernelGGL((modelb_update_kernel<4, 1>), grid, block, 0, s, wl_of(g), from);
+                if (g->march_from > 0) {
+                    const dim3 mgrid((unsigned)(g->mb_ncx * g->mb_ncy));
+                    if (g->conserved)
+                        hipLaunchKernelGGL(modelb_plane_kernel<true>, mgrid, dim3(MbMarch::NT), 0, s, wl_of(g), from,
+                                           g->mb_ncx);
+                    else
+                        hipLaunchKernelGGL(modelb_plane_kernel<false>, mgrid, dim3(MbMarch::NT), 0, s, wl_of(g), from,
+                                           g->mb_ncx);
+                }
+                if (g->march_from != 1) {
+                    hipLaunchKernelGGL((modelb_mu_kernel<4, 1>), grid, block, 0, s, wl_of(g), from);
+                    hipLaunchKernelGGL((modelb_update_kernel<4, 1>), grid, block, 0, s, wl_of(g), from);
+                }
             }
         } else {
             // a wave per block; a multiple of 8 workgroups, so every XCD has as many

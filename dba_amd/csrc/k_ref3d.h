@@ -609,7 +609,8 @@ __global__ __launch_bounds__(64) void modelb_update_kernel(const WorkList wl, in
 }
 
 // ------------------------------------------------------------ Model B, column march
-// Steps of one 3D Model B instance in which at least `from` blocks are awake take
+// Steps of one 3D Model B instance in which at least `from` blocks are awake (where
+// the line lies, and why, stands where the group is built) take
 // one launch: a workgroup walks a column of 32 x 12 cells up `nl` layers of
 // blocks, plane by plane. Plane p of x, y, z (with a 2-cell halo) goes through
 // LDS once; every thread keeps the plane sums of its cell, so plane p completes
@@ -940,6 +941,215 @@ __global__ __launch_bounds__(MbMarch::NT) __attribute__((amdgpu_waves_per_eu(CON
         c2[2] = Z;
         // every read of plane p's sums was before the second barrier
         if (p < last) deposit(p + 1);
+    }
+}
+
+// ------------------------------------------------------------ Model B, one plane
+// The march's step of a grid of one plane (nz == 1, blocks of 4 x 4 x 1): a workgroup
+// takes 32 x 12 cells, the plane above and the one below are the plane itself, and
+// there is nothing to walk. Against the two block kernels, whose waves have a cell
+// on 16 of their 64 lanes: bound by the chain of loads and two barriers of a
+// workgroup on small grids, by FP64 issue on large ones. Same doubles, same stored
+// potentials and detector bytes. us per step, two block kernels -> this: 300^2
+// 36 -> 13, conserved 700^2 153 -> 35, 4096^2 2560 -> 514.
+template <bool CONS>
+struct MbPlaneLds {
+    using M = MbMarch;
+    double c[3 * M::CA], mu[3 * M::MA];
+    uint64_t vote[M::NI / 64];
+    uint64_t par, act;                             // parity and awake bits of the blocks around
+    double shift[CONS ? M::NB * 3 : 1];            // pending shift of each block
+    double part[CONS ? 3 * (M::NI / 64) * 8 : 1];  // change sums of half blocks
+};
+
+template <bool CONS>
+__global__ __launch_bounds__(MbMarch::NT) __attribute__((amdgpu_waves_per_eu(4))) void modelb_plane_kernel(
+    const WorkList wl, int from, int ncx) {
+    using M = MbMarch;
+    __shared__ MbPlaneLds<CONS> S;
+    __shared__ FoldLds FL;
+    Fold FO;
+    const int total = work_open(wl, FO, &FL);
+    if (total < from) return;
+    CInst& I = *(CInst*)wl.insts;
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int nx = I.nx, ny = I.ny, ntx = I.ntx, nty = I.nty;
+    const bool regular = I.mode == 0;
+    const int col = xcd_deal(blockIdx.x, gridDim.x, 0, gridDim.x);
+    const int x0 = (col % ncx) * M::TX, y0 = (col / ncx) * M::TY;
+    const double inv_dx2 = I.invdx2;
+    auto block_at = [&](int bit) {  // the block at a bit of the masks
+        return wrap_any(x0 / 4 + bit % M::BW - 1, ntx) + wrap_any(y0 / 4 + bit / M::BW - 1, nty) * ntx;
+    };
+
+    if (wid == 0) {
+        const int tt = block_at(lane < M::NB ? lane : 0);
+        const gu64 *par0 = I.par[0], *cur0 = I.a_cur[0];
+        asm volatile("" : "+s"(par0), "+s"(cur0));
+        const uint64_t wp = par0[tt >> 6], wa = cur0[tt >> 6];
+        const int pb = (int)((wp >> (tt & 63)) & 1ull);
+        const uint64_t pm = __ballot(pb);
+        const uint64_t am = regular ? ~0ull : __ballot((int)((wa >> (tt & 63)) & 1ull));
+        if (lane == 0) {
+            S.par = pm;
+            S.act = am;
+        }
+        if (CONS && lane < M::NB)
+#pragma unroll
+            for (int f = 0; f < 3; f++)
+                S.shift[lane * 3 + f] = I.scal[8 + f] - I.s_tile[((int64_t)f * 2 + pb) * I.nt + tt];
+    }
+    __syncthreads();
+    auto uniform = [](uint64_t w) {
+        return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(w >> 32)) << 32) |
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)w);
+    };
+    const uint64_t par = uniform(S.par), act = uniform(S.act);
+    const int bw = min(M::TX, nx - x0) / 4, bh = min(M::TY, ny - y0) / 4;
+    uint64_t own = 0ull;
+    for (int j = 0; j < bh; j++) own |= ((1ull << bw) - 1ull) << (M::BW * (j + 1) + 1);
+    if ((act & own) == 0ull) return;
+
+    auto planes = [&](int f, gdouble*& b0, gdouble*& b1) {  // (as in the march)
+        b0 = I.buf[0][f];
+        b1 = I.buf[1][f];
+        asm volatile("" : "+s"(b0), "+s"(b1));
+    };
+    // x, y, z of the region
+    const bool two = tid >= M::NT - 64;
+    double v[2][3];
+    int lbit[2];
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+        const int k = s == 0 ? tid : M::NT + lane, lx = k % M::CW, ly = k / M::CW;
+        lbit[s] = ((lx + 2) >> 2) + M::BW * ((ly + 2) >> 2);
+        const unsigned off = (unsigned)(wrap_any(x0 + lx - 2, nx) + wrap_any(y0 + ly - 2, ny) * nx) * 8u;
+        const bool q = (par >> lbit[s]) & 1ull;
+#pragma unroll
+        for (int f = 0; f < 3; f++) {
+            gdouble *b0, *b1;
+            planes(f, b0, b1);
+            v[s][f] = s == 0 || two ? at_bytes(q ? b1 : b0, off) : 0.0;
+        }
+    }
+    // this thread's cell in the region of the potentials: a cell of the column, or of its ring
+    int mx, my;
+    if (tid < M::NI) {
+        mx = 1 + (tid & 31);
+        my = 1 + (tid >> 5);
+    } else {
+        const int r = min(tid - M::NI, M::NR - 1);
+        if (r < 2 * M::MW) {
+            mx = r < M::MW ? r : r - M::MW;
+            my = r < M::MW ? 0 : M::MH - 1;
+        } else {
+            const int k = r - 2 * M::MW;
+            mx = k < M::TY ? 0 : M::MW - 1;
+            my = 1 + (k < M::TY ? k : k - M::TY);
+        }
+    }
+    const bool cell = tid < M::NI;
+    const bool mine = cell && mx - 1 < nx - x0 && my - 1 < ny - y0;  // a cell of the grid this column owns
+    const int mbit = ((mx + 3) >> 2) + M::BW * ((my + 3) >> 2);
+    const unsigned moff = (unsigned)(wrap_any(x0 + mx - 1, nx) + wrap_any(y0 + my - 1, ny) * nx) * 8u;
+    const bool wakes = (act >> mbit) & 1ull, odd = (par >> mbit) & 1ull;
+    double df[3], lap[3], phi;
+    {
+        gdouble *b0, *b1;
+        planes(3, b0, b1);
+        phi = at_bytes(odd ? b1 : b0, moff);
+    }
+    if (!wakes)
+#pragma unroll
+        for (int f = 0; f < 3; f++) df[f] = at_bytes(I.aux[f], moff);
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        if (CONS) {
+            v[0][f] -= S.shift[lbit[0] * 3 + f];
+            if (two) v[1][f] -= S.shift[lbit[1] * 3 + f];
+        }
+        S.c[f * M::CA + tid] = v[0][f];
+        if (two) S.c[f * M::CA + M::NT + lane] = v[1][f];
+    }
+    __syncthreads();
+
+    // the potentials
+    double c[3];
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        const Plane3 n = plane_sums<M::CW>(S.c + (mx + 1) + (my + 1) * M::CW + f * M::CA);
+        lap[f] = ((n.own + n.side) + n.side) * inv_dx2;
+        c[f] = n.c;
+    }
+    if (wakes) {
+        const double X = c[0], Y = c[1], Z = c[2], B = 1.0 - X - Y - Z;
+        const double com = mb_shared(I, X, Y, Z, log_f64(B));
+        __builtin_amdgcn_sched_barrier(0);
+        df[0] = mb_mu_x(I, Y, Z, B, com, log_f64(X), lap[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        df[1] = mb_mu_y(I, X, Z, B, com, log_f64(Y), lap[1]);
+        __builtin_amdgcn_sched_barrier(0);
+        df[2] = mb_mu_z(I, X, Y, B, com, log_f64(Z), lap[2], phi);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    double* sm = S.mu + mx + my * M::MW;
+    if (tid < M::NI + M::NR)
+#pragma unroll
+        for (int f = 0; f < 3; f++) sm[f * M::MA] = df[f];
+    if (cell && !regular) {
+        const uint64_t w = __ballot(mine && wakes && fabs(lap[2]) > I.thresh_a);
+        if (lane == 0) S.vote[wid] = w;
+    }
+    __syncthreads();
+    if (cell) {
+        const bool ran = mine && wakes;
+        if (!regular && ran) {
+            // the block's cells: four lanes in two rows, of this wave and its partner
+            const uint64_t w = S.vote[wid & ~1] | S.vote[wid | 1];
+            const bool fired = (w & ((0xFull | 0xFull << 32) << (tid & 28))) != 0ull;
+            if (!fired)
+#pragma unroll
+                for (int f = 0; f < 3; f++) at_bytes(I.aux[f], moff) = df[f];
+            if ((tid & 3) == 0 && ((tid >> 5) & 3) == 0) I.nflag[0][block_at(mbit)] = (uint8_t)fired;
+        }
+        // the changes
+#pragma unroll
+        for (int f = 0; f < 3; f++) {
+            const Plane3 n = plane_sums<M::MW>(sm + f * M::MA);
+            lap[f] = ((n.own + n.side) + n.side) * inv_dx2;
+        }
+        double ch[3];
+        mb_change(I, df[0], df[1], df[2], lap[0], lap[1], lap[2], ch);
+        if (ran)
+#pragma unroll
+            for (int f = 0; f < 3; f++) {
+                gdouble *b0, *b1;
+                planes(f, b0, b1);
+                at_bytes(odd ? b0 : b1, moff) = c[f] + ch[f];
+            }
+        if (CONS)
+#pragma unroll
+            for (int f = 0; f < 3; f++) {
+                double s = ran ? ch[f] : 0.0;
+                s += __shfl_xor(s, 1, 64);
+                s += __shfl_xor(s, 2, 64);
+                s += __shfl_xor(s, 32, 64);
+                if ((lane & 35) == 0) S.part[(f * (M::NI / 64) + wid) * 8 + (lane >> 2)] = s;
+            }
+    }
+    if (CONS) {
+        __syncthreads();
+        // a block's change sums: its two waves' halves
+        if (tid < 3 * (M::TY / 4) * 8) {
+            const int f = tid / (8 * (M::TY / 4)), r = tid % (8 * (M::TY / 4)), j = r / 8, i = r % 8;
+            const int bit = (i + 1) + M::BW * (j + 1);
+            if (i < bw && j < bh && ((act >> bit) & 1ull)) {
+                const int t = block_at(bit), b = (int)((par >> bit) & 1ull);
+                const double* h = S.part + (f * (M::NI / 64) + 2 * j) * 8 + i;
+                I.tpart[(int64_t)f * I.nt + t] = h[0] + h[8];
+                I.s_tile[((int64_t)f * 2 + (b ^ 1)) * I.nt + t] = I.scal[8 + f];
+            }
+        }
     }
 }
 

@@ -50,8 +50,9 @@ __device__ __forceinline__ void put_double(uint64_t* p, double v, uint32_t seq) 
     xput(p + 1, s | (uint32_t)(b >> 32));
 }
 
-// Bound of a wait: about a second of polls (each is a trip to memory).
-constexpr int kWaitPolls = 1 << 20;
+// Bound of a wait: about 20 seconds of polls (each is a trip to memory). Other work of
+// the process may hold compute units that a workgroup of the launch still needs.
+constexpr int kWaitPolls = 1 << 24;
 
 // Called while polling: true when the wait must be given up.
 __device__ __forceinline__ bool wait_over(int polls, int* stuck) {

@@ -625,7 +625,7 @@ def measure(ctx, workload, K, W, chunk_cap, timing_steps, single_launch, n=None,
         # state-restoring launch per graph chunk and the gaps between launches)
         avg_k_s = replay_ms / 1e3 / replay_steps
         cells_per_launch = (u5 - u4) / replay_steps
-        kernel = "single-launch step kernel (awake sets + fused stencil + detector)"
+        kernel = "single-launch or resident step kernel (awake sets + fused stencil + detector)"
     else:
         # two launches per step: hipEvents around every step kernel in an eager pass
         avg_k_s = eager_k_s

@@ -436,7 +436,7 @@ struct WorkList {
 constexpr int kFoldLanes = 64, kFoldSegs = 256;
 
 struct FoldLds {
-    int o[kFoldSegs + 4];  // exclusive prefix of the counts; [kFoldSegs] the total
+    alignas(16) int o[kFoldSegs + 4];  // exclusive prefix of the counts (accessed as int4); [kFoldSegs] the total
 };
 
 struct Fold {

@@ -137,6 +137,8 @@ SIGNATURES = [
     ("dba_growth_front", C.c_int32, [C.c_void_p, C.c_int32, C.c_void_p, C.c_int32, C.c_void_p]),
     ("dba_kh_vy_mode", C.c_int32, [C.c_void_p, C.c_int32, C.POINTER(C.c_double)]),
     ("dba_set_single_launch", C.c_int32, [C.c_void_p, C.c_int32]),
+    ("dba_set_resident", C.c_int32, [C.c_void_p, C.c_int32]),
+    ("dba_resident_calls", C.c_int32, [C.c_void_p, C.POINTER(C.c_int64)]),
     ("dba_droplets", C.c_int32, [C.c_void_p, C.c_int32, C.c_int32, C.POINTER(C.c_double), C.POINTER(C.c_int64),
                                  C.POINTER(C.c_int64), C.c_void_p, C.c_int64]),
     ("dba_droplets_noalloc", C.c_int32, [C.c_void_p, C.c_int32, C.c_int32, C.POINTER(C.c_double),

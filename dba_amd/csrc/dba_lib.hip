@@ -176,6 +176,8 @@ struct dba_ctx {
     size_t xwords = 0;
     uint32_t xseq = 1;
     int* stuck = nullptr;          // pinned host word: a resident step's wait ran out
+    bool resident = true;          // resident steps where they can be had (dba_set_resident)
+    int64_t resident_calls = 0;    // step calls that took them
 };
 
 namespace {
@@ -1050,7 +1052,8 @@ int live_contexts(int device, int d) {
 // false where the launch could not be had (the other paths need less) or must not be.
 dba_status enqueue_resident(dba_ctx* ctx, Group* g, int n_steps, bool* taken) {
     *taken = false;
-    if (!g->res_gx || ctx->single_launch == 0 || ctx->timing || n_steps < kResidentMinSteps) return DBA_OK;
+    if (!g->res_gx || !ctx->resident || ctx->single_launch == 0 || ctx->timing || n_steps < kResidentMinSteps)
+        return DBA_OK;
     if (live_contexts(ctx->device, 0) > 1) return DBA_OK;
     const Inst& h = ctx->inst.at(g->ids[0])->h;
     const int nt = h.nt, gx = g->res_gx, gy = g->res_gy;
@@ -1076,6 +1079,7 @@ dba_status enqueue_resident(dba_ctx* ctx, Group* g, int n_steps, bool* taken) {
         return DBA_OK;
     }
     ctx->xseq += (uint32_t)n_steps + 1u;
+    ctx->resident_calls++;
     *taken = true;
     return launch_canon(ctx, g, n_steps);
 }
@@ -1520,6 +1524,18 @@ dba_status dba_set_single_launch(dba_ctx* ctx, int32_t mode) {
     if (mode < 0 || mode > 2) return fail(DBA_ERR_INVALID, "single-launch mode must be 0, 1 or 2 (got %d)", mode);
     // captured graphs are cached per mode, so switching keeps them
     ctx->single_launch = mode;
+    return DBA_OK;
+}
+
+dba_status dba_set_resident(dba_ctx* ctx, int32_t enable) {
+    if (!ctx) return fail(DBA_ERR_INVALID, "null ctx");
+    ctx->resident = enable != 0;
+    return DBA_OK;
+}
+
+dba_status dba_resident_calls(dba_ctx* ctx, int64_t* taken) {
+    if (!ctx || !taken) return fail(DBA_ERR_INVALID, "null argument");
+    *taken = ctx->resident_calls;
     return DBA_OK;
 }
 

@@ -160,6 +160,17 @@ class Context:
         one instance; 2 also for batches. Results are identical in every mode."""
         abi.check(self.lib.dba_set_single_launch(self.h, int(mode)))
 
+    def set_resident(self, enable):
+        """Resident steps (many steps of one instance in one launch) where they can
+        be had: on by default. Results are identical."""
+        abi.check(self.lib.dba_set_resident(self.h, int(bool(enable))))
+
+    def resident_calls(self):
+        """Step calls of this context that took resident steps."""
+        n = C.c_int64()
+        abi.check(self.lib.dba_resident_calls(self.h, C.byref(n)))
+        return n.value
+
     def timing(self, enable):
         abi.check(self.lib.dba_timing_enable(self.h, 1 if enable else 0))
 

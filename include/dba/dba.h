@@ -226,6 +226,14 @@ dba_status dba_sync(dba_ctx* ctx);
  * mode. DBA_ERR_INVALID for another mode. */
 dba_status dba_set_single_launch(dba_ctx* ctx, int32_t mode);
 
+/* Resident steps of this context: 0 keeps it on the paths that launch every step,
+ * not 0 (the default) takes resident steps where dba_set_single_launch's text says.
+ * Results are bit-identical. */
+dba_status dba_set_resident(dba_ctx* ctx, int32_t enable);
+
+/* How many dba_step / dba_step_graph calls of this context took resident steps. */
+dba_status dba_resident_calls(dba_ctx* ctx, int64_t* taken);
+
 /* Active tiles of a set for the NEXT step (after dilation). mask (optional)
    receives ntiles bytes, 1 = awake. Synchronises. */
 dba_status dba_active_tiles(dba_ctx* ctx, int32_t id, int32_t set, int32_t* count, uint8_t* mask);

@@ -958,9 +958,11 @@ size_t resident_bytes(const Group* g, int w, int h) {
 // 24 resident), so at most 24 waves per CU; and a sixteenth is kept free where
 // several share a CU (27 promised by their LDS, 26.7 resident).
 bool all_resident(const dba_ctx* ctx, const void* f, int threads, size_t lds, int64_t wgs) {
-    constexpr size_t kLdsPerCu = 160 * 1024;
-    if (lds + 2048 > kLdsPerCu) return false;
-    if (lds > 64 * 1024 && hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
+    constexpr size_t kLdsPerCu = 160 * 1024, kMostLds = kLdsPerCu - 2048;  // (less the kernels' static LDS)
+    if (lds > kMostLds) return false;
+    // the most any shape asks for, since the attribute is the function's: a smaller
+    // instance's bytes would lower it below what a larger one launches with
+    if (lds > 64 * 1024 && hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMostLds) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }

@@ -138,3 +138,22 @@ def test_resident_and_single_launch_agree(ctx):
     finally:
         ctx.set_resident(True)
     same(a, b)
+
+
+def test_instances_of_several_region_shapes(ctx):
+    """One kernel serves regions of different sizes: instances of each, stepped in turn,
+    keep their resident steps (the largest LDS a launch may ask for belongs to the kernel)."""
+    sizes = [(1534, 1310), (1024, 1024), (1200, 1100), (600, 1000)]   # 3 x 3, 2 x 2, 3 x 2 and single tiles
+    insts = []
+    for k, (nx, ny) in enumerate(sizes):
+        inst = ctx.create(ch_params(nx, ny, 32))
+        inst.upload(0, patchy(nx, ny, 32, seed=k))
+        insts.append(inst)
+    n0 = ctx.resident_calls()
+    for order in (insts, insts[::-1], insts):
+        for inst in order:
+            inst.step(16)
+    assert ctx.resident_calls() == n0 + 12
+    for inst in insts:
+        assert inst.info().steps_done == 48
+        inst.destroy()

@@ -177,6 +177,7 @@ struct dba_ctx {
     uint32_t xseq = 1;
     int* stuck = nullptr;          // pinned host word: a resident step's wait ran out
     bool resident = true;          // resident steps where they can be had (dba_set_resident)
+    int wait_polls = kWaitPolls;   // polls after which one of their waits is given up
     int64_t resident_calls = 0;    // step calls that took them
 };
 
@@ -1068,7 +1069,7 @@ dba_status enqueue_resident(dba_ctx* ctx, Group* g, int n_steps, bool* taken) {
     if (ok) {
         const void* f = resident_kernel(g, g->res_per_tile);
         const size_t lds = resident_bytes(g, gx * g->tile, gy * g->tile);
-        Exchange X{ctx->xbuf, ctx->xbuf + (words - flags), ctx->stuck, ctx->xseq, slots};
+        Exchange X{ctx->xbuf, ctx->xbuf + (words - flags), ctx->stuck, ctx->wait_polls, ctx->xseq, slots};
         const Inst* insts = g->d_insts;
         int n = n_steps, ax = gx, ay = gy;
         void* args[] = {(void*)&insts, (void*)&X, (void*)&n, (void*)&ax, (void*)&ay};
@@ -1532,6 +1533,13 @@ dba_status dba_set_single_launch(dba_ctx* ctx, int32_t mode) {
 dba_status dba_set_resident(dba_ctx* ctx, int32_t enable) {
     if (!ctx) return fail(DBA_ERR_INVALID, "null ctx");
     ctx->resident = enable != 0;
+    return DBA_OK;
+}
+
+dba_status dba_set_resident_wait(dba_ctx* ctx, int32_t polls) {
+    if (!ctx) return fail(DBA_ERR_INVALID, "null ctx");
+    if (polls < 0) return fail(DBA_ERR_INVALID, "polls < 0");
+    ctx->wait_polls = polls ? polls : kWaitPolls;
     return DBA_OK;
 }
 

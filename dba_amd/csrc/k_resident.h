@@ -33,6 +33,7 @@ struct Exchange {
     uint64_t* frame;   // [parity][region][slot][2 words per field]
     uint64_t* flag;    // [parity][tile]: sequence number << 32 | detector bits
     int* stuck;        // host memory: a wait ran out
+    int polls;         // polls after which a wait is given up
     uint32_t base;     // sequence number of the launch's first step
     int slots;         // frame slots of a whole region
 };
@@ -50,24 +51,27 @@ __device__ __forceinline__ void put_double(uint64_t* p, double v, uint32_t seq) 
     xput(p + 1, s | (uint32_t)(b >> 32));
 }
 
-// Bound of a wait: about 20 seconds of polls (each is a trip to memory). Other work of
-// the process may hold compute units that a workgroup of the launch still needs.
+// Bound of a wait, if the caller sets none: about 20 seconds of polls (each is a trip to
+// memory). Other work of the process may hold compute units that a workgroup of the
+// launch still needs.
 constexpr int kWaitPolls = 1 << 24;
 
 // Called while polling: true when the wait must be given up.
-__device__ __forceinline__ bool wait_over(int polls, int* stuck) {
-    if ((polls & 1023) != 1023) return false;
-    if (polls >= kWaitPolls) __hip_atomic_store(stuck, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    return __hip_atomic_load(stuck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0;
+__device__ __forceinline__ bool wait_over(int polls, const Exchange& X) {
+    if (polls >= X.polls) {
+        __hip_atomic_store(X.stuck, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        return true;
+    }
+    return (polls & 1023) == 1023 && __hip_atomic_load(X.stuck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0;
 }
 
-__device__ __forceinline__ double wait_double(const uint64_t* p, uint32_t seq, int* stuck, int* gone) {
+__device__ __forceinline__ double wait_double(const uint64_t* p, uint32_t seq, const Exchange& X, int* gone) {
     uint64_t a, b;
     for (int k = 0;; k++) {
         a = xget(p);
         b = xget(p + 1);
         if ((uint32_t)(a >> 32) == seq && (uint32_t)(b >> 32) == seq) break;
-        if (wait_over(k, stuck)) {
+        if (wait_over(k, X)) {
             *gone = 1;
             break;
         }
@@ -75,12 +79,12 @@ __device__ __forceinline__ double wait_double(const uint64_t* p, uint32_t seq, i
     return __longlong_as_double((long long)((uint64_t)(uint32_t)b << 32 | (uint32_t)a));
 }
 
-__device__ __forceinline__ int wait_flag(const uint64_t* p, uint32_t seq, int* stuck, int* gone) {
+__device__ __forceinline__ int wait_flag(const uint64_t* p, uint32_t seq, const Exchange& X, int* gone) {
     uint64_t a;
     for (int k = 0;; k++) {
         a = xget(p);
         if ((uint32_t)(a >> 32) == seq) break;
-        if (wait_over(k, stuck)) {
+        if (wait_over(k, X)) {
             *gone = 1;
             break;
         }
@@ -372,7 +376,7 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
         // 2. the frames of the tiles outside that ran, the detector bits around
         if (s > 0) {
             const uint64_t ran = sact[(s & 1) ^ 1];
-            if (hpos >= 0 && ((ran >> hpos) & 1ull)) sc[hcell] = wait_double(fin + hslot, seq, X.stuck, &gone);
+            if (hpos >= 0 && ((ran >> hpos) & 1ull)) sc[hcell] = wait_double(fin + hslot, seq, X, &gone);
             if (tid >= nthr - 64) {
                 const uint64_t exist = __ballot(near >= 0);
                 uint64_t m = exist;
@@ -381,7 +385,7 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
                     int b = 0;
                     if (near >= 0)
                         b = own_tile >= 0 ? fp[own_tile]
-                                          : wait_flag(X.flag + (int64_t)((s & 1) ^ 1) * I.nt + near, seq, X.stuck, &gone);
+                                          : wait_flag(X.flag + (int64_t)((s & 1) ^ 1) * I.nt + near, seq, X, &gone);
                     m = G.dilate(__ballot(b), exist);
                 }
                 if (lane == 0) sact[s & 1] = m;
@@ -389,6 +393,7 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
         }
         if (tid < kResMaxTiles) fire[(s + 1) % 3][tid] = 0;
         lds_barrier();
+        if (gone) break;  // the same in every wave: written before this barrier, and not again before two more
         const uint64_t act = sact[s & 1];
         auto runs = [&](int j) { return (act >> tiles[j].pos) & 1ull; };
         // 3. mu of tiles a neighbour woke, of the region's edge, of the ring of running tiles outside
@@ -447,7 +452,6 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
             }
         }
         lds_barrier();
-        if (gone) break;
     }
 
     // ---- the state the other paths read: the cells into the buffer that was not

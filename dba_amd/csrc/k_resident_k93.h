@@ -165,8 +165,8 @@ __global__ __launch_bounds__(1024) void k93_resident_kernel(const Inst* __restri
                 const uint64_t* q = fin + hslot;
                 const bool wp = (sact[(s & 1) ^ 1][0] >> hpos) & 1ull;
                 const bool wT = hT >= 0 && ((sact[(s & 1) ^ 1][1] >> hpos) & 1ull);
-                if (wp) sp[hphi] = wait_double(q, seq, X.stuck, &gone);
-                if (wT) sT[hT] = wait_double(q + 2, seq, X.stuck, &gone);
+                if (wp) sp[hphi] = wait_double(q, seq, X, &gone);
+                if (wT) sT[hT] = wait_double(q + 2, seq, X, &gone);
             }
             if (tid >= nthr - 64) {
                 const uint64_t exist = __ballot(near >= 0);
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(1024) void k93_resident_kernel(const Inst* __restri
                 if (!regular) {
                     int f = 0;
                     if (own >= 0) f = fire[0][prev][own] | fire[1][prev][own] << 1;
-                    else if (near >= 0) f = wait_flag(X.flag + (int64_t)((s & 1) ^ 1) * nt + near, seq, X.stuck, &gone);
+                    else if (near >= 0) f = wait_flag(X.flag + (int64_t)((s & 1) ^ 1) * nt + near, seq, X, &gone);
                     a = G.dilate(__ballot(f & 1), exist);
                     b = G.dilate(__ballot(f & 2), exist);
                 }
@@ -186,6 +186,7 @@ __global__ __launch_bounds__(1024) void k93_resident_kernel(const Inst* __restri
         }
         if (tid < kResMaxTiles) fire[0][(s + 1) % 3][tid] = fire[1][(s + 1) % 3][tid] = 0;
         lds_barrier();
+        if (gone) break;  // the same in every wave: written before this barrier, and not again before two more
         const uint64_t actp = sact[s & 1][0], actT = sact[s & 1][1];
         // 3. the rest
         const bool ap = in && ((actp >> pos) & 1ull), aT = in && ((actT >> pos) & 1ull);
@@ -253,7 +254,6 @@ __global__ __launch_bounds__(1024) void k93_resident_kernel(const Inst* __restri
                 }
             }
         }
-        if (gone) break;
     }
     __syncthreads();
 

@@ -165,6 +165,11 @@ class Context:
         be had: on by default. Results are identical."""
         abi.check(self.lib.dba_set_resident(self.h, int(bool(enable))))
 
+    def set_resident_wait(self, polls):
+        """Looks at another workgroup's word before a resident step's wait is given up
+        (0: the default)."""
+        abi.check(self.lib.dba_set_resident_wait(self.h, int(polls)))
+
     def resident_calls(self):
         """Step calls of this context that took resident steps."""
         n = C.c_int64()

@@ -231,6 +231,10 @@ dba_status dba_set_single_launch(dba_ctx* ctx, int32_t mode);
  * Results are bit-identical. */
 dba_status dba_set_resident(dba_ctx* ctx, int32_t enable);
 
+/* How often a workgroup of a resident step looks for a word of another one (each look
+ * is a trip to memory, about a microsecond) before it gives the wait up; 0: the default. */
+dba_status dba_set_resident_wait(dba_ctx* ctx, int32_t polls);
+
 /* How many dba_step / dba_step_graph calls of this context took resident steps. */
 dba_status dba_resident_calls(dba_ctx* ctx, int64_t* taken);
 

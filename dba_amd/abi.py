@@ -140,6 +140,7 @@ SIGNATURES = [
     ("dba_set_resident", C.c_int32, [C.c_void_p, C.c_int32]),
     ("dba_set_resident_wait", C.c_int32, [C.c_void_p, C.c_int32]),
     ("dba_resident_calls", C.c_int32, [C.c_void_p, C.POINTER(C.c_int64)]),
+    ("dba_resident_redone", C.c_int32, [C.c_void_p, C.POINTER(C.c_int64)]),
     ("dba_droplets", C.c_int32, [C.c_void_p, C.c_int32, C.c_int32, C.POINTER(C.c_double), C.POINTER(C.c_int64),
                                  C.POINTER(C.c_int64), C.c_void_p, C.c_int64]),
     ("dba_droplets_noalloc", C.c_int32, [C.c_void_p, C.c_int32, C.c_int32, C.POINTER(C.c_double),

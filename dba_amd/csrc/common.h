@@ -42,7 +42,7 @@ struct Inst {
     gdouble* tspeed;              // KH: per-tile max wave speed, [0..nt) fresh (current U), [nt..2nt) stale
     gdouble* s_tile;              // conserved: per-tile epoch of the cumulative shift, [field][parity][nt]
     gdouble* scal;                // [1] dt of the next step, [2] time, [3] last dt, [8+f] cumulative shift S_f
-    gi64* ctr;                    // [0] steps done, [1] active cell updates, [2] worklist length
+    gi64* ctr;                    // [0] steps done, [1] active cell updates, [2] worklist length, [3] resident steps given up
     gi32* hist;                   // per-step active tile counts, [2*step + set]
     gi32* seg;                    // this instance's compacted worklist (ascending tiles)
     gu64* nbrec;                  // per worklist position (2D): the 3x3 neighbours' parity and awake bits

@@ -175,10 +175,13 @@ struct dba_ctx {
     uint64_t* xbuf = nullptr;
     size_t xwords = 0;
     uint32_t xseq = 1;
-    int* stuck = nullptr;          // pinned host word: a resident step's wait ran out
+    uint32_t* xstate = nullptr;    // state of the resident launches, workgroups done (k_resident.h)
+    int* stuck = nullptr;          // pinned host word: a resident launch was given up
+    std::vector<int> unsettled;    // instances with resident launches since the host last waited
     bool resident = true;          // resident steps where they can be had (dba_set_resident)
     int wait_polls = kWaitPolls;   // polls after which one of their waits is given up
     int64_t resident_calls = 0;    // step calls that took them
+    int64_t resident_redone = 0;   // steps of launches given up, made again on another path
 };
 
 namespace {
@@ -909,15 +912,15 @@ dba_status partition(dba_ctx* ctx, const int32_t* ids, int32_t n_ids, std::vecto
 }
 
 // The state-restoring launches after n_steps single-launch or resident steps.
-dba_status launch_canon(dba_ctx* ctx, const Group* g, int n_steps) {
+dba_status launch_canon(dba_ctx* ctx, const Group* g, int n_steps, uint32_t* res = nullptr) {
     if (!g->d_dmap) {
-        hipLaunchKernelGGL(dense_canon_kernel, dim3(1), dim3(kFinNT), 0, ctx->stream, g->d_insts, n_steps);
+        hipLaunchKernelGGL(dense_canon_kernel, dim3(1), dim3(kFinNT), 0, ctx->stream, g->d_insts, n_steps, res);
     } else {
         hipLaunchKernelGGL(dense_canon_seg_kernel, dim3((unsigned)g->nseg), dim3(kFinNT), 0, ctx->stream, g->d_insts,
-                           g->d_segs, g->d_parts, g->d_counts, n_steps);
+                           g->d_segs, g->d_parts, g->d_counts, n_steps, (const uint32_t*)res);
         LAUNCH_CHECK();
         hipLaunchKernelGGL(dense_canon_merge_kernel, dim3(1), dim3(kFinNT), 0, ctx->stream, g->d_insts, g->d_isegs,
-                           (int)g->ids.size(), g->d_parts, g->d_counts, n_steps);
+                           (int)g->ids.size(), g->d_parts, g->d_counts, n_steps, res);
     }
     LAUNCH_CHECK();
     return DBA_OK;
@@ -1025,6 +1028,10 @@ bool resident_buffer(dba_ctx* ctx, size_t words, int n_steps) {
         if (hipHostMalloc((void**)&ctx->stuck, sizeof(int)) != hipSuccess) return false;
         *ctx->stuck = 0;
     }
+    if (!ctx->xstate) {
+        if (hipMalloc(&ctx->xstate, 2 * sizeof(uint32_t)) != hipSuccess) return false;
+        if (hipMemsetAsync(ctx->xstate, 0, 2 * sizeof(uint32_t), ctx->stream) != hipSuccess) return false;
+    }
     const bool wrap = ctx->xseq > 0xffffffffu - (uint32_t)n_steps - 2u;
     if (words <= ctx->xwords && !wrap) return true;
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
@@ -1051,6 +1058,11 @@ int live_contexts(int device, int d) {
     return (*live)[device] += d;
 }
 
+// Whether an instance has resident launches that the host has not waited for.
+bool is_unsettled(const dba_ctx* ctx, int id) {
+    return std::find(ctx->unsettled.begin(), ctx->unsettled.end(), id) != ctx->unsettled.end();
+}
+
 // n_steps of one group as a resident launch and its canonicalising kernels; *taken is
 // false where the launch could not be had (the other paths need less) or must not be.
 dba_status enqueue_resident(dba_ctx* ctx, Group* g, int n_steps, bool* taken) {
@@ -1058,33 +1070,38 @@ dba_status enqueue_resident(dba_ctx* ctx, Group* g, int n_steps, bool* taken) {
     if (!g->res_gx || !ctx->resident || ctx->single_launch == 0 || ctx->timing || n_steps < kResidentMinSteps)
         return DBA_OK;
     if (live_contexts(ctx->device, 0) > 1) return DBA_OK;
-    const Inst& h = ctx->inst.at(g->ids[0])->h;
+    const int h_id = g->ids[0];
+    const Inst& h = ctx->inst.at(h_id)->h;
     const int nt = h.nt, gx = g->res_gx, gy = g->res_gy;
     const unsigned wgs = (unsigned)(((h.ntx + gx - 1) / gx) * ((h.nty + gy - 1) / gy));
     const int slots = frame_slots(gx * g->tile, gy * g->tile);
     const size_t flags = 2 * (size_t)nt;
     const int fields = g->model == DBA_MODEL_DENDRITE_K93 ? 2 : 1;
     const size_t words = 2 * (size_t)wgs * (size_t)slots * 2 * fields + flags;
-    bool ok = resident_buffer(ctx, words, n_steps);
-    if (ok) {
+    const bool have = resident_buffer(ctx, words, n_steps);
+    hipError_t e = hipErrorOutOfMemory;
+    if (have) {
         const void* f = resident_kernel(g, g->res_per_tile);
         const size_t lds = resident_bytes(g, gx * g->tile, gy * g->tile);
-        Exchange X{ctx->xbuf, ctx->xbuf + (words - flags), ctx->stuck, ctx->wait_polls, ctx->xseq, slots};
+        Exchange X{ctx->xbuf, ctx->xbuf + (words - flags), ctx->xstate, ctx->stuck, ctx->wait_polls, ctx->xseq, slots};
         const Inst* insts = g->d_insts;
         int n = n_steps, ax = gx, ay = gy;
         void* args[] = {(void*)&insts, (void*)&X, (void*)&n, (void*)&ax, (void*)&ay};
-        ok = hipLaunchCooperativeKernel(f, dim3(wgs), dim3((unsigned)g->res_threads), args, (unsigned)lds,
-                                        ctx->stream) == hipSuccess;
+        e = hipLaunchCooperativeKernel(f, dim3(wgs), dim3((unsigned)g->res_threads), args, (unsigned)lds, ctx->stream);
     }
-    if (!ok) {  // too little memory, or no such launch here: the other paths from now on
+    if (e != hipSuccess) {
         (void)hipGetLastError();
-        g->res_gx = 0;
+        // too little memory is tried again; another process may have the GPU's queue for
+        // cooperative launches, and every attempt to get it takes 15 ms
+        if (e == hipErrorCooperativeLaunchTooLarge) g->res_gx = 0;
+        else if (have) ctx->resident = false;
         return DBA_OK;
     }
     ctx->xseq += (uint32_t)n_steps + 1u;
     ctx->resident_calls++;
+    if (!is_unsettled(ctx, h_id)) ctx->unsettled.push_back(h_id);
     *taken = true;
-    return launch_canon(ctx, g, n_steps);
+    return launch_canon(ctx, g, n_steps, ctx->xstate);
 }
 
 dba_status enqueue_steps(dba_ctx* ctx, const std::vector<Group*>& gs, int n_steps, bool timed) {
@@ -1181,20 +1198,77 @@ dba_status ensure_staging(dba_ctx* ctx, size_t n) {
 
 }  // namespace
 
-// Waits for the compute stream; an error if a resident step's wait ran out.
 namespace {
-dba_status wait_stream(dba_ctx* ctx) {
+// Waits for the compute stream. Steps of resident launches that were given up are then
+// made on the other paths, so the caller never sees them missing; *redone says so to
+// calls that had already read the state. The context keeps to the other paths after
+// that: what held the launch up (another process on the GPU) may still be there.
+dba_status wait_stream(dba_ctx* ctx, bool* redone = nullptr) {
     HIP_TRY(hipStreamSynchronize(ctx->stream));
-    if (ctx->stuck && *(volatile int*)ctx->stuck)
-        return fail(DBA_ERR_HIP, "a resident step waited too long for another workgroup: the fields are not valid");
+    std::vector<int> ids;
+    ids.swap(ctx->unsettled);
+    if (!ctx->stuck || !*(volatile int*)ctx->stuck) return DBA_OK;
+    *ctx->stuck = 0;
+    ctx->resident = false;
+    HIP_TRY(hipMemsetAsync(ctx->xstate, 0, 2 * sizeof(uint32_t), ctx->stream));
+    for (int id : ids) {
+        Instance* in = ctx->inst.at(id);
+        int64_t ctr[4];
+        HIP_TRY(hipMemcpy(ctr, in->h.ctr, sizeof(ctr), hipMemcpyDeviceToHost));
+        if (ctr[3] == 0) continue;
+        HIP_TRY(hipMemsetAsync(in->h.ctr + 3, 0, sizeof(int64_t), ctx->stream));
+        // (the launch counted in the history of its steps as it went)
+        if (ctr[0] < in->h.hist_cap)
+            HIP_TRY(hipMemsetAsync(in->h.hist + 2 * ctr[0], 0, sizeof(int32_t) * 2 * (size_t)(in->h.hist_cap - ctr[0]),
+                                   ctx->stream));
+        std::vector<Group*> gs;
+        const int32_t one = id;
+        dba_status st = prepare_groups(ctx, &one, 1, &gs);
+        for (int64_t left = ctr[3]; st == DBA_OK && left > 0;) {
+            const int n = (int)std::min<int64_t>(left, 1 << 16);
+            st = enqueue_steps(ctx, gs, n, false);
+            left -= n;
+        }
+        if (st != DBA_OK) return st;
+        ctx->resident_redone += ctr[3];
+        if (redone) *redone = true;
+    }
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
     return DBA_OK;
+}
+
+// Before work on an instance that a redone step must not come after.
+dba_status settle(dba_ctx* ctx, int id, bool* redone = nullptr) {
+    return is_unsettled(ctx, id) ? wait_stream(ctx, redone) : DBA_OK;
+}
+
+// ... of a step call: the groups anew if steps were redone.
+dba_status settle_groups(dba_ctx* ctx, const int32_t* ids, int32_t n_ids, std::vector<Group*>* gs) {
+    bool redone = false;
+    for (int k = 0; k < n_ids; k++) {
+        const dba_status st = settle(ctx, ids[k], &redone);
+        if (st != DBA_OK) return st;
+    }
+    if (!redone) return DBA_OK;
+    gs->clear();
+    return prepare_groups(ctx, ids, n_ids, gs);
 }
 }  // namespace
 
-#define WAIT_STREAM(ctx)                              \
+#define DBA_TRY(expr)                                 \
     do {                                              \
-        const dba_status w_ = wait_stream(ctx);       \
-        if (w_ != DBA_OK) return w_;                  \
+        const dba_status t_ = (expr);                 \
+        if (t_ != DBA_OK) return t_;                  \
+    } while (0)
+
+#define WAIT_STREAM(ctx) DBA_TRY(wait_stream(ctx))
+
+// ... after the state was read on the stream: `again` (the same call) if steps were redone
+#define WAIT_READ(ctx, again)                         \
+    do {                                              \
+        bool redone_ = false;                         \
+        DBA_TRY(wait_stream(ctx, &redone_));          \
+        if (redone_) return again;                    \
     } while (0)
 
 // ===================================================================== C ABI
@@ -1275,6 +1349,7 @@ dba_status dba_finalize(dba_ctx* ctx) {
     for (auto m : ctx->markers) (void)hipEventDestroy(m);
     if (ctx->staging) (void)hipFree(ctx->staging);
     if (ctx->xbuf) (void)hipFree(ctx->xbuf);
+    if (ctx->xstate) (void)hipFree(ctx->xstate);
     if (ctx->stuck) (void)hipHostFree(ctx->stuck);
     if (ctx->d_flag) (void)hipFree(ctx->d_flag);
     if (ctx->d_diag) (void)hipFree(ctx->d_diag);
@@ -1405,6 +1480,7 @@ dba_status dba_instance_destroy(dba_ctx* ctx, int32_t id) {
     Instance* in = find(ctx, id);
     if (!in) return fail(DBA_ERR_NOTFOUND, "unknown instance %d", id);
     (void)hipStreamSynchronize(ctx->stream);
+    ctx->unsettled.erase(std::remove(ctx->unsettled.begin(), ctx->unsettled.end(), id), ctx->unsettled.end());
     invalidate_groups(ctx, id);
     free_instance(in);
     ctx->inst.erase(id);
@@ -1447,6 +1523,7 @@ dba_status dba_upload(dba_ctx* ctx, int32_t id, int32_t field, const double* hos
     // upload overlaps the steps of other instances; otherwise it is ordered
     // after them on the compute stream.
     hipStream_t s = in->stepped ? ctx->stream : ctx->setup;
+    DBA_TRY(settle(ctx, id));
     HIP_TRY(hipMemcpyAsync(in->h.buf[0][field], host, n * sizeof(double), hipMemcpyHostToDevice, s));
     HIP_TRY(hipMemcpyAsync(in->h.buf[1][field], in->h.buf[0][field], n * sizeof(double), hipMemcpyDeviceToDevice, s));
     if (in->h.ncons > 0) {
@@ -1471,7 +1548,7 @@ dba_status dba_download(dba_ctx* ctx, int32_t id, int32_t field, double* host, s
                        ctx->staging);
     LAUNCH_CHECK();
     HIP_TRY(hipMemcpyAsync(host, ctx->staging, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    WAIT_STREAM(ctx);
+    WAIT_READ(ctx, dba_download(ctx, id, field, host, n));
     return DBA_OK;
 }
 
@@ -1484,6 +1561,7 @@ dba_status dba_step(dba_ctx* ctx, const int32_t* ids, int32_t n_ids, int32_t n_s
     bool taken = false;
     if (gs.size() == 1) st = enqueue_resident(ctx, gs[0], n_steps, &taken);
     if (st != DBA_OK || taken) return st;
+    DBA_TRY(settle_groups(ctx, ids, n_ids, &gs));
     return enqueue_steps(ctx, gs, n_steps, ctx->timing);
 }
 
@@ -1496,6 +1574,7 @@ dba_status dba_step_graph(dba_ctx* ctx, const int32_t* ids, int32_t n_ids, int32
     bool taken = false;
     if (gs.size() == 1) st = enqueue_resident(ctx, gs[0], n_steps, &taken);
     if (st != DBA_OK || taken) return st;
+    DBA_TRY(settle_groups(ctx, ids, n_ids, &gs));
     int reps = n_steps / chunk, rem = n_steps % chunk;
     if (reps > 0) {
         GraphKey key{std::vector<int>(ids, ids + n_ids), chunk, ctx->single_launch};
@@ -1549,6 +1628,12 @@ dba_status dba_resident_calls(dba_ctx* ctx, int64_t* taken) {
     return DBA_OK;
 }
 
+dba_status dba_resident_redone(dba_ctx* ctx, int64_t* steps) {
+    if (!ctx || !steps) return fail(DBA_ERR_INVALID, "null argument");
+    *steps = ctx->resident_redone;
+    return DBA_OK;
+}
+
 dba_status dba_sync(dba_ctx* ctx) {
     if (!ctx) return fail(DBA_ERR_INVALID, "null ctx");
     WAIT_STREAM(ctx);
@@ -1579,6 +1664,7 @@ dba_status dba_worklist(dba_ctx* ctx, int32_t id, int32_t* tiles, int32_t cap, i
     Instance* in = find(ctx, id);
     if (!in) return fail(DBA_ERR_NOTFOUND, "unknown instance %d", id);
     // compact the instance's current awake set (the list the next step runs)
+    DBA_TRY(settle(ctx, id));
     std::vector<Group*> gs;
     dba_status st = prepare_groups(ctx, &id, 1, &gs);
     if (st != DBA_OK) return st;
@@ -1663,7 +1749,7 @@ dba_status dba_check_finite(dba_ctx* ctx, int32_t id) {
     LAUNCH_CHECK();
     int bad = 0;
     HIP_TRY(hipMemcpyAsync(&bad, ctx->d_flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    WAIT_STREAM(ctx);
+    WAIT_READ(ctx, dba_check_finite(ctx, id));
     if (bad) return fail(DBA_ERR_NUMERIC, "instance %d holds non-finite values", id);
     return DBA_OK;
 }
@@ -1681,7 +1767,7 @@ dba_status dba_field_sum(dba_ctx* ctx, int32_t id, int32_t field, double* sum) {
     hipLaunchKernelGGL(reduce_parts_kernel, dim3(1), dim3(64), 0, ctx->stream, part, 1, res);
     LAUNCH_CHECK();
     HIP_TRY(hipMemcpyAsync(sum, res, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    WAIT_STREAM(ctx);
+    WAIT_READ(ctx, dba_field_sum(ctx, id, field, sum));
     return DBA_OK;
 }
 
@@ -1702,7 +1788,7 @@ dba_status dba_growth_front(dba_ctx* ctx, int32_t id, const int32_t* xs, int32_t
                        ctx->d_cols, n, res);
     LAUNCH_CHECK();
     HIP_TRY(hipMemcpyAsync(front, res, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
-    WAIT_STREAM(ctx);
+    WAIT_READ(ctx, dba_growth_front(ctx, id, xs, n, front));
     return DBA_OK;
 }
 
@@ -1738,7 +1824,7 @@ dba_status dba_droplets(dba_ctx* ctx, int32_t id, int32_t field, double* avg, in
     int64_t cnt[2];
     HIP_TRY(hipMemcpyAsync(cnt, counters, sizeof(cnt), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipMemcpyAsync(avg, d_avg, sizeof(double), hipMemcpyDeviceToHost, st));
-    WAIT_STREAM(ctx);
+    WAIT_READ(ctx, dba_droplets(ctx, id, field, avg, volume, n_droplets, sizes, cap));
     *n_droplets = cnt[0];
     *volume = cnt[1];
     if (cap == 0 || cnt[0] == 0) return DBA_OK;
@@ -1803,7 +1889,7 @@ dba_status dba_droplets_noalloc(dba_ctx* ctx, int32_t id, int32_t field, double*
     int64_t cnt[2];
     HIP_TRY(hipMemcpyAsync(cnt, counters, sizeof(cnt), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipMemcpyAsync(avg, d_avg, sizeof(double), hipMemcpyDeviceToHost, st));
-    WAIT_STREAM(ctx);
+    WAIT_READ(ctx, dba_droplets_noalloc(ctx, id, field, avg, volume, n_droplets, sizes, cap));
     *n_droplets = cnt[0];
     *volume = cnt[1];
     if (cap == 0 || cnt[0] == 0) return DBA_OK;

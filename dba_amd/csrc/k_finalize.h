@@ -648,14 +648,28 @@ __device__ __forceinline__ void dense_canon_finish(CInst& I, int n, unsigned lon
     I.scal[3] = dt;
 }
 
+// After a resident launch (res: its state, k_resident.h; null after single-launch
+// steps): whether it was given up. Then its steps are counted in ctr[3], for the host,
+// and everything else stays as it was before them.
+__device__ __forceinline__ bool resident_given_up(const uint32_t* res) { return res && res[0] == 1u; }
+
+__device__ __forceinline__ void resident_skip_seg(CInst& I, int t0, int ntile) {
+    if ((int)threadIdx.x < ntile) I.druns[t0 + threadIdx.x] = 0;
+}
+
 // One instance in one segment: one workgroup does it all. Conserved (CH): the
 // cumulative shift after the last step, from the last step's change sums in the
 // finalize's order (block_sum over the tiles, 0 for tiles that did not run).
-__global__ __launch_bounds__(kFinNT) void dense_canon_kernel(const Inst* __restrict__ insts, int n) {
+__global__ __launch_bounds__(kFinNT) void dense_canon_kernel(const Inst* __restrict__ insts, int n, uint32_t* res) {
     __shared__ unsigned long long scells[kFinNT / 64];
     __shared__ int scnt[kFinNT / 64];
     __shared__ double sd[kFinNT / 64 + 1];
     CInst& I = ((CInst*)insts)[0];
+    if (resident_given_up(res)) {
+        resident_skip_seg(I, 0, I.nt);
+        if (threadIdx.x == 0) I.ctr[3] += n;
+        return;
+    }
     unsigned long long c;
     int cnt;
     dense_canon_seg(I, 0, I.nt, n, scells, scnt, &c, &cnt);
@@ -665,7 +679,10 @@ __global__ __launch_bounds__(kFinNT) void dense_canon_kernel(const Inst* __restr
         const double tot = block_sum<kFinNT>(v, sd);
         if (t == 0) I.scal[8] = I.scal[12 + last] + tot / I.ntotal;
     }
-    if (threadIdx.x == 0) dense_canon_finish(I, n, c, cnt);
+    if (threadIdx.x == 0) {
+        dense_canon_finish(I, n, c, cnt);
+        if (res) res[0] = res[1] = 0u;  // (every thread read it before the segment's barrier)
+    }
 }
 
 // Several segments or instances: one workgroup per segment writes its partial
@@ -673,11 +690,16 @@ __global__ __launch_bounds__(kFinNT) void dense_canon_kernel(const Inst* __restr
 __global__ __launch_bounds__(kFinNT) void dense_canon_seg_kernel(const Inst* __restrict__ insts,
                                                                  const Seg* __restrict__ segs,
                                                                  SegPart* __restrict__ parts,
-                                                                 int32_t* __restrict__ counts, int n) {
+                                                                 int32_t* __restrict__ counts, int n,
+                                                                 const uint32_t* res) {
     __shared__ unsigned long long scells[kFinNT / 64];
     __shared__ int scnt[kFinNT / 64];
     const Seg sg = segs[blockIdx.x];
     CInst& I = ((CInst*)insts)[sg.inst];
+    if (resident_given_up(res)) {
+        resident_skip_seg(I, sg.tile0, sg.ntile);
+        return;
+    }
     unsigned long long c;
     int cnt;
     dense_canon_seg(I, sg.tile0, sg.ntile, n, scells, scnt, &c, &cnt);
@@ -691,8 +713,15 @@ __global__ __launch_bounds__(kFinNT) void dense_canon_seg_kernel(const Inst* __r
 __global__ __launch_bounds__(kFinNT) void dense_canon_merge_kernel(const Inst* __restrict__ insts,
                                                                    const InstSegs* __restrict__ isegs, int n_inst,
                                                                    const SegPart* __restrict__ parts,
-                                                                   const int32_t* __restrict__ counts, int n) {
+                                                                   const int32_t* __restrict__ counts, int n,
+                                                                   uint32_t* res) {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if (resident_given_up(res)) {  // (a resident launch is one instance's)
+        if (threadIdx.x == 0) ((CInst*)insts)[0].ctr[3] += n;
+        return;
+    }
+    __syncthreads();
+    if (res && threadIdx.x == 0) res[0] = res[1] = 0u;
     for (int i = wid; i < n_inst; i += kFinNT / 64) {
         const InstSegs r = isegs[i];
         unsigned long long c = 0;

@@ -17,11 +17,16 @@
 // s + 2 only after step s + 1, for which it has received every neighbour's word of
 // step s, and those were sent after the neighbour had read generation s.
 //
-// Progress: the launch is cooperative, so all workgroups are resident; a workgroup
-// waits only for words of the step before, which their owners send without waiting
-// for anything of this step, so by induction over the steps every wait ends. Each
-// wait is bounded all the same: past the bound, or once any other wait has passed
-// it, a workgroup says so in *stuck and ends its steps, and the host returns an error.
+// Progress: the launch is cooperative and its size is checked against the chip, so all
+// workgroups are resident unless something else holds compute units (another process);
+// a workgroup waits only for words of the step before, which their owners send without
+// waiting for anything of this step, so by induction over the steps every wait ends.
+// Each wait is bounded all the same: past the bound, or once any other wait has passed
+// it, a workgroup gives the launch up, and the host has its steps made on another path.
+// So a launch that is given up leaves the instance as it was. What it stores before its
+// end only counts once the canonicalising kernel takes it over (the cells go to the
+// buffers that are not current); what replaces state in place (the stored potential
+// rings of CH) waits until every workgroup has made all its steps (resident_all_done).
 #pragma once
 #include "common.h"
 #include "k_ch.h"
@@ -32,7 +37,8 @@ namespace dba {
 struct Exchange {
     uint64_t* frame;   // [parity][region][slot][2 words per field]
     uint64_t* flag;    // [parity][tile]: sequence number << 32 | detector bits
-    int* stuck;        // host memory: a wait ran out
+    uint32_t* state;   // kRes..., and the number of workgroups that have made all their steps
+    int* stuck;        // host memory: the launch was given up
     int polls;         // polls after which a wait is given up
     uint32_t base;     // sequence number of the launch's first step
     int slots;         // frame slots of a whole region
@@ -51,18 +57,51 @@ __device__ __forceinline__ void put_double(uint64_t* p, double v, uint32_t seq) 
     xput(p + 1, s | (uint32_t)(b >> 32));
 }
 
-// Bound of a wait, if the caller sets none: about 20 seconds of polls (each is a trip to
+// State of the context's resident launches. A launch that starts in kResGivenUp makes no
+// steps: the host has not taken notice of the one before it yet.
+constexpr uint32_t kResRunning = 0, kResGivenUp = 1, kResDone = 2;
+
+// Bound of a wait, if the caller sets none: about a second of polls (each is a trip to
 // memory). Other work of the process may hold compute units that a workgroup of the
-// launch still needs.
-constexpr int kWaitPolls = 1 << 24;
+// launch still needs, and a launch given up costs that second once: the context then
+// keeps to the other paths.
+constexpr int kWaitPolls = 1 << 20;
+
+__device__ __forceinline__ uint32_t resident_state(const Exchange& X) {
+    return __hip_atomic_load(X.state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Gives the launch up, unless it is done.
+__device__ __forceinline__ void resident_give_up(const Exchange& X) {
+    uint32_t s = kResRunning;
+    if (__hip_atomic_compare_exchange_strong(X.state, &s, kResGivenUp, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT))
+        __hip_atomic_store(X.stuck, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // Called while polling: true when the wait must be given up.
 __device__ __forceinline__ bool wait_over(int polls, const Exchange& X) {
     if (polls >= X.polls) {
-        __hip_atomic_store(X.stuck, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        resident_give_up(X);
         return true;
     }
-    return (polls & 1023) == 1023 && __hip_atomic_load(X.stuck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0;
+    return (polls & 1023) == 1023 && resident_state(X) == kResGivenUp;
+}
+
+// One thread of a workgroup that has made all its steps: true once all workgroups have,
+// false if the launch was given up instead. Costs a trip to memory and the last
+// workgroup's lag, once per launch.
+__device__ __forceinline__ bool resident_all_done(const Exchange& X) {
+    if (__hip_atomic_fetch_add(X.state + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x) {
+        uint32_t s = kResRunning;
+        __hip_atomic_compare_exchange_strong(X.state, &s, kResDone, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+    }
+    for (int k = 0;; k++) {
+        const uint32_t s = resident_state(X);
+        if (s != kResRunning) return s == kResDone;
+        if (k >= X.polls) resident_give_up(X);
+    }
 }
 
 __device__ __forceinline__ double wait_double(const uint64_t* p, uint32_t seq, const Exchange& X, int* gone) {
@@ -217,7 +256,7 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
     extern __shared__ __align__(16) double lds[];
     __shared__ ResTile tiles[kResMaxTiles];
     __shared__ int fire[3][kResMaxTiles];  // detector bits of step s in fire[s % 3]
-    __shared__ int gone;                   // a wait ran out
+    __shared__ int gone;                   // the launch was given up
     __shared__ uint64_t sact[2];           // awake tiles of step s: positions of the region and two tiles around it
     CInst& I = ((CInst*)insts)[0];
     const int tid = threadIdx.x, lane = tid & 63, nthr = blockDim.x;
@@ -257,7 +296,7 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
         if (lane == 0) {
             sact[0] = m;
             sact[1] = 0ull;
-            gone = 0;
+            gone = resident_state(X) == kResGivenUp;
         }
     }
     for (int k = tid; k < w * h; k += nthr) {
@@ -452,6 +491,13 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
             }
         }
         lds_barrier();
+    }
+
+    if (gone) return;
+    if (!regular) {
+        if (tid == 0) gone = !resident_all_done(X);
+        __syncthreads();
+        if (gone) return;
     }
 
     // ---- the state the other paths read: the cells into the buffer that was not

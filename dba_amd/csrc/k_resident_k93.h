@@ -37,7 +37,7 @@ __global__ __launch_bounds__(1024) void k93_resident_kernel(const Inst* __restri
     __shared__ int runsT[kResMaxTiles];           // steps that ran the T set (tiles[].runs: the phi set)
     __shared__ int fire[2][3][kResMaxTiles];      // detector bits of set and step s in fire[set][s % 3]
     __shared__ int cells[kResMaxTiles];           // field-set updates
-    __shared__ int gone;                          // a wait ran out
+    __shared__ int gone;                          // the launch was given up
     __shared__ uint64_t sact[2][2];               // [s & 1][set]: awake positions of step s
     CInst& I = ((CInst*)insts)[0];
     const int tid = threadIdx.x, lane = tid & 63, nthr = blockDim.x;
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(1024) void k93_resident_kernel(const Inst* __restri
                 sact[1][q] = 0ull;
             }
         }
-        if (lane == 0) gone = 0;
+        if (lane == 0) gone = resident_state(X) == kResGivenUp;
     }
     for (int k = tid; k < w * h; k += nthr) {
         const int x = k % w, y = k / w, t = (G.ti0 + x / TB) + (G.tj0 + y / TB) * ntx;
@@ -256,6 +256,7 @@ __global__ __launch_bounds__(1024) void k93_resident_kernel(const Inst* __restri
         }
     }
     __syncthreads();
+    if (gone) return;
 
     // ---- the state the other paths read: per set the cells into the buffer that was
     //      not current (others may still read this launch's start from that one), the

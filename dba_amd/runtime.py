@@ -176,6 +176,12 @@ class Context:
         abi.check(self.lib.dba_resident_calls(self.h, C.byref(n)))
         return n.value
 
+    def resident_redone(self):
+        """Resident steps that were given up and made again on the other paths."""
+        n = C.c_int64()
+        abi.check(self.lib.dba_resident_redone(self.h, C.byref(n)))
+        return n.value
+
     def timing(self, enable):
         abi.check(self.lib.dba_timing_enable(self.h, 1 if enable else 0))
 

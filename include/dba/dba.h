@@ -218,9 +218,14 @@ dba_status dba_sync(dba_ctx* ctx);
  * A call of 12 steps or more for one reactive CH or K93 instance (threads 0, no timing) whose
  * tiles fit the GPU at once, by a context alone on its device in this process, takes
  * resident steps in modes 1 and 2: all its steps in one cooperative launch that keeps
- * the fields on chip. Processes that share a GPU take turns with such launches; set
- * mode 0 there. Should a workgroup wait in vain, the context's next synchronising call
- * returns DBA_ERR_HIP.
+ * the fields on chip. (A context that is not finalised counts as one on its device.)
+ * One process at a time has the GPU's queue for such launches; a context of another one
+ * is refused its first and keeps to the other paths.
+ * Such a launch needs all its workgroups on the GPU together. Where something else, such
+ * as another process, keeps some of them off it, the others wait for about a second
+ * (dba_set_resident_wait) and then give the launch up, which leaves the instance as it
+ * was; the next call that waits for the GPU has its steps made on the other paths, and
+ * the context keeps to those until dba_set_resident.
  * mode 0: worklist path for every group; 1 (default): single-launch steps for
  * groups of one instance; 2: also for batches. Results are bit-identical in every
  * mode. DBA_ERR_INVALID for another mode. */
@@ -235,8 +240,10 @@ dba_status dba_set_resident(dba_ctx* ctx, int32_t enable);
  * is a trip to memory, about a microsecond) before it gives the wait up; 0: the default. */
 dba_status dba_set_resident_wait(dba_ctx* ctx, int32_t polls);
 
-/* How many dba_step / dba_step_graph calls of this context took resident steps. */
+/* How many dba_step / dba_step_graph calls of this context took resident steps, and how
+ * many of their steps were given up and made again on the other paths. */
 dba_status dba_resident_calls(dba_ctx* ctx, int64_t* taken);
+dba_status dba_resident_redone(dba_ctx* ctx, int64_t* steps);
 
 /* Active tiles of a set for the NEXT step (after dilation). mask (optional)
    receives ntiles bytes, 1 = awake. Synchronises. */

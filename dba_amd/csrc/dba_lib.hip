@@ -172,10 +172,9 @@ struct dba_ctx {
     unsigned char* scratch = nullptr;  // this device's address of the scratch array
     // exchange of the resident steps: one workspace for every instance (its launches
     // follow each other on the one stream; sequence numbers never repeat)
-    uint64_t* xbuf = nullptr;
+    ResHead* xbuf = nullptr;       // the launches' state, then xwords words of frames and flags
     size_t xwords = 0;
     uint32_t xseq = 1;
-    uint32_t* xstate = nullptr;    // state of the resident launches, workgroups done (k_resident.h)
     int* stuck = nullptr;          // pinned host word: a resident launch was given up
     std::vector<int> unsettled;    // instances with resident launches since the host last waited
     bool resident = true;          // resident steps where they can be had (dba_set_resident)
@@ -1028,10 +1027,6 @@ bool resident_buffer(dba_ctx* ctx, size_t words, int n_steps) {
         if (hipHostMalloc((void**)&ctx->stuck, sizeof(int)) != hipSuccess) return false;
         *ctx->stuck = 0;
     }
-    if (!ctx->xstate) {
-        if (hipMalloc(&ctx->xstate, 2 * sizeof(uint32_t)) != hipSuccess) return false;
-        if (hipMemsetAsync(ctx->xstate, 0, 2 * sizeof(uint32_t), ctx->stream) != hipSuccess) return false;
-    }
     const bool wrap = ctx->xseq > 0xffffffffu - (uint32_t)n_steps - 2u;
     if (words <= ctx->xwords && !wrap) return true;
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
@@ -1039,11 +1034,17 @@ bool resident_buffer(dba_ctx* ctx, size_t words, int n_steps) {
         if (ctx->xbuf) (void)hipFree(ctx->xbuf);
         ctx->xbuf = nullptr;
         ctx->xwords = 0;
-        if (hipMalloc(&ctx->xbuf, words * sizeof(uint64_t)) != hipSuccess) return false;
+        if (hipMalloc(&ctx->xbuf, sizeof(ResHead) + words * sizeof(uint64_t)) != hipSuccess) {
+            ctx->xbuf = nullptr;
+            return false;
+        }
+        // (a launch given up before this that the host has not taken notice of)
+        const ResHead head{*(volatile int*)ctx->stuck ? kResGivenUp : kResRunning, 0, ctx->stuck, {}};
+        if (hipMemcpy(ctx->xbuf, &head, sizeof(head), hipMemcpyHostToDevice) != hipSuccess) return false;
         ctx->xwords = words;
     }
     ctx->xseq = 1;
-    return hipMemsetAsync(ctx->xbuf, 0, ctx->xwords * sizeof(uint64_t), ctx->stream) == hipSuccess;
+    return hipMemsetAsync(ctx->xbuf + 1, 0, ctx->xwords * sizeof(uint64_t), ctx->stream) == hipSuccess;
 }
 
 // The process's contexts on a device, after adding `d`. A context alone on its device
@@ -1083,7 +1084,8 @@ dba_status enqueue_resident(dba_ctx* ctx, Group* g, int n_steps, bool* taken) {
     if (have) {
         const void* f = resident_kernel(g, g->res_per_tile);
         const size_t lds = resident_bytes(g, gx * g->tile, gy * g->tile);
-        Exchange X{ctx->xbuf, ctx->xbuf + (words - flags), ctx->xstate, ctx->stuck, ctx->wait_polls, ctx->xseq, slots};
+        uint64_t* frames = (uint64_t*)(ctx->xbuf + 1);
+        Exchange X{frames, frames + (words - flags), ctx->wait_polls, ctx->xseq, slots};
         const Inst* insts = g->d_insts;
         int n = n_steps, ax = gx, ay = gy;
         void* args[] = {(void*)&insts, (void*)&X, (void*)&n, (void*)&ax, (void*)&ay};
@@ -1101,7 +1103,7 @@ dba_status enqueue_resident(dba_ctx* ctx, Group* g, int n_steps, bool* taken) {
     ctx->resident_calls++;
     if (!is_unsettled(ctx, h_id)) ctx->unsettled.push_back(h_id);
     *taken = true;
-    return launch_canon(ctx, g, n_steps, ctx->xstate);
+    return launch_canon(ctx, g, n_steps, &ctx->xbuf->state);
 }
 
 dba_status enqueue_steps(dba_ctx* ctx, const std::vector<Group*>& gs, int n_steps, bool timed) {
@@ -1210,7 +1212,7 @@ dba_status wait_stream(dba_ctx* ctx, bool* redone = nullptr) {
     if (!ctx->stuck || !*(volatile int*)ctx->stuck) return DBA_OK;
     *ctx->stuck = 0;
     ctx->resident = false;
-    HIP_TRY(hipMemsetAsync(ctx->xstate, 0, 2 * sizeof(uint32_t), ctx->stream));
+    HIP_TRY(hipMemsetAsync(ctx->xbuf, 0, 2 * sizeof(uint32_t), ctx->stream));  // (not the stuck pointer)
     for (int id : ids) {
         Instance* in = ctx->inst.at(id);
         int64_t ctr[4];
@@ -1349,7 +1351,6 @@ dba_status dba_finalize(dba_ctx* ctx) {
     for (auto m : ctx->markers) (void)hipEventDestroy(m);
     if (ctx->staging) (void)hipFree(ctx->staging);
     if (ctx->xbuf) (void)hipFree(ctx->xbuf);
-    if (ctx->xstate) (void)hipFree(ctx->xstate);
     if (ctx->stuck) (void)hipHostFree(ctx->stuck);
     if (ctx->d_flag) (void)hipFree(ctx->d_flag);
     if (ctx->d_diag) (void)hipFree(ctx->d_diag);

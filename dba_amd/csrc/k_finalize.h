@@ -648,7 +648,7 @@ __device__ __forceinline__ void dense_canon_finish(CInst& I, int n, unsigned lon
     I.scal[3] = dt;
 }
 
-// After a resident launch (res: its state, k_resident.h; null after single-launch
+// After a resident launch (res: its state and count, k_resident.h; null after single-launch
 // steps): whether it was given up. Then its steps are counted in ctr[3], for the host,
 // and everything else stays as it was before them.
 __device__ __forceinline__ bool resident_given_up(const uint32_t* res) { return res && res[0] == 1u; }

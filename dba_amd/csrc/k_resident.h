@@ -21,12 +21,14 @@
 // workgroups are resident unless something else holds compute units (another process);
 // a workgroup waits only for words of the step before, which their owners send without
 // waiting for anything of this step, so by induction over the steps every wait ends.
-// Each wait is bounded all the same: past the bound, or once any other wait has passed
-// it, a workgroup gives the launch up, and the host has its steps made on another path.
-// So a launch that is given up leaves the instance as it was. What it stores before its
-// end only counts once the canonicalising kernel takes it over (the cells go to the
-// buffers that are not current); what replaces state in place (the stored potential
-// rings of CH) waits until every workgroup has made all its steps (resident_all_done).
+// Each wait is bounded all the same: a workgroup past the bound gives the launch up and
+// ends; those that wait for its words run out a few steps later, those that only get a
+// place on the chip then see it as they start, and the host has the steps made on
+// another path. So a launch that is given up leaves the instance as it was. What it
+// stores before its end only counts once the canonicalising kernel takes it over (the
+// cells go to the buffers that are not current); what replaces state in place (the
+// stored potential rings of CH) waits until every workgroup has made all its steps
+// (resident_all_done).
 #pragma once
 #include "common.h"
 #include "k_ch.h"
@@ -34,14 +36,24 @@
 
 namespace dba {
 
+// State of the context's resident launches, in front of the exchange's frames (a pointer
+// of its own would be one more to keep in registers through the steps). A launch that
+// starts with kResGivenUp makes no steps: the host has not taken notice of the one before
+// it yet.
+constexpr uint32_t kResRunning = 0, kResGivenUp = 1, kResDone = 2;
+struct ResHead {
+    uint32_t state, done;  // done: workgroups that have made all their steps
+    int* stuck;            // host memory: a launch was given up
+    uint64_t pad[14];      // a cache line of its own
+};
+
 struct Exchange {
     uint64_t* frame;   // [parity][region][slot][2 words per field]
     uint64_t* flag;    // [parity][tile]: sequence number << 32 | detector bits
-    uint32_t* state;   // kRes..., and the number of workgroups that have made all their steps
-    int* stuck;        // host memory: the launch was given up
     int polls;         // polls after which a wait is given up
     uint32_t base;     // sequence number of the launch's first step
     int slots;         // frame slots of a whole region
+    __device__ __forceinline__ ResHead* head() const { return (ResHead*)frame - 1; }
 };
 
 __device__ __forceinline__ void xput(uint64_t* p, uint64_t v) {
@@ -57,10 +69,6 @@ __device__ __forceinline__ void put_double(uint64_t* p, double v, uint32_t seq) 
     xput(p + 1, s | (uint32_t)(b >> 32));
 }
 
-// State of the context's resident launches. A launch that starts in kResGivenUp makes no
-// steps: the host has not taken notice of the one before it yet.
-constexpr uint32_t kResRunning = 0, kResGivenUp = 1, kResDone = 2;
-
 // Bound of a wait, if the caller sets none: about a second of polls (each is a trip to
 // memory). Other work of the process may hold compute units that a workgroup of the
 // launch still needs, and a launch given up costs that second once: the context then
@@ -68,35 +76,26 @@ constexpr uint32_t kResRunning = 0, kResGivenUp = 1, kResDone = 2;
 constexpr int kWaitPolls = 1 << 20;
 
 __device__ __forceinline__ uint32_t resident_state(const Exchange& X) {
-    return __hip_atomic_load(X.state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __hip_atomic_load(&X.head()->state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Gives the launch up, unless it is done.
-__device__ __forceinline__ void resident_give_up(const Exchange& X) {
+__device__ __forceinline__ bool resident_end(const Exchange& X, uint32_t how) {
     uint32_t s = kResRunning;
-    if (__hip_atomic_compare_exchange_strong(X.state, &s, kResGivenUp, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT))
-        __hip_atomic_store(X.stuck, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return __hip_atomic_compare_exchange_strong(&X.head()->state, &s, how, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Called while polling: true when the wait must be given up.
-__device__ __forceinline__ bool wait_over(int polls, const Exchange& X) {
-    if (polls >= X.polls) {
-        resident_give_up(X);
-        return true;
-    }
-    return (polls & 1023) == 1023 && resident_state(X) == kResGivenUp;
+// Gives the launch up, unless it is done (one thread).
+__device__ __forceinline__ void resident_give_up(const Exchange& X) {
+    if (resident_end(X, kResGivenUp)) __hip_atomic_store(X.head()->stuck, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // One thread of a workgroup that has made all its steps: true once all workgroups have,
 // false if the launch was given up instead. Costs a trip to memory and the last
 // workgroup's lag, once per launch.
 __device__ __forceinline__ bool resident_all_done(const Exchange& X) {
-    if (__hip_atomic_fetch_add(X.state + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x) {
-        uint32_t s = kResRunning;
-        __hip_atomic_compare_exchange_strong(X.state, &s, kResDone, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (__hip_atomic_fetch_add(&X.head()->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x)
+        resident_end(X, kResDone);
     for (int k = 0;; k++) {
         const uint32_t s = resident_state(X);
         if (s != kResRunning) return s == kResDone;
@@ -104,13 +103,15 @@ __device__ __forceinline__ bool resident_all_done(const Exchange& X) {
     }
 }
 
+// A word of another workgroup. Past the bound only *gone is set: what giving up takes is
+// kept out of the loops, where its registers cost 2% of a step.
 __device__ __forceinline__ double wait_double(const uint64_t* p, uint32_t seq, const Exchange& X, int* gone) {
     uint64_t a, b;
     for (int k = 0;; k++) {
         a = xget(p);
         b = xget(p + 1);
         if ((uint32_t)(a >> 32) == seq && (uint32_t)(b >> 32) == seq) break;
-        if (wait_over(k, X)) {
+        if (k >= X.polls) {
             *gone = 1;
             break;
         }
@@ -123,7 +124,7 @@ __device__ __forceinline__ int wait_flag(const uint64_t* p, uint32_t seq, const 
     for (int k = 0;; k++) {
         a = xget(p);
         if ((uint32_t)(a >> 32) == seq) break;
-        if (wait_over(k, X)) {
+        if (k >= X.polls) {
             *gone = 1;
             break;
         }
@@ -256,7 +257,7 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
     extern __shared__ __align__(16) double lds[];
     __shared__ ResTile tiles[kResMaxTiles];
     __shared__ int fire[3][kResMaxTiles];  // detector bits of step s in fire[s % 3]
-    __shared__ int gone;                   // the launch was given up
+    __shared__ int gone[2];                // a wait of step s ran out: gone[s & 1]
     __shared__ uint64_t sact[2];           // awake tiles of step s: positions of the region and two tiles around it
     CInst& I = ((CInst*)insts)[0];
     const int tid = threadIdx.x, lane = tid & 63, nthr = blockDim.x;
@@ -296,7 +297,8 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
         if (lane == 0) {
             sact[0] = m;
             sact[1] = 0ull;
-            gone = resident_state(X) == kResGivenUp;
+            gone[0] = resident_state(X) == kResGivenUp;
+            gone[1] = 0;
         }
     }
     for (int k = tid; k < w * h; k += nthr) {
@@ -415,7 +417,7 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
         // 2. the frames of the tiles outside that ran, the detector bits around
         if (s > 0) {
             const uint64_t ran = sact[(s & 1) ^ 1];
-            if (hpos >= 0 && ((ran >> hpos) & 1ull)) sc[hcell] = wait_double(fin + hslot, seq, X, &gone);
+            if (hpos >= 0 && ((ran >> hpos) & 1ull)) sc[hcell] = wait_double(fin + hslot, seq, X, &gone[s & 1]);
             if (tid >= nthr - 64) {
                 const uint64_t exist = __ballot(near >= 0);
                 uint64_t m = exist;
@@ -424,7 +426,7 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
                     int b = 0;
                     if (near >= 0)
                         b = own_tile >= 0 ? fp[own_tile]
-                                          : wait_flag(X.flag + (int64_t)((s & 1) ^ 1) * I.nt + near, seq, X, &gone);
+                                          : wait_flag(X.flag + (int64_t)((s & 1) ^ 1) * I.nt + near, seq, X, &gone[s & 1]);
                     m = G.dilate(__ballot(b), exist);
                 }
                 if (lane == 0) sact[s & 1] = m;
@@ -432,7 +434,6 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
         }
         if (tid < kResMaxTiles) fire[(s + 1) % 3][tid] = 0;
         lds_barrier();
-        if (gone) break;  // the same in every wave: written before this barrier, and not again before two more
         const uint64_t act = sact[s & 1];
         auto runs = [&](int j) { return (act >> tiles[j].pos) & 1ull; };
         // 3. mu of tiles a neighbour woke, of the region's edge, of the ring of running tiles outside
@@ -491,13 +492,17 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
             }
         }
         lds_barrier();
+        if (gone[s & 1]) break;  // the same in every wave: the next write of this word is past the next step's barriers
     }
 
-    if (gone) return;
+    if (gone[0] | gone[1]) {
+        if (tid == 0) resident_give_up(X);
+        return;
+    }
     if (!regular) {
-        if (tid == 0) gone = !resident_all_done(X);
+        if (tid == 0) sact[0] = resident_all_done(X);
         __syncthreads();
-        if (gone) return;
+        if (!sact[0]) return;
     }
 
     // ---- the state the other paths read: the cells into the buffer that was not

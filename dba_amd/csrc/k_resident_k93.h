@@ -37,7 +37,7 @@ __global__ __launch_bounds__(1024) void k93_resident_kernel(const Inst* __restri
     __shared__ int runsT[kResMaxTiles];           // steps that ran the T set (tiles[].runs: the phi set)
     __shared__ int fire[2][3][kResMaxTiles];      // detector bits of set and step s in fire[set][s % 3]
     __shared__ int cells[kResMaxTiles];           // field-set updates
-    __shared__ int gone;                          // the launch was given up
+    __shared__ int gone[2];                       // a wait of step s ran out: gone[s & 1]
     __shared__ uint64_t sact[2][2];               // [s & 1][set]: awake positions of step s
     CInst& I = ((CInst*)insts)[0];
     const int tid = threadIdx.x, lane = tid & 63, nthr = blockDim.x;
@@ -79,7 +79,10 @@ __global__ __launch_bounds__(1024) void k93_resident_kernel(const Inst* __restri
                 sact[1][q] = 0ull;
             }
         }
-        if (lane == 0) gone = resident_state(X) == kResGivenUp;
+        if (lane == 0) {
+            gone[0] = resident_state(X) == kResGivenUp;
+            gone[1] = 0;
+        }
     }
     for (int k = tid; k < w * h; k += nthr) {
         const int x = k % w, y = k / w, t = (G.ti0 + x / TB) + (G.tj0 + y / TB) * ntx;
@@ -165,8 +168,8 @@ __global__ __launch_bounds__(1024) void k93_resident_kernel(const Inst* __restri
                 const uint64_t* q = fin + hslot;
                 const bool wp = (sact[(s & 1) ^ 1][0] >> hpos) & 1ull;
                 const bool wT = hT >= 0 && ((sact[(s & 1) ^ 1][1] >> hpos) & 1ull);
-                if (wp) sp[hphi] = wait_double(q, seq, X, &gone);
-                if (wT) sT[hT] = wait_double(q + 2, seq, X, &gone);
+                if (wp) sp[hphi] = wait_double(q, seq, X, &gone[s & 1]);
+                if (wT) sT[hT] = wait_double(q + 2, seq, X, &gone[s & 1]);
             }
             if (tid >= nthr - 64) {
                 const uint64_t exist = __ballot(near >= 0);
@@ -174,7 +177,7 @@ __global__ __launch_bounds__(1024) void k93_resident_kernel(const Inst* __restri
                 if (!regular) {
                     int f = 0;
                     if (own >= 0) f = fire[0][prev][own] | fire[1][prev][own] << 1;
-                    else if (near >= 0) f = wait_flag(X.flag + (int64_t)((s & 1) ^ 1) * nt + near, seq, X, &gone);
+                    else if (near >= 0) f = wait_flag(X.flag + (int64_t)((s & 1) ^ 1) * nt + near, seq, X, &gone[s & 1]);
                     a = G.dilate(__ballot(f & 1), exist);
                     b = G.dilate(__ballot(f & 2), exist);
                 }
@@ -186,7 +189,6 @@ __global__ __launch_bounds__(1024) void k93_resident_kernel(const Inst* __restri
         }
         if (tid < kResMaxTiles) fire[0][(s + 1) % 3][tid] = fire[1][(s + 1) % 3][tid] = 0;
         lds_barrier();
-        if (gone) break;  // the same in every wave: written before this barrier, and not again before two more
         const uint64_t actp = sact[s & 1][0], actT = sact[s & 1][1];
         // 3. the rest
         const bool ap = in && ((actp >> pos) & 1ull), aT = in && ((actT >> pos) & 1ull);
@@ -254,9 +256,13 @@ __global__ __launch_bounds__(1024) void k93_resident_kernel(const Inst* __restri
                 }
             }
         }
+        if (gone[s & 1]) break;  // the same in every wave: the next write of this word is past the next step's barriers
     }
     __syncthreads();
-    if (gone) return;
+    if (gone[0] | gone[1]) {
+        if (tid == 0) resident_give_up(X);
+        return;
+    }
 
     // ---- the state the other paths read: per set the cells into the buffer that was
     //      not current (others may still read this launch's start from that one), the

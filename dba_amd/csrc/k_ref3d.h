@@ -272,23 +272,36 @@ __device__ __forceinline__ int64_t mb_own_index(const MbBlock& b, int lane) {
 
 // The chemical potentials of a cell (example_Reactive_ModelB/kernel.cu:557-587)
 // from x, y, z, phi, the logarithms and the three Laplacians, in parts: what the
-// three share (the solvent's terms), then each one's own.
+// three share (the solvent's terms), then each one's own. The quotients by r_x, r_y,
+// r_z and 1 - z_crit are rounded to nearest, from reciprocals the host takes once.
+// FIN: the logarithms are finite.
+template <bool FIN>
+__device__ __forceinline__ double mb_over(double a, double b, double y) {
+    return FIN ? quotient(a, b, y) : quotient_any(a, b, y);
+}
+
 __device__ __forceinline__ double mb_shared(CInst& I, double X, double Y, double Z, double logB) {
     return -(I.chi_xb * X + I.chi_yb * Y + I.chi_zb * Z) - logB;
 }
 
+template <bool FIN>
 __device__ __forceinline__ double mb_mu_x(CInst& I, double Y, double Z, double B, double com, double logX, double lap) {
-    return (I.mb_cx + I.chi_xy * Y + I.chi_xz * Z + I.chi_xb * B + com + logX * I.mb_irx) - I.epsx_sq * lap;
+    return (I.mb_cx + I.chi_xy * Y + I.chi_xz * Z + I.chi_xb * B + com + mb_over<FIN>(logX, I.r_x, I.mb_irx)) -
+           I.epsx_sq * lap;
 }
 
+template <bool FIN>
 __device__ __forceinline__ double mb_mu_y(CInst& I, double X, double Z, double B, double com, double logY, double lap) {
-    return (I.mb_cy + I.chi_xy * X + I.chi_yz * Z + I.chi_yb * B + com + logY * I.mb_iry) - I.epsy_sq * lap;
+    return (I.mb_cy + I.chi_xy * X + I.chi_yz * Z + I.chi_yb * B + com + mb_over<FIN>(logY, I.r_y, I.mb_iry)) -
+           I.epsy_sq * lap;
 }
 
+template <bool FIN>
 __device__ __forceinline__ double mb_mu_z(CInst& I, double X, double Y, double B, double com, double logZ, double lap,
                                           double phi) {
-    return (I.mb_cz + I.chi_xz * X + I.chi_yz * Y + I.chi_zb * B + com + logZ * I.mb_irz -
-            I.p_gel * phi * phi * I.mb_hiomz) - I.epsz_sq * lap - I.mb_lk;
+    const double gel = quotient_any(0.5 * (I.p_gel * phi * phi), I.mb_omz, I.mb_iomz);
+    return (I.mb_cz + I.chi_xz * X + I.chi_yz * Y + I.chi_zb * B + com + mb_over<FIN>(logZ, I.r_z, I.mb_irz) - gel) -
+           I.epsz_sq * lap - I.mb_lk;
 }
 
 // The changes of x, y, z of a cell (example_Reactive_ModelB/kernel.cu:419-432):
@@ -320,9 +333,9 @@ __device__ __forceinline__ double mb_mu_at(CInst& I, const double* sc, int cx, i
     const double lz_ = lds_lap27<RX, PZ>(sc + 2 * AP, cx, cy, cz, inv_dx2);
     __builtin_amdgcn_sched_barrier(0);
     const double com = mb_shared(I, X, Y, Z, logB);
-    df[0] = mb_mu_x(I, Y, Z, B, com, logX, lx_);
-    df[1] = mb_mu_y(I, X, Z, B, com, logY, ly_);
-    df[2] = mb_mu_z(I, X, Y, B, com, logZ, lz_, phi);
+    df[0] = mb_mu_x<false>(I, Y, Z, B, com, logX, lx_);
+    df[1] = mb_mu_y<false>(I, X, Z, B, com, logY, ly_);
+    df[2] = mb_mu_z<false>(I, X, Y, B, com, logZ, lz_, phi);
     return lz_;
 }
 
@@ -833,17 +846,17 @@ __global__ __launch_bounds__(MbMarch::NT) __attribute__((amdgpu_waves_per_eu(CON
                     // one logarithm at a time: together they spill
                     const double com = mb_shared(I, X, Y, Z, log_positive(B));
                     __builtin_amdgcn_sched_barrier(0);
-                    df[0] = mb_mu_x(I, Y, Z, B, com, log_positive(X), lap[0]);
+                    df[0] = mb_mu_x<true>(I, Y, Z, B, com, log_positive(X), lap[0]);
                     __builtin_amdgcn_sched_barrier(0);
-                    df[1] = mb_mu_y(I, X, Z, B, com, log_positive(Y), lap[1]);
+                    df[1] = mb_mu_y<true>(I, X, Z, B, com, log_positive(Y), lap[1]);
                     __builtin_amdgcn_sched_barrier(0);
-                    df[2] = mb_mu_z(I, X, Y, B, com, log_positive(Z), lap[2], phi);
+                    df[2] = mb_mu_z<true>(I, X, Y, B, com, log_positive(Z), lap[2], phi);
                     __builtin_amdgcn_sched_barrier(0);
                 } else {
                     const double com = mb_shared(I, X, Y, Z, log_f64(B));
-                    df[0] = mb_mu_x(I, Y, Z, B, com, log_f64(X), lap[0]);
-                    df[1] = mb_mu_y(I, X, Z, B, com, log_f64(Y), lap[1]);
-                    df[2] = mb_mu_z(I, X, Y, B, com, log_f64(Z), lap[2], phi);
+                    df[0] = mb_mu_x<false>(I, Y, Z, B, com, log_f64(X), lap[0]);
+                    df[1] = mb_mu_y<false>(I, X, Z, B, com, log_f64(Y), lap[1]);
+                    df[2] = mb_mu_z<false>(I, X, Y, B, com, log_f64(Z), lap[2], phi);
                 }
             } else {
                 const int64_t zo = (int64_t)zof(p - 1) * nxy;
@@ -1085,11 +1098,11 @@ __global__ __launch_bounds__(MbMarch::NT) __attribute__((amdgpu_waves_per_eu(4))
         const double X = c[0], Y = c[1], Z = c[2], B = 1.0 - X - Y - Z;
         const double com = mb_shared(I, X, Y, Z, log_f64(B));
         __builtin_amdgcn_sched_barrier(0);
-        df[0] = mb_mu_x(I, Y, Z, B, com, log_f64(X), lap[0]);
+        df[0] = mb_mu_x<false>(I, Y, Z, B, com, log_f64(X), lap[0]);
         __builtin_amdgcn_sched_barrier(0);
-        df[1] = mb_mu_y(I, X, Z, B, com, log_f64(Y), lap[1]);
+        df[1] = mb_mu_y<false>(I, X, Z, B, com, log_f64(Y), lap[1]);
         __builtin_amdgcn_sched_barrier(0);
-        df[2] = mb_mu_z(I, X, Y, B, com, log_f64(Z), lap[2], phi);
+        df[2] = mb_mu_z<false>(I, X, Y, B, com, log_f64(Z), lap[2], phi);
         __builtin_amdgcn_sched_barrier(0);
     }
     double* sm = S.mu + mx + my * M::MW;

@@ -1,4 +1,4 @@
-// mathf64.h - FP64 natural logarithm for the Model B chemical potentials.
+// mathf64.h - FP64 natural logarithm and quotients for the Model B chemical potentials.
 //
 // The device library's log carries double-double corrections (about 90 VALU
 // instructions on gfx950); the potentials take four logarithms per cell, which
@@ -45,6 +45,22 @@ DBA_HD inline double log_quotient(double f, double b) {
 #else
     return f / b;
 #endif
+}
+
+// a / b for a constant b with y = 1 / b rounded to nearest: the product, corrected once by
+// its exact remainder. The product alone is up to 1.5 ulp off; this is the quotient
+// rounded to nearest (but for quotients within 2^-51 ulp of a tie). Two operations more
+// than the product where a division is a dozen. For finite quotients and remainders
+// above the subnormals.
+DBA_HD inline double quotient(double a, double b, double y) {
+    const double q = a * y;
+    return std::fma(std::fma(-b, q, a), y, q);
+}
+
+// ... and an infinite or NaN quotient as the product gives it.
+DBA_HD inline double quotient_any(double a, double b, double y) {
+    const double q = a * y, c = std::fma(std::fma(-b, q, a), y, q);
+    return std::fabs(q) < INFINITY ? c : q;
 }
 
 // A constant of the series. On the device it is put into scalar registers where it

@@ -558,9 +558,9 @@ dba_status get_group(dba_ctx* ctx, const std::vector<int>& ids, Group** out) {
     int64_t cap = g->model == DBA_MODEL_MODELB ? 65536 : (g->model == DBA_MODEL_DENDRITE_K94 ? 20 * ctx->n_cu : 4096);
     g->grid = (int)std::max<int64_t>(1, std::min<int64_t>(g->total_tiles, cap));
     // Model B column march (modelb_march_kernel, nz == 1: modelb_plane_kernel): one
-    // instance, steps whose list is long enough. DBA_MODELB_SUPERBLOCKS=0 turns it off
-    // and =1 uses it for every non-empty list (both give the same doubles). Layers per
-    // strip: the fewest rounds of resident workgroups, each round 4 nl + 4 planes long.
+    // instance, steps whose list is long enough. DBA_MODELB_SUPERBLOCKS set to a number
+    // is the shortest list that takes it (0: none does); all give the same doubles. Layers
+    // per strip: the fewest rounds of resident workgroups, each round 4 nl + 4 planes long.
     if (g->model == DBA_MODEL_MODELB && ids.size() == 1 && g->tile == 4) {
         const Inst& h = first->h;
         if (h.full_tiles && (h.nz > 1) == (g->tile_z == 4) && (int64_t)h.nx * h.ny < (1 << 28)) {
@@ -591,8 +591,8 @@ dba_status get_group(dba_ctx* ctx, const std::vector<int>& ids, Group** out) {
             // nothing awake does its one workgroup per column cost more (2048^2 at 1% 63
             // and 42, 4096^2 at 0.6% 79 and 109, at 5% 214 and 122).
             int64_t from = h.nz > 1 ? planes * (g->conserved ? 550 : 1000) : (cols <= 8 * slots ? 1 : cols * 2 / 5);
-            if (e == "0" || from > h.nt) from = 0;
-            if (e == "1") from = 1;
+            if (!e.empty() && e.find_first_not_of("0123456789") == std::string::npos) from = std::atoll(e.c_str());
+            if (from > h.nt) from = 0;
             g->march_from = (int)from;
             // the block kernels then only take lists shorter than that, and return at once
             // from the others (160 x 160 x 100, all awake: 20000 workgroups 4 us more per

@@ -379,7 +379,8 @@ __device__ __forceinline__ bool kh_tile(const KhItem& it, const KhStep& c, KhLds
         const int k0 = (tx + 2) + (ty + 2) * W2;
 #pragma unroll
         for (int q = 0; q < 4; q++) sP[q * A2 + k0] = w[q];
-        if (cfl) vstale = kh_wave_speed<FAST>(c, w);  // the speed at the start of the step
+        // the speed at the start of the step; one that is no number does not count
+        if (cfl) vstale = fmax(0.0, kh_wave_speed<FAST>(c, w));
     }
 #pragma unroll
     for (int j = 0; j < H::HK; j++) {
@@ -582,7 +583,7 @@ __device__ __forceinline__ bool kh_tile(const KhItem& it, const KhStep& c, KhLds
             vfresh = kh_wave_speed<FAST>(c, w);
         } else {
             kh_prim<P2, false>(c, U, w);
-            vfresh = kh_wave_speed<false>(c, w);
+            vfresh = fmax(0.0, kh_wave_speed<false>(c, w));
         }
     }
     return true;

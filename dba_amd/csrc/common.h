@@ -318,13 +318,6 @@ __device__ __forceinline__ double block_max(double v, double* lds_scratch) {
     return r;
 }
 
-// Map a grid-stride round-robin block index so that consecutive worklist
-// items land on the same XCD (workgroups are dealt to the 8 XCDs in turn).
-__device__ __forceinline__ int xcd_remap(int b, int G) {
-    if ((G & 7) != 0) return b;
-    return (b & 7) * (G >> 3) + (b >> 3);
-}
-
 // A worklist segment: up to kSegTiles consecutive tiles of one instance. The
 // finalize kernel compacts each segment into inst.seg[tile0 ...]; offsets is
 // the exclusive prefix of the segment counts.

@@ -596,7 +596,7 @@ __global__ __launch_bounds__(256) void ch_march_kernel(const Inst* __restrict__ 
             const gu8 *F, *P;
             dense_bytes(I, prev, &F, &P);
             par = P[o];
-            if (!regular) act = dilated2d(F, oi, oj, ntx, nb2_of(oi, oj, ntx, nty, 0, 0), 0);
+            if (!regular) act = dilated2d(F, oi, oj, ntx, nb2_of(oi, oj, ntx, nty, 0, 0));
         }
         s_tile[tid] = o;
         s_par[tid] = par;

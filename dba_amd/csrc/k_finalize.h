@@ -14,9 +14,11 @@
 //   (c) compacts the segment's union awake set into an ascending list
 //       (popcount prefix over the segment's words, then the lane's rank in
 //       its word), i.e. the order copy_if over tile indices gives;
-//   (d) the last workgroup to finish reduces the segment partials per
-//       instance in segment order (history, counters, conserved shift, KH CFL
-//       dt) and writes the exclusive prefix of the segment counts.
+//   (d) of a one-segment group, updates the instance (history, counters, conserved
+//       shift, KH CFL dt); of several segments it leaves partial sums and counts,
+//       which a merge launch sums per instance in segment order and scans into the
+//       list's offsets, or, where no step needs the sums of the one before, which the
+//       next step's kernel scans and the next finalize sums (folded merges, common.h).
 #pragma once
 #include "common.h"
 
@@ -49,19 +51,16 @@ __device__ __forceinline__ Nb2 nb2_of(int ti, int tj, int ntx, int nty, int bcx,
     return n;
 }
 
-// Awake flag of tile (ti, tj) for the next step: OR of the detector bytes over the
-// tile and its neighbours (kind 0: faces; kind 1: 3x3).
-__device__ __forceinline__ int dilated2d(const gu8* N, int ti, int tj, int ntx, const Nb2& n, int kind) {
-    // A missing neighbour (zero-flux or wall boundary) reads the tile itself
-    // instead, which the OR already holds (a missing corner falls back to the
-    // edge neighbour that exists, or to the tile): no load depends on a branch,
-    // so all of them are in flight at once instead of one after another.
+// Awake flag of tile (ti, tj) for the next step (CH, K93): OR of the detector bytes
+// over the tile and its face neighbours.
+__device__ __forceinline__ int dilated2d(const gu8* N, int ti, int tj, int ntx, const Nb2& n) {
+    // A missing neighbour (zero-flux boundary) reads the tile itself instead, which
+    // the OR already holds: no load depends on a branch, so all of them are in flight
+    // at once instead of one after another.
     const int xm = n.xm >= 0 ? n.xm : ti, xp = n.xp >= 0 ? n.xp : ti;
     const int ym = n.ym >= 0 ? n.ym : tj, yp = n.yp >= 0 ? n.yp : tj;
     const int row = tj * ntx, rm = ym * ntx, rp = yp * ntx;
-    int r = N[ti + row] | N[xm + row] | N[xp + row] | N[ti + rm] | N[ti + rp];
-    if (kind == 1) r |= N[xm + rm] | N[xp + rm] | N[xm + rp] | N[xp + rp];
-    return r != 0;
+    return (N[ti + row] | N[xm + row] | N[xp + row] | N[ti + rm] | N[ti + rp]) != 0;
 }
 
 template <int NT>
@@ -558,7 +557,7 @@ __device__ __forceinline__ void dense_nb_fill(NbTable& nb, CInst& I, int t, int 
         dense_bytes(I, prev, &F, &P);
         for (int s = 0; s < nsets; s++) par[s] = P[s * nt + o];
         if (!regular)
-            for (int s = 0; s < nsets; s++) act[s] = dilated2d(F + s * nt, oi, oj, ntx, n, 0);
+            for (int s = 0; s < nsets; s++) act[s] = dilated2d(F + s * nt, oi, oj, ntx, n);
     }
     for (int s = 0; s < nsets; s++) {
         nb.par[s][d] = par[s];
@@ -601,7 +600,7 @@ __device__ __forceinline__ void dense_canon_seg(CInst& I, int t0, int ntile, int
         const int so = s < nsets ? s * nt : 0;
         fv[s] = F[so + tc];
         pv[s] = P[so + tc];
-        av[s] = regular ? 1 : dilated2d(F + so, ti, tj, ntx, nbr, 0);
+        av[s] = regular ? 1 : dilated2d(F + so, ti, tj, ntx, nbr);
     }
     const int r = valid ? r0 : 0;
     uint64_t wa = 0ull;

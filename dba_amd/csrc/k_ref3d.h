@@ -1,5 +1,5 @@
 // k_ref3d.h - fused DBA steps of the reference's own 3D models on 4x4x4
-// activation blocks (4x4x1 when nz == 1), one wave64 per block, periodic.
+// activation blocks (4x4x1 when nz == 1), periodic.
 //
 //  * Kobayashi-94 dendrite: Evolve_p(_wakeup) + Evolve_T(_wakeup) + the detector
 //    of Wakeup_Next (example_Dendritic_growth/kernel.cu:181-293, 322-574):
@@ -9,58 +9,14 @@
 //    |lap z| > eps, then Update(_wakeup) + copy-back (example_Reactive_ModelB/
 //    kernel.cu:290-763), conserved change capture (example_Reactive_ModelB/
 //    Conserved/kernel.cu:630-702). The chemical potentials of sleeping
-//    neighbours are the ones they stored when they last ran.
+//    neighbours are the ones they stored when they last ran. Three ways: short lists
+//    take two launches with one wave64 per block, longer ones a march up columns of
+//    blocks, grids of one plane a kernel of their own.
 #pragma once
 #include "common.h"
 #include "mathf64.h"
 
 namespace dba {
-
-struct NbTable3 {
-    int tile[27];
-    int par[2][27];
-    int act[2][27];
-    double shift[kMaxFields][27];
-};
-
-template <int TB, int TZ>
-__device__ __forceinline__ void nb_fill3(NbTable3& nb, CInst& I, int x0, int y0, int z0, bool regular,
-                                         int nsets, int ncons) {
-    const int d = threadIdx.x;
-    if (d >= 27) return;
-    const int dx = d % 3 - 1, dy = (d / 3) % 3 - 1, dz = d / 9 - 1;
-    const int rx = dx < 0 ? x0 - 1 : (dx > 0 ? x0 + TB : x0);
-    const int ry = dy < 0 ? y0 - 1 : (dy > 0 ? y0 + TB : y0);
-    const int rz = dz < 0 ? z0 - 1 : (dz > 0 ? z0 + TZ : z0);
-    const int mx = map_index(rx, I.nx, 0), my = map_index(ry, I.ny, 0), mz = map_index(rz, I.nz, 0);
-    const int tt = mx / TB + (my / TB) * I.ntx + (mz / TZ) * I.ntx * I.nty;
-    nb.tile[d] = tt;
-    // both sets' bitmap words loaded together (a one-set instance reads set 0
-    // twice), from pointers selected out of one scalar batch, so no load waits
-    // on a branch or on a pointer load of its own
-    const gu64 *par0 = I.par[0], *par1 = I.par[1], *cur0 = I.a_cur[0], *cur1 = I.a_cur[1];
-    asm volatile("" : "+s"(par0), "+s"(par1), "+s"(cur0), "+s"(cur1));
-    const bool two = nsets > 1;
-    const uint64_t wp0 = par0[tt >> 6], wp1 = (two ? par1 : par0)[tt >> 6];
-    const uint64_t wa0 = cur0[tt >> 6], wa1 = (two ? cur1 : cur0)[tt >> 6];
-    const int b = tt & 63;
-    nb.par[0][d] = (int)((wp0 >> b) & 1ull);
-    nb.act[0][d] = regular ? 1 : (int)((wa0 >> b) & 1ull);
-    if (two) {
-        nb.par[1][d] = (int)((wp1 >> b) & 1ull);
-        nb.act[1][d] = regular ? 1 : (int)((wa1 >> b) & 1ull);
-    }
-    const int p0 = (int)((wp0 >> b) & 1ull);
-    for (int f = 0; f < kMaxFields; f++)
-        nb.shift[f][d] = f < ncons ? (I.scal[8 + f] - I.s_tile[((int64_t)f * 2 + p0) * I.nt + tt]) : 0.0;
-}
-
-// 3D wrap of a small periodic offset
-__device__ __forceinline__ int wrapi(int i, int n) {
-    while (i < 0) i += n;
-    while (i >= n) i -= n;
-    return i;
-}
 
 // 27-point isotropic Laplacian (the weights of example_Reactive_ModelB/kernel.cu:
 // 333-344) from three planes: with c the centre of a plane, e its four edge
@@ -101,7 +57,7 @@ __device__ __forceinline__ int nb_dir3(int lx, int ly, int lz) {
     return a + 3 * b + 9 * c;
 }
 
-// ------------------------------------------------------------ Model B (ternary)
+// ------------------------------------------------------------ Model B (ternary), block kernels
 // Two launches per step, like the reference's Calc_mu / Update pair: the first
 // computes the chemical potentials of every awake block's own cells into the
 // stored-mu arrays (aux 0..2), the second updates x, y, z from the potentials

@@ -31,7 +31,8 @@ Workloads (--workload):
             of 256 MB - 2 GB FP64 arrays move on this GPU, the yardstick for
             the step kernels' achieved bandwidth.
 A step is one DBA time step of the whole instance (stencil kernel + finalize
-kernel), replayed from a captured hipGraph. Inputs are resident in HBM before
+kernel), replayed from a captured hipGraph or, for one instance that fits the chip,
+made with all the others of its call in one resident launch. Inputs are resident in HBM before
 the timed region. value = active cell-updates/s over the timed steps (device
 counter of cells in awake tiles).
 
@@ -53,9 +54,11 @@ same process after the default one (--no-companions skips them).
 roofline: the step kernel's algorithmic bytes per launch (B_alg x active cells
 of that launch: CH fused pass 16 B = read c + write c'; dendrite 16 B per (cell,
 field) update; KH 64 B = read and write the 4 conserved fields) over its average
-duration. One launch per step (single-launch steps): the GPU time per step of a
-separate graph-replayed run of at least --timing-steps steps, between hipEvents
-on the library stream. Two launches per step: hipEvents around every step
+duration. Resident steps (all steps of the timed call in one launch): the GPU time
+of the timed call over its steps; "long_run" has the same of one call of at least
+--timing-steps steps. One launch per step (single-launch steps): the GPU time per
+step of a separate graph-replayed run of at least --timing-steps steps, between
+hipEvents on the library stream. Two launches per step: hipEvents around every step
 kernel in an eager pass.
 cpu_baseline: the oracle's regular-mode loop on a bounded sample of the same
 grid: serial, y-slab threads on the job's CPU share, and for CH the MPI slab
@@ -579,6 +582,7 @@ def measure(ctx, workload, K, W, chunk_cap, timing_steps, single_launch, n=None,
     info0 = inst.info()
     u0 = info0.cell_updates
     single = bool(info0.single_launch)
+    resident0 = ctx.resident_calls()
     ctx.marker(0)
     t0 = time.perf_counter()
     inst.step(K, graph_chunk=chunk)
@@ -586,6 +590,7 @@ def measure(ctx, workload, K, W, chunk_cap, timing_steps, single_launch, n=None,
     ctx.sync()
     t1 = time.perf_counter()
     u1 = inst.info().cell_updates
+    resident = ctx.resident_calls() > resident0   # the timed call was one resident launch
     if warm is not None:
         warm.destroy()
     gpu_ms = ctx.elapsed_ms(0, 1)
@@ -594,8 +599,8 @@ def measure(ctx, workload, K, W, chunk_cap, timing_steps, single_launch, n=None,
     value = active_updates / wall_s
     active_frac = active_updates / (K * ncell)
 
-    # kernel time of a long graph-replayed run (the host enqueues every replay
-    # before the first ends, so no launch latency sits between the two events)
+    # GPU time of a long run (one call: graph replays that the host enqueues before the
+    # first ends, or one resident launch), between two events at its ends
     reps = max(1, -(-timing_steps // chunk))
     u4 = inst.info().cell_updates
     ctx.marker(2)
@@ -619,17 +624,28 @@ def measure(ctx, workload, K, W, chunk_cap, timing_steps, single_launch, n=None,
     inst.destroy()
 
     eager_k_s = k_ms / 1e3 / max(1, k_n)
-    if single:
-        # one launch per step: the kernel's duration is the GPU time per step of
-        # a long graph-replayed run (hipEvents at its two ends; it also holds one
+    long_run = None
+    if resident:
+        # all steps of a call in one launch: the GPU time of the timed call itself, its
+        # worklist and state-restoring launches included; a longer call beside it
+        avg_k_s = gpu_ms / 1e3 / K
+        cells_per_launch = active_updates / K
+        timed_launches = 1
+        kernel = f"resident steps: {K} steps in one launch, with the launches before and after it (per step)"
+        long_run = {"steps": replay_steps, "us_per_step": replay_ms * 1e3 / replay_steps,
+                    "frac": w["b_alg"] * (u5 - u4) / (replay_ms / 1e3) / 1e9 / HBM_PEAK_GBS}
+    elif single:
+        # one launch per step: the GPU time per step of the long run (it also holds one
         # state-restoring launch per graph chunk and the gaps between launches)
         avg_k_s = replay_ms / 1e3 / replay_steps
         cells_per_launch = (u5 - u4) / replay_steps
-        kernel = "single-launch or resident step kernel (awake sets + fused stencil + detector)"
+        timed_launches = replay_steps
+        kernel = "single-launch step kernel (awake sets + fused stencil + detector)"
     else:
         # two launches per step: hipEvents around every step kernel in an eager pass
         avg_k_s = eager_k_s
         cells_per_launch = (u3 - u2) / max(1, k_n)
+        timed_launches = k_n
         kernel = "step kernel (fused stencil + detector)"
     bytes_per_launch = w["b_alg"] * cells_per_launch
     achieved = bytes_per_launch / avg_k_s / 1e9
@@ -669,9 +685,11 @@ def measure(ctx, workload, K, W, chunk_cap, timing_steps, single_launch, n=None,
             "avg_kernel_us": avg_k_s * 1e6,
             "eager_kernel_us": eager_k_s * 1e6,
             "avg_finalize_us": f_ms * 1e3 / max(1, f_n),
-            "launches_timed": K if single else k_n,
+            "launches_timed": timed_launches,
         },
     }
+    if long_run:
+        out["roofline"]["long_run"] = long_run
     return out
 
 

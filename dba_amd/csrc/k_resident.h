@@ -91,15 +91,18 @@ __device__ __forceinline__ void resident_give_up(const Exchange& X) {
 }
 
 // One thread of a workgroup that has made all its steps: true once all workgroups have,
-// false if the launch was given up instead. Costs a trip to memory and the last
-// workgroup's lag, once per launch.
-__device__ __forceinline__ bool resident_all_done(const Exchange& X) {
-    if (__hip_atomic_fetch_add(&X.head()->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x)
-        resident_end(X, kResDone);
+// false if the launch was given up instead. A workgroup that has nothing to hold back
+// does not wait (the wait cost a 20-step call 3 us: a trip to memory and the last one's lag).
+__device__ __forceinline__ bool resident_all_done(const Exchange& X, bool wait) {
+    __hip_atomic_fetch_add(&X.head()->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!wait) return true;
     for (int k = 0;; k++) {
         const uint32_t s = resident_state(X);
         if (s != kResRunning) return s == kResDone;
-        if (k >= X.polls) resident_give_up(X);
+        if (__hip_atomic_load(&X.head()->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x)
+            resident_end(X, kResDone);
+        else if (k >= X.polls)
+            resident_give_up(X);
     }
 }
 
@@ -500,7 +503,10 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
         return;
     }
     if (!regular) {
-        if (tid == 0) sact[0] = resident_all_done(X);
+        // rings to store: of tiles that ran but did not fire when they last did
+        bool rings = false;
+        for (int j = 0; j < nk; j++) rings |= tiles[j].runs > 0 && !tiles[j].last;
+        if (tid == 0) sact[0] = resident_all_done(X, rings);
         __syncthreads();
         if (!sact[0]) return;
     }

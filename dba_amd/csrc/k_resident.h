@@ -437,6 +437,8 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
         }
         if (tid < kResMaxTiles) fire[(s + 1) % 3][tid] = 0;
         lds_barrier();
+        // the same in every wave: the next write of this word is past the next step's barriers
+        const int quit = gone[s & 1];
         const uint64_t act = sact[s & 1];
         auto runs = [&](int j) { return (act >> tiles[j].pos) & 1ull; };
         // 3. mu of tiles a neighbour woke, of the region's edge, of the ring of running tiles outside
@@ -495,7 +497,7 @@ __global__ __launch_bounds__(1024) void ch_resident_kernel(const Inst* __restric
             }
         }
         lds_barrier();
-        if (gone[s & 1]) break;  // the same in every wave: the next write of this word is past the next step's barriers
+        if (quit) break;
     }
 
     if (gone[0] | gone[1]) {

@@ -65,7 +65,7 @@ struct Inst {
     double invdx2, inv6dx2, inv2dx, dt_tau, alpha_pi, cos_jt0, sin_jt0, k_epsp;
     double k94_f0, k94_f1, k94_f2, k94_f3;  // K94: 1 / (2 dx), 1 / dx / dx, -alpha / 3.14159, 1 / tau
     double mb_cx, mb_cy, mb_cz, mb_lk;  // Model B: -1 + 1/r_x.., log(k_eq)/r_z
-    double mb_irx, mb_iry, mb_irz, mb_omz, mb_iomz;  // ... 1/r_x.., 1 - z_crit, 1 / (1 - z_crit)
+    double mb_irx, mb_iry, mb_irz, mb_gel;  // ... 1/r_x.., p_gel / (2 (1 - z_crit))
     // model constants
     double tau, eps_bar, delta, alpha, gamma, theta0, latent_k, t_eq;
     double mobility, kappa, react_gamma, cbar;

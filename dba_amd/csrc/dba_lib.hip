@@ -209,8 +209,7 @@ void derive_constants(const dba_params& p, Inst& h) {
     h.mb_irx = 1.0 / p.r_x;
     h.mb_iry = 1.0 / p.r_y;
     h.mb_irz = 1.0 / p.r_z;
-    h.mb_omz = 1.0 - p.z_crit;
-    h.mb_iomz = 1.0 / h.mb_omz;
+    h.mb_gel = 0.5 * p.p_gel / (1.0 - p.z_crit);
 }
 
 dba_status validate(const dba_params& p) {

@@ -228,9 +228,10 @@ __device__ __forceinline__ int64_t mb_own_index(const MbBlock& b, int lane) {
 
 // The chemical potentials of a cell (example_Reactive_ModelB/kernel.cu:557-587)
 // from x, y, z, phi, the logarithms and the three Laplacians, in parts: what the
-// three share (the solvent's terms), then each one's own. The quotients by r_x, r_y,
-// r_z and 1 - z_crit are rounded to nearest, from reciprocals the host takes once.
-// FIN: the logarithms are finite.
+// three share (the solvent's terms), then each one's own. The quotients by r_x, r_y and
+// r_z are rounded to nearest, from reciprocals the host takes once; the constant of the
+// gel term is one quotient on the host, so the term rounds three times, as
+// p_gel phi phi / (2 (1 - z_crit)) does. FIN: the logarithms are finite.
 template <bool FIN>
 __device__ __forceinline__ double mb_over(double a, double b, double y) {
     return FIN ? quotient(a, b, y) : quotient_any(a, b, y);
@@ -255,9 +256,8 @@ __device__ __forceinline__ double mb_mu_y(CInst& I, double X, double Z, double B
 template <bool FIN>
 __device__ __forceinline__ double mb_mu_z(CInst& I, double X, double Y, double B, double com, double logZ, double lap,
                                           double phi) {
-    const double gel = quotient_any(0.5 * (I.p_gel * phi * phi), I.mb_omz, I.mb_iomz);
-    return (I.mb_cz + I.chi_xz * X + I.chi_yz * Y + I.chi_zb * B + com + mb_over<FIN>(logZ, I.r_z, I.mb_irz) - gel) -
-           I.epsz_sq * lap - I.mb_lk;
+    return (I.mb_cz + I.chi_xz * X + I.chi_yz * Y + I.chi_zb * B + com + mb_over<FIN>(logZ, I.r_z, I.mb_irz) -
+            I.mb_gel * phi * phi) - I.epsz_sq * lap - I.mb_lk;
 }
 
 // The changes of x, y, z of a cell (example_Reactive_ModelB/kernel.cu:419-432):

@@ -1,5 +1,5 @@
 """CPU: the quotients by constants of dba_amd/csrc/mathf64.h (Model B's logarithms over
-r_x, r_y, r_z and its gel term over 1 - z_crit), compiled as plain C++.
+r_x, r_y, r_z), compiled as plain C++.
 
 Bar: the correctly rounded quotient, bit for bit, as a division gives it. The product
 with the reciprocal alone, which is one rounding more, has to fail the same bar."""

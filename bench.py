@@ -55,8 +55,8 @@ roofline: the step kernel's algorithmic bytes per launch (B_alg x active cells
 of that launch: CH fused pass 16 B = read c + write c'; dendrite 16 B per (cell,
 field) update; KH 64 B = read and write the 4 conserved fields) over its average
 duration. Resident steps (all steps of the timed call in one launch): the GPU time
-of the timed call over its steps; "long_run" has the same of one call of at least
---timing-steps steps. One launch per step (single-launch steps): the GPU time per
+of the timed call over its steps; "long_run" has the same of another call of at
+least --timing-steps steps. One launch per step (single-launch steps): the GPU time per
 step of a separate graph-replayed run of at least --timing-steps steps, between
 hipEvents on the library stream. Two launches per step: hipEvents around every step
 kernel in an eager pass.
@@ -627,7 +627,7 @@ def measure(ctx, workload, K, W, chunk_cap, timing_steps, single_launch, n=None,
     long_run = None
     if resident:
         # all steps of a call in one launch: the GPU time of the timed call itself, its
-        # worklist and state-restoring launches included; a longer call beside it
+        # worklist and state-restoring launches included; the other call beside it
         avg_k_s = gpu_ms / 1e3 / K
         cells_per_launch = active_updates / K
         timed_launches = 1

@@ -1048,10 +1048,10 @@ bool resident_buffer(dba_ctx* ctx, size_t words, int n_steps) {
 }
 
 // The process's contexts on a device, after adding `d`. A context alone on its device
-// takes resident launches. Where there are others it does not: two such launches, each
-// half resident, would wait for ever, and single-launch steps of two contexts overlap,
-// so they finish sooner than resident ones after each other (two contexts of 1024^2,
-// 2000 steps: 18.5 ms against 22).
+// takes resident launches. Where there are others it does not: of two such launches,
+// each half resident, both would be given up, and single-launch steps of two contexts
+// overlap, so they finish sooner than resident ones after each other (two contexts of
+// 1024^2, 2000 steps: 18.5 ms against 22).
 int live_contexts(int device, int d) {
     static std::mutex m;
     static std::map<int, int>* live = new std::map<int, int>();  // kept until the process ends
